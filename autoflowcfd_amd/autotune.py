@@ -1,10 +1,9 @@
 """Autotuner of the launch shapes of the residual kernels on one mesh.
 
 Every residual kernel walks its cells with a persistent grid; how many workgroups that grid
-has trades latency hiding against tail effects and L2 sharing, and two kernels also come in two
-tile shapes (``VARIANTS``: the prism inviscid kernel with or without its five slot sources staged
-in LDS, the SST cell kernel with two prisms or one cell per wavefront, which trade LDS and lanes
-against occupancy).  The best choice depends on the kernel, the order, the precision and the
+has trades latency hiding against tail effects and L2 sharing, and the SST cell kernel also comes in
+two tile shapes (``VARIANTS``: two prisms or one cell per wavefront, which trade LDS and lanes
+against occupancy; the prism inviscid kernel takes both codes for one shape).  The best choice depends on the kernel, the order, the precision and the
 mesh size.  ``autotune`` times each kernel's phase with HIP events on the launch stream for every
 (tile variant, grid size) candidate (results do not depend on either: only the time does) and
 leaves the fastest set on the mesh (``afr_mesh_set_variant``, ``afr_mesh_set_grid``).  Choices
@@ -100,13 +99,13 @@ def autotune(dm, U, mu_t=None, mu=1.8e-5, sst_fields=None, reps=3, candidates=No
         with open(cache_path) as f:
             cache = json.load(f)
     R = torch.empty_like(U)
+    mean = lambda: dm.residual(U, mu_t, R, mu=mu)  # noqa: E731  the mean-flow kernels as one call; one varies
     phases = {}
     if dm.mesh.n_prism:
-        phases["prism_inviscid"] = lambda: dm.inviscid_from_primitives(dm.work_q, dm.work_umean, R)
+        phases["prism_inviscid"] = mean
     if dm.mesh.n_tet:
-        phases["tet_inviscid"] = lambda: dm.inviscid_from_primitives(dm.work_q, dm.work_umean, R)
-    phases["visc_volume"] = lambda: dm.viscous_volume(U, mu_t, mu=mu)
-    phases["visc_iface"] = lambda: dm.viscous_interface(U, mu_t, R, mu=mu)
+        phases["tet_inviscid"] = mean
+    phases["visc_volume"] = phases["visc_iface"] = mean
     if sst_fields is not None and dm.turbulence == "SST":
         k, w, nut, mut = sst_fields
         rates = torch.empty((dm.n_cells, dm.ns, 2), dtype=dm.dtype, device=dm.device)
@@ -115,7 +114,6 @@ def autotune(dm, U, mu_t=None, mu=1.8e-5, sst_fields=None, reps=3, candidates=No
         sst = lambda: dm.sst_step(U, k, w, dt, nut, mut, mu=mu, rates=rates)  # noqa: E731
         for name in ("sst_cell", "sst_face", "sst_update"):
             phases[name] = sst                   # the SST call times its three kernels; one varies
-    dm.viscous_volume(U, mu_t, mu=mu)            # dQ / field means for the inviscid phase
     out = {}
     for name, fn in phases.items():
         key = _key(dm, name)

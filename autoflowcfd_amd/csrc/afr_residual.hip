@@ -1,20 +1,9 @@
-// Cell-centric FR residual kernels for gfx950 and the afr C ABI.
-//
-// Tets: one workgroup of 256 threads processes tiles of CPB cells at one
-// order with the dense operators (prisms use the Kronecker-factored kernel of
-// afr_prism.hip).  Per tile, everything stays in LDS:
-//   1. primitive states of the tile's cells,
-//   2. contravariant fluxes at the over-integration points
-//      (Q_fine = c2f Q, F~ = adj_fine F(Q_fine)),
-//   3. the FR interface jumps of every face slot (own trace E Q, other side
-//      by cross-interpolation rows or a ghost state, AUSM+up),
-//   4. residual = -(Op F~ + sum_slots g' jump) / det  with Op = f2c D_fine,
-//   5. outlier suppression (median over solution points),
-// and the tile is written once.  No scatter, coloring or atomics.
+// The afr C ABI: meshes, the residual entry points over the mean-flow kernels (afr_volume.hip,
+// afr_iface.hip), the pseudo-step, the SST step, graphs.
 //
 // Reference semantics: src/autoflowcfd/core/fr_residual/inviscid.py:139-345,
-// src/autoflowcfd/core/fr_residual/inviscid_kernel.py:87-284,
-// src/autoflowcfd/core/fr_operators/troubled_cell.py:339-408.
+// src/autoflowcfd/core/fr_residual/viscous_flux.py:113-302,
+// src/autoflowcfd/core/fr_solver/step.py:15-221.
 #include <hip/hip_runtime.h>
 #include <vector>
 
@@ -26,9 +15,9 @@
 #include <type_traits>
 
 #include "../../include/afr.h"
+#include "afr_meanflow.hpp"
 #include "afr_physics.hpp"
 #include "afr_prism.hpp"
-#include "afr_viscous.hpp"
 #include "afr_step.hpp"
 #include "afr_sst.hpp"
 #include "afr_forces.hpp"
@@ -66,57 +55,6 @@ struct AfrMesh {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kSlots = 5;
-
-template <int P> struct Ord {
-    static constexpr int N1 = P + 1;
-    static constexpr int NS = N1 * N1 * N1;
-    static constexpr int NFP = N1 * N1;
-    static constexpr int OV = (2 * P < 3 ? 2 * P : 3);
-    static constexpr int NF = (OV + 1) * (OV + 1) * (OV + 1);
-    static constexpr int CPB = kThreads / NF;  // cells per tile
-};
-
-template <int CT> struct Cell {
-    static constexpr int NSLOT = CT == 0 ? 5 : 4;
-    __device__ static int code(int slot) {
-        // prism slots: a=-1, a=+1, b=-1, c=-1, c=+1 ; tet slots: a=-1, a=+1, b=-1, c=-1
-        return slot < 3 ? slot : (slot == 3 ? 4 : 5);
-    }
-};
-
-template <typename real>
-struct Args {
-    int64_t cell_begin, n_cells_type;
-    const real* Q;        // (C, NS, 5) primitive
-    const real* umean;    // (C, 5) mean |U| per cell and variable (outlier reference)
-    real* R;
-    const real* det;
-    const real* adjf;
-    const int* slot_nb;
-    const int* slot_blk;
-    const int* slot_mask;
-    const int* slot_bc;
-    const int* slot_fb;
-    const real* slot_tn;
-    const real* slot_adjrow;
-    const real* rows;
-    const real* c2f;
-    const real* op;
-    const real* E;
-    const real* gL;
-    const real* gR;
-    const int* fp_of_sp;
-    const int* coord_of_sp;
-    const real* gcl;      // (C, NS, 3) constant-state divergence
-    const double* bcp;    // (8, 5) per-BC reference states ((n_cases, 8, 5) with cell_case)
-    const int* cell_case; // null: one case
-    double qref[5];       // primitive reference state
-    double fref[15];      // F(qref)[i][v]
-    int suppress;
-    int n_rows;
-};
-
 template <typename real>
 __global__ void __launch_bounds__(kThreads) k_primitives(const real* __restrict__ U, real* __restrict__ Q, int64_t n,
                                                          Ref5 ref) {
@@ -130,320 +68,6 @@ __global__ void __launch_bounds__(kThreads) k_primitives(const real* __restrict_
 #pragma unroll
         for (int v = 0; v < 5; ++v) Q[i * 5 + v] = (real)(q[v] - ref.q[v]);
     }
-}
-
-// median of |x[0..n)| as troubled_cell.py:347-379 takes it: the sorted values (NaN last), the
-// middle one or the mean of the two middle ones for even n; NaN when a median position holds NaN
-template <typename real, int N>
-__device__ real median_abs(const real* x, int stride) {
-    real a[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        real t = x[i * stride];
-        a[i] = t < real(0) ? -t : t;
-    }
-    const int k1 = (N - 1) / 2, k2 = N / 2;
-    const real qnan = real(__builtin_nan(""));
-    real m1 = qnan, m2 = qnan;
-    for (int i = 0; i < N; ++i) {
-        int lt = 0, le = 0;
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            lt += a[j] < a[i];
-            le += a[j] <= a[i];
-        }
-        if (lt <= k1 && k1 < le) m1 = a[i];
-        if (lt <= k2 && k2 < le) m2 = a[i];
-    }
-    return (N % 2) ? m1 : real(0.5) * (m1 + m2);
-}
-
-template <int P, int CT, typename real>
-__global__ void __launch_bounds__(kThreads) k_inviscid(Args<real> a) {
-    using O = Ord<P>;
-    constexpr int NS = O::NS, NF = O::NF, NFP = O::NFP, CPB = O::CPB, N1 = O::N1;
-    constexpr int NSLOT = Cell<CT>::NSLOT;
-    // P3 operator tables (64 x 64 and larger) do not fit LDS beside the tiles: they are read
-    // from global memory (L1/L2 resident) instead
-    constexpr bool OPS_LDS = P <= 2;
-    __shared__ real s_c2f_l[OPS_LDS ? NF * NS : 1];
-    __shared__ real s_op_l[OPS_LDS ? NS * 3 * NF : 1];
-    __shared__ real s_E_l[OPS_LDS ? NSLOT * NFP * NS : 1];
-    const real* const s_c2f = OPS_LDS ? s_c2f_l : a.c2f;
-    const real* const s_op = OPS_LDS ? s_op_l : a.op;
-    const real* const s_E = OPS_LDS ? s_E_l : a.E;
-    __shared__ real s_Q[CPB * NS * 5];
-    __shared__ real s_Ft[CPB * 3 * NF * 5];
-    __shared__ real s_J[CPB * NSLOT * NFP * 5];
-    __shared__ real s_R[CPB * NS * 5];
-    __shared__ real s_g[2 * N1];
-    __shared__ int s_fp[3 * NS];
-    __shared__ int s_co[3 * NS];
-
-    const int t = threadIdx.x;
-    if constexpr (OPS_LDS) {
-        for (int i = t; i < NF * NS; i += kThreads) s_c2f_l[i] = a.c2f[i];
-        for (int i = t; i < NS * 3 * NF; i += kThreads) s_op_l[i] = a.op[i];
-        for (int i = t; i < NSLOT * NFP * NS; i += kThreads) s_E_l[i] = a.E[i];
-    }
-    for (int i = t; i < 3 * NS; i += kThreads) {
-        s_fp[i] = a.fp_of_sp[i];
-        s_co[i] = a.coord_of_sp[i];
-    }
-    if (t < N1) {
-        s_g[t] = a.gL[t];
-        s_g[N1 + t] = a.gR[t];
-    }
-    __syncthreads();
-
-    const int64_t n_tiles = (a.n_cells_type + CPB - 1) / CPB;
-    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const int64_t first = a.cell_begin + tile * CPB;
-        const int ncell = (int)((a.n_cells_type - tile * CPB) < CPB ? (a.n_cells_type - tile * CPB) : CPB);
-
-        // 1. primitive states of the tile (contiguous)
-        for (int i = t; i < CPB * NS * 5; i += kThreads)
-            s_Q[i] = (i < ncell * NS * 5) ? a.Q[first * NS * 5 + i] : real(0);
-        __syncthreads();
-
-        // 2. contravariant fluxes at the fine points
-        if (t < CPB * NF) {
-            const int c = t / NF, j = t % NF;
-            if (c < ncell) {
-                real dq[5] = {0, 0, 0, 0, 0};
-                for (int s = 0; s < NS; ++s) {
-                    const real w = s_c2f[j * NS + s];
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) dq[v] += w * s_Q[(c * NS + s) * 5 + v];
-                }
-                // point flux in FP64 about the reference state, then back to storage precision
-                double q[5], Fd[3][5];
-#pragma unroll
-                for (int v = 0; v < 5; ++v) q[v] = a.qref[v] + (double)dq[v];
-                euler_flux(q, Fd);
-                real F[3][5];
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) F[i][v] = (real)(Fd[i][v] - a.fref[i * 5 + v]);
-                const real* ad = a.adjf + ((first + c) * NF + j) * 9;
-                real A[9];
-#pragma unroll
-                for (int k = 0; k < 9; ++k) A[k] = ad[k];
-#pragma unroll
-                for (int m = 0; m < 3; ++m)
-#pragma unroll
-                    for (int v = 0; v < 5; ++v)
-                        s_Ft[((c * 3 + m) * NF + j) * 5 + v] = A[m * 3 + 0] * F[0][v] + A[m * 3 + 1] * F[1][v] +
-                                                               A[m * 3 + 2] * F[2][v];
-            }
-        }
-
-        // 3. interface jumps, one thread per (cell, slot, flux point)
-        if (t < CPB * NSLOT * NFP) {
-            const int c = t / (NSLOT * NFP), r = t % (NSLOT * NFP);
-            const int slot = r / NFP, fp = r % NFP;
-            if (c < ncell) {
-                const int64_t gc = first + c;
-                const int64_t sidx = gc * kSlots + slot;
-                const int code = Cell<CT>::code(slot);
-                const double side = (code & 1) ? 1.0 : -1.0;
-                real dqo[5] = {0, 0, 0, 0, 0};
-                for (int s = 0; s < NS; ++s) {
-                    const real w = s_E[(slot * NFP + fp) * NS + s];
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) dqo[v] += w * s_Q[(c * NS + s) * 5 + v];
-                }
-                double qo[5], qn[5];
-#pragma unroll
-                for (int v = 0; v < 5; ++v) qo[v] = a.qref[v] + (double)dqo[v];
-                double tn[3] = {(double)a.slot_tn[sidx * 3 + 0], (double)a.slot_tn[sidx * 3 + 1],
-                                (double)a.slot_tn[sidx * 3 + 2]};
-                const int bc = a.slot_bc[sidx];
-                if (bc == BC_INTERIOR) {
-                    real dqn[5] = {0, 0, 0, 0, 0};
-                    const int src = (a.slot_mask[sidx] >> fp) & 1;
-                    const int nbc = a.slot_nb[sidx * 2 + src];
-                    const int blk = a.slot_blk[sidx * 2 + src];
-                    const int row = blk * NFP + fp;
-                    if (nbc >= 0 && row < a.n_rows) {
-                        const real* rw = a.rows + (int64_t)row * NS;
-                        const real* qn_src = a.Q + (int64_t)nbc * NS * 5;
-                        for (int s = 0; s < NS; ++s) {
-                            const real w = rw[s];
-#pragma unroll
-                            for (int v = 0; v < 5; ++v) dqn[v] += w * qn_src[s * 5 + v];
-                        }
-                    }
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) qn[v] = a.qref[v] + (double)dqn[v];
-                } else {
-                    ghost_state(bc, qo, tn, a.bcp + (a.cell_case ? 40 * a.cell_case[gc] : 0), qn);
-                }
-                const real* ar = a.slot_adjrow + (sidx * NFP + fp) * 3;
-                double A0 = ar[0], A1 = ar[1], A2 = ar[2];
-                double mag = rmax(sqrt(A0 * A0 + A1 * A1 + A2 * A2), 1e-300);
-                double d[3];
-                if ((a.slot_fb[sidx] >> fp) & 1) {
-                    d[0] = tn[0]; d[1] = tn[1]; d[2] = tn[2];
-                } else {
-                    d[0] = A0 / mag * side; d[1] = A1 / mag * side; d[2] = A2 / mag * side;
-                }
-                double fc[5];
-                ausm_up(qo, qn, d, fc);
-                double F[3][5];
-                euler_flux(qo, F);
-                const double sc = mag * side;
-#pragma unroll
-                for (int v = 0; v < 5; ++v)
-                    s_J[((c * NSLOT + slot) * NFP + fp) * 5 + v] =
-                        (real)(fc[v] * sc - (A0 * F[0][v] + A1 * F[1][v] + A2 * F[2][v]));
-            }
-        }
-        __syncthreads();
-
-        // 4. volume divergence (folded restriction) + interface correction
-        for (int o = t; o < CPB * NS * 5; o += kThreads) {
-            const int c = o / (NS * 5), rem = o % (NS * 5), s = rem / 5, v = rem % 5;
-            real val = real(0);
-            if (c < ncell) {
-                real acc = real(0);
-                const real* opr = s_op + s * 3 * NF;
-                const real* ft = s_Ft + (c * 3 * NF) * 5 + v;
-                for (int k = 0; k < 3 * NF; ++k) acc += opr[k] * ft[k * 5];
-                const real* gc = a.gcl + ((first + c) * NS + s) * 3;
-                acc += gc[0] * (real)a.fref[v] + gc[1] * (real)a.fref[5 + v] + gc[2] * (real)a.fref[10 + v];
-                real corr = real(0);
-#pragma unroll
-                for (int slot = 0; slot < NSLOT; ++slot) {
-                    const int code = Cell<CT>::code(slot);
-                    const int axis = code >> 1;
-                    const real g = s_g[((code & 1) ? N1 : 0) + s_co[axis * NS + s]];
-                    corr += g * s_J[((c * NSLOT + slot) * NFP + s_fp[axis * NS + s]) * 5 + v];
-                }
-                const real dj = a.det[(first + c) * NS + s];
-                val = -acc / dj - corr / dj;
-            }
-            s_R[o] = val;
-        }
-        __syncthreads();
-
-        // 5. outlier suppression per (cell, variable)
-        if (a.suppress && t < CPB * 5) {
-            const int c = t / 5, v = t % 5;
-            if (c < ncell) {
-                real med = median_abs<real, NS>(s_R + c * NS * 5 + v, 5);
-                const real mu = a.umean[(first + c) * 5 + v];
-                real ref = nan_max(nan_max(med, real(1e-9) * mu), Tiny<real>::v);
-                real thr = real(1e4) * ref;
-                for (int s = 0; s < NS; ++s) {
-                    real x = s_R[(c * NS + s) * 5 + v];
-                    if ((x < real(0) ? -x : x) > thr) s_R[(c * NS + s) * 5 + v] = real(0);
-                }
-            }
-        }
-        __syncthreads();
-
-        for (int i = t; i < ncell * NS * 5; i += kThreads) a.R[first * NS * 5 + i] = s_R[i];
-        __syncthreads();
-    }
-}
-
-int grid_for(int64_t tiles, int cap = 0) {
-    const int64_t c = cap > 0 ? cap : 4096;
-    int64_t g = tiles < c ? tiles : c;
-    return (int)(g > 0 ? g : 1);
-}
-
-template <int P, typename real>
-int launch_inviscid(const AfrMeshDesc& d, const real* Q, const real* umean, real* R, int suppress, hipStream_t st) {
-    using O = Ord<P>;
-    double fref[15];
-    {
-        double F[3][5];
-        euler_flux(d.ref_state, F);
-        for (int i = 0; i < 3; ++i)
-            for (int v = 0; v < 5; ++v) fref[i * 5 + v] = F[i][v];
-    }
-    if constexpr (P >= 3) {
-        if (d.n_prism > 0) return fail("order 3 is supported on tet meshes only");
-    } else if (d.n_prism > 0) {
-        // prisms: Kronecker-factored wave-per-cell kernel
-        afr_prism::PrismArgs<real> p;
-        p.n_cells = d.n_prism;
-        p.schedule = d.prism_schedule;
-        p.grid_cap = d.grid_cap[AFR_K_PRISM_INVISCID];
-        p.variant = d.variant[AFR_K_PRISM_INVISCID];
-        p.dQ = Q;
-        p.umean = umean;
-        p.R = R;
-        p.det = (const real*)d.det;
-        p.adjf = (const real*)d.adj_fine;
-        p.gcl = (const real*)d.gcl;
-        p.slot_nb = d.slot_nb;
-        p.slot_blk = d.slot_blk;
-        p.slot_mask = d.slot_mask;
-        p.slot_bc = d.slot_bc;
-        p.slot_fb = d.slot_fallback;
-        p.slot_tn = (const real*)d.slot_tn;
-        p.slot_adjrow = (const real*)d.slot_adjrow;
-        p.rows_nnz = d.rows_nnz;
-        p.rows_idx = d.rows_idx;
-        p.rows_w = (const real*)d.rows_w;
-        p.knz = d.rows_knz;
-        p.n_rows = d.n_rows;
-        p.tab = (const real*)d.prism_tab;
-        p.gL = (const real*)d.gL;
-        p.gR = (const real*)d.gR;
-        p.fp_of_sp = d.fp_of_sp;
-        p.coord_of_sp = d.coord_of_sp;
-        p.bcp = d.bc_params;
-        p.cell_case = d.cell_case;
-        for (int v = 0; v < 5; ++v) p.qref[v] = d.ref_state[v];
-        for (int k = 0; k < 15; ++k) p.fref[k] = fref[k];
-        p.suppress = suppress;
-        if (afr_prism::launch_prism_inviscid<P, real>(p, st)) return fail("k_prism_inviscid launch failed");
-    }
-    // tets: tile-per-workgroup kernel with dense operators
-    for (int ct = 1; ct < 2; ++ct) {
-        const int64_t begin = ct == 0 ? 0 : d.n_prism;
-        const int64_t n = ct == 0 ? d.n_prism : d.n_cells - d.n_prism;
-        if (n <= 0) continue;
-        Args<real> a;
-        a.cell_begin = begin;
-        a.n_cells_type = n;
-        a.Q = Q;
-        a.umean = umean;
-        a.R = R;
-        a.det = (const real*)d.det;
-        a.adjf = (const real*)d.adj_fine;
-        a.slot_nb = d.slot_nb;
-        a.slot_blk = d.slot_blk;
-        a.slot_mask = d.slot_mask;
-        a.slot_bc = d.slot_bc;
-        a.slot_fb = d.slot_fallback;
-        a.slot_tn = (const real*)d.slot_tn;
-        a.slot_adjrow = (const real*)d.slot_adjrow;
-        a.rows = (const real*)d.rows;
-        a.c2f = (const real*)d.c2f[ct];
-        a.op = (const real*)d.op[ct];
-        a.E = (const real*)d.E[ct];
-        a.gL = (const real*)d.gL;
-        a.gR = (const real*)d.gR;
-        a.fp_of_sp = d.fp_of_sp;
-        a.coord_of_sp = d.coord_of_sp;
-        a.gcl = (const real*)d.gcl;
-        a.bcp = d.bc_params;
-        a.cell_case = d.cell_case;
-        for (int v = 0; v < 5; ++v) a.qref[v] = d.ref_state[v];
-        for (int k = 0; k < 15; ++k) a.fref[k] = fref[k];
-        a.suppress = suppress;
-        a.n_rows = d.n_rows;
-        const int grid = grid_for((n + O::CPB - 1) / O::CPB, d.grid_cap[AFR_K_TET_INVISCID]);
-        hipLaunchKernelGGL((k_inviscid<P, 1, real>), dim3(grid), dim3(kThreads), 0, st, a);
-        HIP_TRY(hipGetLastError());
-    }
-    return 0;
 }
 
 template <typename real>
@@ -627,6 +251,119 @@ int afr_primitives(const void* U, void* Q, int64_t n_points, int32_t dtype, cons
                             : launch_primitives<float>(U, Q, n_points, ref, st);
 }
 
+}  // extern "C"
+
+namespace {
+
+enum Part { VISC_VOLUME, INV_VOLUME, IFACE_FULL, IFACE_VISC, IFACE_INV };
+
+// One part of the mean-flow residual over the prisms and the tets of a mesh.  U: the state of the
+// parts that start from it; dQ / umean: the prepared state instead (inviscid parts) or, with
+// VISC_VOLUME, where to write it (null: nowhere).
+template <typename real>
+int run_part(const AfrMesh* mesh, Part part, const void* U, const void* mu_t, const void* dQ, const void* umean,
+             void* R, double mu, double Pr, double Prt, int suppress, int accumulate, hipStream_t st) {
+    const AfrMeshDesc& d = mesh->d;
+    afr_mean::MeanArgs<real> a{};
+    a.U = (const real*)U;
+    a.so = mesh->so;
+    a.mu_t = (const real*)mu_t;
+    if (part == VISC_VOLUME) {
+        a.dQ_out = (real*)const_cast<void*>(dQ);
+        a.umean_out = (real*)const_cast<void*>(umean);
+    } else {
+        a.dQ = (const real*)dQ;
+        a.umean = (const real*)umean;
+    }
+    a.pack = (real*)d.work_vpack;
+    a.rvisc = (real*)d.work_rvol;
+    a.R = (real*)R;
+    a.det = (const real*)d.det;
+    a.adj = (const real*)d.adj;
+    a.adjf = (const real*)d.adj_fine;
+    a.gcl = (const real*)d.gcl;
+    a.tab = (const real*)d.prism_tab;
+    a.slot_nb = d.slot_nb;
+    a.slot_blk = d.slot_blk;
+    a.slot_mask = d.slot_mask;
+    a.slot_bc = d.slot_bc;
+    a.slot_fb = d.slot_fallback;
+    a.slot_tn = (const real*)d.slot_tn;
+    a.slot_adjrow = (const real*)d.slot_adjrow;
+    a.rows_nnz = d.rows_nnz;
+    a.rows_idx = d.rows_idx;
+    a.rows_w = (const real*)d.rows_w;
+    a.knz = d.rows_knz;
+    a.n_rows = d.n_rows;
+    a.gL = (const real*)d.gL;
+    a.gR = (const real*)d.gR;
+    a.bcp = d.bc_params;
+    a.cell_case = d.cell_case;
+    for (int v = 0; v < 5; ++v) a.qref[v] = d.ref_state[v];
+    double F[3][5];
+    euler_flux(d.ref_state, F);
+    for (int i = 0; i < 3; ++i)
+        for (int v = 0; v < 5; ++v) a.fref[i * 5 + v] = F[i][v];
+    a.mu = mu;
+    a.Pr = Pr;
+    a.Prt = Prt;
+    a.suppress = suppress;
+    a.accumulate = accumulate;
+    a.n_cells_mesh = d.n_cells;
+    for (int ct = 0; ct < 2; ++ct) {
+        a.cell_begin = ct == 0 ? 0 : d.n_prism;
+        a.n_cells = ct == 0 ? d.n_prism : d.n_cells - d.n_prism;
+        if (a.n_cells <= 0) continue;
+        a.D = (const real*)d.D[ct];
+        a.E = (const real*)d.E[ct];
+        a.c2f = (const real*)d.c2f[ct];
+        a.op = (const real*)d.op[ct];
+        const bool iface = part >= IFACE_FULL;
+        // the interface kernel reads neighbour data: locality order; the volume kernels only their
+        // own cells: storage order (contiguous reads)
+        a.schedule = (ct == 0 && iface) ? d.prism_schedule : nullptr;
+        a.grid_cap = d.grid_cap[part == VISC_VOLUME ? AFR_K_VISC_VOLUME
+                                : iface             ? AFR_K_VISC_IFACE
+                                : ct == 0           ? AFR_K_PRISM_INVISCID
+                                                    : AFR_K_TET_INVISCID];
+        auto go = [&](auto P, auto CT) -> int {
+            constexpr int p = decltype(P)::value, c = decltype(CT)::value;
+            switch (part) {
+                case VISC_VOLUME: return afr_mean::launch_visc_volume<p, c, real>(a, st);
+                case INV_VOLUME: return afr_mean::launch_inv_volume<p, c, real>(a, st);
+                default: return afr_mean::launch_iface<p, c, real>(a, part != IFACE_VISC, part != IFACE_INV, st);
+            }
+        };
+        using std::integral_constant;
+        typedef integral_constant<int, 0> I0;
+        typedef integral_constant<int, 1> I1;
+        typedef integral_constant<int, 2> I2;
+        int rc = -1;
+        if (d.order == 3) {
+            if constexpr (std::is_same<real, double>::value) {
+                if (ct == 1) rc = go(integral_constant<int, 3>(), I1());
+            }
+        } else if (d.order == 1) {
+            rc = ct == 0 ? go(I1(), I0()) : go(I1(), I1());
+        } else {
+            rc = ct == 0 ? go(I2(), I0()) : go(I2(), I1());
+        }
+        if (rc) return fail("mean-flow kernel launch failed");
+    }
+    return 0;
+}
+
+int mean_part(const AfrMesh* mesh, Part part, const void* U, const void* mu_t, const void* dQ, const void* umean,
+              void* R, double mu, double Pr, double Prt, int suppress, int accumulate, hipStream_t st) {
+    return mesh->d.dtype == AFR_F32
+               ? run_part<float>(mesh, part, U, mu_t, dQ, umean, R, mu, Pr, Prt, suppress, accumulate, st)
+               : run_part<double>(mesh, part, U, mu_t, dQ, umean, R, mu, Pr, Prt, suppress, accumulate, st);
+}
+
+}  // namespace
+
+extern "C" {
+
 int afr_prepare_state(const AfrMesh* mesh, const void* U, void* dQ, void* umean, void* stream) {
     if (!mesh || !U || !dQ || !umean) return fail("afr_prepare_state: null argument");
     const AfrMeshDesc& d = mesh->d;
@@ -654,20 +391,9 @@ int afr_prepare_state(const AfrMesh* mesh, const void* U, void* dQ, void* umean,
 int afr_inviscid_from_primitives(const AfrMesh* mesh, const void* dQ, const void* umean, void* R,
                                  int32_t suppress, void* stream) {
     if (!mesh || !dQ || !umean || !R) return fail("afr_inviscid_from_primitives: null argument");
-    const AfrMeshDesc& d = mesh->d;
     hipStream_t st = (hipStream_t)stream;
-    if (d.dtype == AFR_F32) {
-        auto* q = (const float*)dQ;
-        auto* m = (const float*)umean;
-        return d.order == 1   ? launch_inviscid<1, float>(d, q, m, (float*)R, suppress, st)
-               : d.order == 2 ? launch_inviscid<2, float>(d, q, m, (float*)R, suppress, st)
-                              : launch_inviscid<3, float>(d, q, m, (float*)R, suppress, st);
-    }
-    auto* q = (const double*)dQ;
-    auto* m = (const double*)umean;
-    return d.order == 1   ? launch_inviscid<1, double>(d, q, m, (double*)R, suppress, st)
-           : d.order == 2 ? launch_inviscid<2, double>(d, q, m, (double*)R, suppress, st)
-                          : launch_inviscid<3, double>(d, q, m, (double*)R, suppress, st);
+    if (mean_part(mesh, INV_VOLUME, nullptr, nullptr, dQ, umean, R, 0, 1, 1, 0, 0, st)) return -1;
+    return mean_part(mesh, IFACE_INV, nullptr, nullptr, dQ, umean, R, 0, 1, 1, suppress, 0, st);
 }
 
 int afr_inviscid_residual(const AfrMesh* mesh, const void* U, void* R, int32_t suppress, void* stream) {
@@ -681,82 +407,9 @@ int afr_inviscid_residual(const AfrMesh* mesh, const void* U, void* R, int32_t s
 
 namespace {
 
-template <typename real>
-int run_viscous(const AfrMeshDesc& d, const StateOff& so, const void* U, const void* mu_t, void* R, double mu,
-                double Pr, double Prt, int suppress, int accumulate, int phase, hipStream_t st) {
-    // phase 0: volume kernel only; 1: interface kernel only
-    for (int ct = 0; ct < 2; ++ct) {
-        afr_visc::ViscArgs<real> a;
-        a.cell_begin = ct == 0 ? 0 : d.n_prism;
-        a.n_cells = ct == 0 ? d.n_prism : d.n_cells - d.n_prism;
-        if (a.n_cells <= 0) continue;
-        a.U = (const real*)U;
-        a.so = so;
-        a.mu_t = (const real*)mu_t;
-        a.dQ = (real*)d.work_q;
-        a.umean = (real*)d.work_umean;
-        a.grad = (real*)d.work_grad;
-        a.rvol = (real*)d.work_rvol;
-        a.h_ip = (real*)d.work_h;
-        a.R = (real*)R;
-        a.det = (const real*)d.det;
-        a.adj = (const real*)d.adj;
-        a.vpack = (real*)d.work_vpack;
-        // the interface kernel reads neighbour data: locality order; the volume kernel only
-        // its own cell: storage order (contiguous reads)
-        a.schedule = (ct == 0 && phase != 0) ? d.prism_schedule : nullptr;
-        a.grid_cap = d.grid_cap[phase == 0 ? AFR_K_VISC_VOLUME : AFR_K_VISC_IFACE];
-        a.Dsp_w = (const real*)d.dsp_w[ct];
-        a.Dsp_i = d.dsp_i[ct];
-        a.Esp_w = (const real*)d.esp_w[ct];
-        a.Esp_i = d.esp_i[ct];
-        a.slot_nb = d.slot_nb;
-        a.slot_blk = d.slot_blk;
-        a.slot_mask = d.slot_mask;
-        a.slot_bc = d.slot_bc;
-        a.slot_tn = (const real*)d.slot_tn;
-        a.slot_adjrow = (const real*)d.slot_adjrow;
-        a.rows_idx = d.rows_idx;
-        a.rows_w = (const real*)d.rows_w;
-        a.knz = d.rows_knz;
-        a.n_rows = d.n_rows;
-        a.gL = (const real*)d.gL;
-        a.gR = (const real*)d.gR;
-        a.fp_of_sp = d.fp_of_sp;
-        a.coord_of_sp = d.coord_of_sp;
-        a.bcp = d.bc_params;
-        a.cell_case = d.cell_case;
-        for (int v = 0; v < 5; ++v) a.qref[v] = d.ref_state[v];
-        a.mu = mu;
-        a.Pr = Pr;
-        a.Prt = Prt;
-        a.suppress = suppress;
-        a.accumulate = accumulate;
-        int rc;
-        if (d.order == 3)
-            rc = ct == 0 ? -1 : afr_visc::launch_viscous_phase<3, 1, real>(a, phase, st);
-        else if (d.order == 1)
-            rc = ct == 0 ? afr_visc::launch_viscous_phase<1, 0, real>(a, phase, st)
-                         : afr_visc::launch_viscous_phase<1, 1, real>(a, phase, st);
-        else
-            rc = ct == 0 ? afr_visc::launch_viscous_phase<2, 0, real>(a, phase, st)
-                         : afr_visc::launch_viscous_phase<2, 1, real>(a, phase, st);
-        if (rc) return fail("viscous kernel launch failed");
-    }
-    return 0;
-}
-
-int viscous_phase(const AfrMesh* mesh, const void* U, const void* mu_t, void* R, double mu, double Pr, double Prt,
-                  int suppress, int accumulate, int phase, hipStream_t st) {
-    const AfrMeshDesc& d = mesh->d;
-    return d.dtype == AFR_F32
-               ? run_viscous<float>(d, mesh->so, U, mu_t, R, mu, Pr, Prt, suppress, accumulate, phase, st)
-               : run_viscous<double>(d, mesh->so, U, mu_t, R, mu, Pr, Prt, suppress, accumulate, phase, st);
-}
-
 bool viscous_ready(const AfrMeshDesc& d) {
     return d.adj && d.work_grad && d.work_rvol && d.work_h && d.work_vpack && d.dsp_w[0] && d.dsp_w[1] && d.dsp_i[0] &&
-           d.dsp_i[1] && d.esp_w[0] && d.esp_w[1] && d.esp_i[0] && d.esp_i[1];
+           d.dsp_i[1] && d.esp_w[0] && d.esp_w[1] && d.esp_i[0] && d.esp_i[1] && d.D[0] && d.D[1] && d.E[0] && d.E[1];
 }
 
 }  // namespace
@@ -769,8 +422,8 @@ int afr_viscous_residual(const AfrMesh* mesh, const void* U, const void* mu_t, v
     const AfrMeshDesc& d = mesh->d;
     if (!viscous_ready(d)) return fail("afr_viscous_residual: mesh has no viscous work buffers");
     hipStream_t st = (hipStream_t)stream;
-    if (viscous_phase(mesh, U, mu_t, R, mu, Pr, Pr_t, suppress, 0, 0, st)) return -1;
-    return viscous_phase(mesh, U, mu_t, R, mu, Pr, Pr_t, suppress, 0, 1, st);
+    if (mean_part(mesh, VISC_VOLUME, U, mu_t, d.work_q, d.work_umean, nullptr, mu, Pr, Pr_t, 0, 0, st)) return -1;
+    return mean_part(mesh, IFACE_VISC, U, mu_t, nullptr, d.work_umean, R, mu, Pr, Pr_t, suppress, 0, st);
 }
 
 int afr_viscous_volume(const AfrMesh* mesh, const void* U, const void* mu_t, double mu, double Pr, double Pr_t,
@@ -778,7 +431,8 @@ int afr_viscous_volume(const AfrMesh* mesh, const void* U, const void* mu_t, dou
     if (!mesh || !U) return fail("afr_viscous_volume: null argument");
     const AfrMeshDesc& d = mesh->d;
     if (!viscous_ready(d)) return fail("afr_viscous_volume: mesh has no viscous work buffers");
-    return viscous_phase(mesh, U, mu_t, nullptr, mu, Pr, Pr_t, 0, 0, 0, (hipStream_t)stream);
+    return mean_part(mesh, VISC_VOLUME, U, mu_t, d.work_q, d.work_umean, nullptr, mu, Pr, Pr_t, 0, 0,
+                     (hipStream_t)stream);
 }
 
 int afr_viscous_interface(const AfrMesh* mesh, const void* U, const void* mu_t, void* R, double mu, double Pr,
@@ -786,7 +440,8 @@ int afr_viscous_interface(const AfrMesh* mesh, const void* U, const void* mu_t, 
     if (!mesh || !U || !R) return fail("afr_viscous_interface: null argument");
     const AfrMeshDesc& d = mesh->d;
     if (!viscous_ready(d)) return fail("afr_viscous_interface: mesh has no viscous work buffers");
-    return viscous_phase(mesh, U, mu_t, R, mu, Pr, Pr_t, suppress, accumulate, 1, (hipStream_t)stream);
+    return mean_part(mesh, IFACE_VISC, U, mu_t, nullptr, d.work_umean, R, mu, Pr, Pr_t, suppress, accumulate,
+                     (hipStream_t)stream);
 }
 
 int afr_residual(const AfrMesh* mesh, const void* U, const void* mu_t, void* R, double mu, double Pr, double Pr_t,
@@ -795,10 +450,10 @@ int afr_residual(const AfrMesh* mesh, const void* U, const void* mu_t, void* R, 
     const AfrMeshDesc& d = mesh->d;
     if (!viscous_ready(d)) return fail("afr_residual: mesh has no viscous work buffers");
     hipStream_t st = (hipStream_t)stream;
-    // volume kernel: prepared state (dQ, umean), gradients, viscous volume term
-    if (viscous_phase(mesh, U, mu_t, R, mu, Pr, Pr_t, suppress, 0, 0, st)) return -1;
-    if (afr_inviscid_from_primitives(mesh, d.work_q, d.work_umean, R, suppress, stream)) return -1;
-    return viscous_phase(mesh, U, mu_t, R, mu, Pr, Pr_t, suppress, 1, 1, st);
+    // viscous pack and volume term, inviscid volume term (into R), then both interface terms at once
+    if (mean_part(mesh, VISC_VOLUME, U, mu_t, nullptr, nullptr, nullptr, mu, Pr, Pr_t, 0, 0, st)) return -1;
+    if (mean_part(mesh, INV_VOLUME, U, nullptr, nullptr, nullptr, R, mu, Pr, Pr_t, 0, 0, st)) return -1;
+    return mean_part(mesh, IFACE_FULL, U, mu_t, nullptr, nullptr, R, mu, Pr, Pr_t, suppress, 0, st);
 }
 
 namespace {

@@ -1,0 +1,583 @@
+// Volume terms of the mean-flow residual (gfx950).
+//
+//   k_visc_volume  U -> gradients of (u, v, w, T), viscous flux, its divergence, and the per-point
+//                  pack of the interface kernel (gradients.py:23-90, flux_kernels.py:72-137,
+//                  viscous_flux.py:113-302 under src/autoflowcfd/core/fr_operators, fr_residual)
+//   k_inv_volume   U -> over-integrated inviscid divergence of the prisms, by the Kronecker factors
+//                  of the collapsed prism basis (src/autoflowcfd/fr/collapsed_basis.py:197-230,
+//                  src/autoflowcfd/core/fr_residual/inviscid.py:139-345):
+//                      X = c2f_c dQ,  Qf = c2f_ab X,  F~ = adj_fine (F(Q_ref + Qf) - F(Q_ref)),
+//                      Y = A_a F~_a + A_b F~_b,  W = B_c F~_c,  div = f2c_c Y + f2c_ab W + gcl F(Q_ref)
+#include <hip/hip_runtime.h>
+
+#include "../../include/afr.h"
+#include "afr_meanflow.hpp"
+#include "afr_physics.hpp"
+#include "afr_prism.hpp"
+
+using namespace afr;
+
+namespace afr_mean {
+
+// ------------------------------------------------------------------ viscous volume kernel
+// Lanes of a wavefront: (cell, solution point), LW lanes per cell (P1: 8 cells of 8 lanes, P2: 2
+// cells of 27 of 32 lanes).  A lane keeps the non-zeros of its derivative rows in registers for the
+// whole kernel (d/da couples the N1 points of an a line, d/db the N1^2 of an (a, b) plane, d/dc the
+// N1 of a c line for a prism and all points for a tet, whose d/dc rows stay in LDS), reads its
+// neighbours' four fields with one 16-byte LDS load per non-zero at a fixed offset, and keeps its
+// gradients, stress and metrics in registers from the gradient to the flux.
+// Bound: HBM (reads U, mu_t, adj, det; writes the 16-value pack and the 4-value divergence: 4.5 GB at
+// 82^3 P2 FP32, 830 us = 5.4 TB/s).  Before: 2080 us with gradients staged through LDS, an 18-of-20-value
+// pack and a divided residual.  152k P1 prisms 57 us (285), P3 tets FP64 578 us (1168).
+template <int P, int CT, typename real> struct VV {
+    static constexpr int N1 = P + 1, NS = N1 * N1 * N1;
+    static constexpr int LW = NS <= 8 ? 8 : (NS <= 32 ? 32 : 64), CPW = 64 / LW;
+    static constexpr bool DENSE = P >= 3;   // P3 tets: the round-off entries of their rows count
+    static constexpr int KP = kPack + 4;    // LDS stride of a pack point (bank-conflict-free 16-byte access)
+    static constexpr int PER = NS * 4 + NS * KP;
+    static constexpr int WAVES = sizeof(real) == 8 && NS > 27 ? 2 : 4;
+    static constexpr int DT = CT == 1 && !DENSE ? NS * (NS | 1) : 4;   // d/dc rows of a tet
+};
+
+template <int P, int CT, typename real>
+__global__ void __launch_bounds__((64 * VV<P, CT, real>::WAVES)) k_visc_volume(MeanArgs<real> a) {
+    using L = VV<P, CT, real>;
+    using v4 = typename V4<real>::type;
+    constexpr int N1 = L::N1, NS = L::NS, LW = L::LW, CPW = L::CPW, KP = L::KP, WAVES = L::WAVES;
+    constexpr int RS = NS | 1;
+    __shared__ __attribute__((aligned(16))) real s_w[WAVES][CPW * L::PER];
+    __shared__ real s_dc[L::DT];
+    const int tid = threadIdx.x, wid = __builtin_amdgcn_readfirstlane(tid >> 6), t = tid & 63;
+    const int h = t / LW, s = t % LW;
+    const bool on = s < NS;
+    const int sp = on ? s : 0, i = sp / (N1 * N1), j = (sp / N1) % N1, k = sp % N1;
+    if constexpr (CT == 1 && !L::DENSE) {
+        for (int q = tid; q < NS * NS; q += 64 * WAVES) s_dc[(q / NS) * RS + q % NS] = a.D[2 * NS * NS + q];
+        __syncthreads();
+    }
+    real* const sF = s_w[wid] + h * L::PER;   // (du, dv, dw, dT) [s][4]
+    real* const sP = sF + NS * 4;             // pack [s][KP], then G~ [m][s][4]
+    real wa[N1], wb[N1 * N1], wc[N1];
+    if constexpr (!L::DENSE) {
+#pragma unroll
+        for (int q = 0; q < N1; ++q) {
+            wa[q] = a.D[sp * NS + (q * N1 + j) * N1 + k];
+            wc[q] = CT == 0 ? a.D[(2 * NS + sp) * NS + (i * N1 + j) * N1 + q] : real(0);
+        }
+#pragma unroll
+        for (int q = 0; q < N1 * N1; ++q) wb[q] = a.D[(NS + sp) * NS + q * N1 + k];
+    }
+    // sum_k row_m[k] x[k] over a field of 4 values per point
+    auto apply = [&](int m, const real* x) -> v4 {
+        v4 acc = {0, 0, 0, 0};
+        if constexpr (L::DENSE) {
+            const real* row = a.D + ((int64_t)m * NS + sp) * NS;
+#pragma unroll 4
+            for (int q = 0; q < NS; ++q) acc += row[q] * ld4(x + q * 4);
+        } else if (m == 0) {
+#pragma unroll
+            for (int q = 0; q < N1; ++q) acc += wa[q] * ld4(x + (q * N1 * N1 + j * N1 + k) * 4);
+        } else if (m == 1) {
+#pragma unroll
+            for (int q = 0; q < N1 * N1; ++q) acc += wb[q] * ld4(x + (q * N1 + k) * 4);
+        } else if constexpr (CT == 0) {
+#pragma unroll
+            for (int q = 0; q < N1; ++q) acc += wc[q] * ld4(x + ((i * N1 + j) * N1 + q) * 4);
+        } else {
+#pragma unroll
+            for (int q = 0; q < NS; ++q) acc += s_dc[sp * RS + q] * ld4(x + q * 4);
+        }
+        return acc;
+    };
+    const double T0 = a.qref[4] / (rmax(a.qref[0], 1e-10) * kRair);
+    const int64_t n_units = (a.n_cells + CPW - 1) / CPW;
+    for (CellWalk cw(n_units, WAVES, wid); cw.it < cw.hi; cw.it += cw.step) {
+        const int64_t c0 = cw.it * CPW;
+        const int nc = (int)(a.n_cells - c0 < CPW ? a.n_cells - c0 : CPW);
+        const bool live = on && h < nc;
+        const int64_t cell = a.cell_begin + c0 + (h < nc ? h : 0);
+        const int64_t pt = cell * NS + sp;
+        real ad[9], dq[5], mt = real(0), idet = real(0);
+        if (live) {
+#pragma unroll
+            for (int q = 0; q < 9; ++q) ad[q] = a.adj[pt * 9 + q];
+            idet = a.det[pt];
+            if (a.mu_t) mt = a.mu_t[pt];
+            double u[5], q[5];
+            load_state(a.U, pt, a.so, cell, u);
+            cons2prim(u, q);
+#pragma unroll
+            for (int v = 0; v < 5; ++v) dq[v] = (real)(q[v] - a.qref[v]);
+            const double T = q[4] / (rmax(q[0], 1e-10) * kRair);
+            st4(sF + s * 4, (v4){dq[1], dq[2], dq[3], (real)(T - T0)});
+            if (a.dQ_out) {
+#pragma unroll
+                for (int v = 0; v < 5; ++v) {
+                    a.dQ_out[pt * 5 + v] = dq[v];
+                    sP[s * 5 + v] = (real)fabs(u[v]);
+                }
+            }
+            idet = recip(idet);
+        }
+        wave_sync();
+        if (a.dQ_out) {   // per-cell mean |U| (outlier reference) of callers that prepare the state
+            if (h < nc && s < 5) {
+                real acc = 0;
+                for (int q = 0; q < NS; ++q) acc += sP[q * 5 + s];
+                a.umean_out[cell * 5 + s] = acc / real(NS);
+            }
+            wave_sync();
+        }
+        v4 gr[3];   // gr[n][f] = d f / dx_n
+        if (live) {
+            const v4 d0 = apply(0, sF), d1 = apply(1, sF), d2 = apply(2, sF);
+#pragma unroll
+            for (int n = 0; n < 3; ++n) gr[n] = (ad[n] * d0 + ad[3 + n] * d1 + ad[6 + n] * d2) * idet;
+            real* vp = sP + s * KP;
+            st4(vp, (v4){dq[0], dq[1], dq[2], dq[3]});
+            st4(vp + 4, (v4){dq[4], gr[0][0] + gr[0][0], gr[1][1] + gr[1][1], gr[2][2] + gr[2][2]});
+            st4(vp + 8, (v4){gr[1][0] + gr[0][1], gr[2][0] + gr[0][2], gr[2][1] + gr[1][2], gr[0][3]});
+            st4(vp + 12, (v4){gr[1][3], gr[2][3], mt, real(0)});
+        }
+        wave_sync();
+        // the packs of the wave's cells, contiguous in HBM: whole-line stores
+        {
+            real* dst = a.pack + (a.cell_begin + c0) * NS * kPack;
+            for (int o = t; o < nc * NS * 4; o += 64) {
+                const int c = o / (NS * 4), r = o % (NS * 4);
+                st4(dst + o * 4, ld4(s_w[wid] + c * L::PER + NS * 4 + (r >> 2) * KP + (r & 3) * 4));
+            }
+        }
+        wave_sync();
+        if (live) {
+            // viscous flux and its contravariant components
+            const real mu = (real)a.mu, mts = mu + mt;
+            const real lam = real(-2.0 / 3.0) * mts * (gr[0][0] + gr[1][1] + gr[2][2]);
+            const real cp = real(kGamma * kRair / (kGamma - 1.0));
+            const real kc = mu * cp / (real)a.Pr + mt * cp / (real)a.Prt;
+            real tau[3][3], e[3];
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) tau[p][q] = mts * (gr[q][p] + gr[p][q]) + (p == q ? lam : real(0));
+            real vel[3];
+#pragma unroll
+            for (int p = 0; p < 3; ++p) vel[p] = (real)(a.qref[1 + p] + (double)dq[1 + p]);
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                e[p] = vel[0] * tau[0][p] + vel[1] * tau[1][p] + vel[2] * tau[2][p] - kc * gr[p][3];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                v4 g;
+#pragma unroll
+                for (int v = 0; v < 3; ++v)
+                    g[v] = ad[m * 3] * tau[0][v] + ad[m * 3 + 1] * tau[1][v] + ad[m * 3 + 2] * tau[2][v];
+                g[3] = ad[m * 3] * e[0] + ad[m * 3 + 1] * e[1] + ad[m * 3 + 2] * e[2];
+                st4(sP + (m * NS + s) * 4, g);
+            }
+        }
+        wave_sync();
+        if (live) {
+            const v4 r = apply(0, sP) + apply(1, sP + NS * 4) + apply(2, sP + 2 * NS * 4);
+            st4(a.rvisc + pt * 4, r);
+        }
+        wave_sync();
+    }
+}
+
+template <int P, int CT, typename real>
+int launch_visc_volume(const MeanArgs<real>& a, hipStream_t st) {
+    using L = VV<P, CT, real>;
+    if (a.n_cells <= 0) return 0;
+    const int64_t units = (a.n_cells + L::CPW - 1) / L::CPW;
+    const int grid = walk_grid(units, L::WAVES, a.grid_cap > 0 ? a.grid_cap : 8192);
+    hipLaunchKernelGGL((k_visc_volume<P, CT, real>), dim3(grid), dim3(64 * L::WAVES), 0, st, a);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// ------------------------------------------------------------------ inviscid volume kernel (prisms)
+// A workgroup of N1 wavefronts takes CPT cells at a time (P2: 3 waves, 3 cells; P1: 2 waves, 4
+// cells).  In every contraction the wave index is the output row group, so the operator entries are
+// the same for all lanes of a wave and come from scalar loads; the lanes are (cell, fine line
+// coordinate, variable), 60 of 64, and hold their inputs in registers.  LDS carries only the data
+// from stage to stage; the row stride of F~ and W is padded so that 16-byte reads of successive
+// rows fall on different banks.
+// Bound: waits (59% of the wave cycles: barriers between the stages, scalar loads of the operators);
+// VALU issue takes 0.86 ms of it, HBM 3.5 GB.  Measured (82^3 P2 FP32): 1.21 ms; with the arguments held
+// in registers over the tile loop 1.48 ms.  Before, jumps included: 2.98 ms (one wave per cell, LDS
+// operator tables).  152k P1 prisms 143 us (1014 with jumps).
+template <int P, typename real> struct IV {
+    using K = afr_prism::PK<P>;
+    static constexpr int N1 = K::N1, NAB = K::NAB, NF1 = K::NF1, NABF = K::NABF, NF = K::NF, NS = K::NS;
+    static constexpr int NW = N1, CPT = 64 / (NF1 * 5);
+    static constexpr int QB = (NABF + 3) / 4, RS = QB * 4 + (QB % 2 == 0 ? 4 : 0);
+    static constexpr int CPWV = CPT / NW;                       // cells per wave at the fine points
+    static constexpr int OQ = 0, OX = OQ + NAB * 20, OF = OX + NAB * 20;   // q, X [ab][v][4], Qf [f][5]
+    static constexpr int OW = 0, OY = OW + N1 * 5 * RS;         // W [c][v][RS], Y [ab][v][4] (over q, X, Qf)
+    static constexpr int N0 = (OF + NF * 5 > OY + NAB * 20 ? OF + NF * 5 : OY + NAB * 20);
+    static constexpr int OT = (N0 + 3) / 4 * 4;                 // F~ [m][cf][v][RS]
+    static constexpr int PER = OT + 3 * NF1 * 5 * RS;
+    static constexpr int WPE = sizeof(real) == 4 ? (P == 1 ? 5 : 6) : 3;
+    static_assert(CPT % NW == 0 && CPWV * NF <= 64 && QB == NF1 && NAB == NW * N1, "lane maps");
+};
+
+template <int P, typename real>
+__global__ void __launch_bounds__((64 * IV<P, real>::NW))
+    __attribute__((amdgpu_waves_per_eu(IV<P, real>::WPE))) k_inv_volume(MeanArgs<real> args) {
+    using L = IV<P, real>;
+    using K = typename L::K;
+    using v4 = typename V4<real>::type;
+    using uni = typename Uni<real>::type;
+    constexpr int N1 = L::N1, NAB = L::NAB, NF1 = L::NF1, NABF = L::NABF, NF = L::NF, NS = L::NS;
+    constexpr int CPT = L::CPT, NW = L::NW, RS = L::RS, QB = L::QB, PER = L::PER, CPWV = L::CPWV;
+    __shared__ __attribute__((aligned(16))) real s_w[CPT * PER];
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = tid & 63;
+    // the arguments and the operator table are read anew in every stage (scalar loads): held over the
+    // tile loop they would be spilled to vector lanes
+    typedef const __attribute__((address_space(4))) MeanArgs<real> Args;
+    Args* const kernarg = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+    auto fresh = [&]() -> Args* {
+        Args* p = kernarg;
+        asm volatile("" : "+s"(p));
+        return p;
+    };
+    if constexpr (NABF % 4 != 0) {   // the padding of the F~ rows is read (times zero) and never written
+        for (int q = tid; q < CPT * PER; q += 64 * NW) s_w[q] = real(0);
+        __syncthreads();
+    }
+    // fine point of this lane: cell fc of the tile, point ff
+    const int fc = w * CPWV + t / NF, ff = t % NF;
+    const bool fon = t < CPWV * NF;
+    // contraction lanes: (cell lc, line coordinate cf, variable lv)
+    const int lc = t / (NF1 * 5), cf = (t / 5) % NF1, lv = t % 5;
+    const bool con = t < CPT * NF1 * 5;
+    // output lanes: (cell oc, c coordinate, variable)
+    const int oc = t / (N1 * 5), ocl = (t / 5) % N1;
+    const bool oon = t < CPT * N1 * 5;
+    real fcc[NF1];
+#pragma unroll
+    for (int q = 0; q < NF1; ++q) fcc[q] = args.tab[K::O_F2CC + (oon ? ocl : 0) * NF1 + q];
+    real fr[3];                       // F(q_ref) of the lane's variable
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+        fr[m] = (real)args.fref[m * 5];
+#pragma unroll
+        for (int v = 1; v < 5; ++v) fr[m] = lv == v ? (real)args.fref[m * 5 + v] : fr[m];
+    }
+
+    const int64_t n_cells = args.n_cells, n_tiles = (n_cells + CPT - 1) / CPT;
+    for (CellWalk cw(n_tiles, 1, 0); cw.it < cw.hi; cw.it += cw.step) {
+        Args* a = fresh();
+        const int64_t c0 = a->cell_begin + cw.it * CPT;
+        const int64_t left = n_cells - cw.it * CPT;
+        const int nc = (int)(left < CPT ? left : CPT);
+        // the adjugate of this lane's fine point, loaded before the stages that lead to it
+        real ad[9];
+        if (fon && fc < nc) {
+            GlobalPtr<real> src = (GlobalPtr<real>)a->adjf + ((c0 + fc) * NF + ff) * 9;
+#pragma unroll
+            for (int q = 0; q < 9; ++q) ad[q] = src[q];
+        }
+        // 0. dQ of the tile
+        for (int o = tid; o < nc * NS; o += 64 * NW) {
+            const int c = o / NS, s = o % NS;
+            real* x = s_w + c * PER + L::OQ + (s / N1) * 20 + s % N1;
+            if (a->dQ) {
+#pragma unroll
+                for (int v = 0; v < 5; ++v) x[v * 4] = ((GlobalPtr<real>)a->dQ)[(c0 * NS + o) * 5 + v];
+            } else {
+                double u[5], q[5];
+                load_state(args.U, c0 * NS + o, args.so, c0 + c, u);
+                cons2prim(u, q);
+#pragma unroll
+                for (int v = 0; v < 5; ++v) x[v * 4] = (real)(q[v] - a->qref[v]);
+            }
+        }
+        __syncthreads();
+        // 1. coarse -> fine along c
+        uni tab = (uni)fresh()->tab;
+        for (int o = tid; o < nc * NAB * 5; o += 64 * NW) {
+            real* cell = s_w + (o / (NAB * 5)) * PER;
+            const int r = o % (NAB * 5);
+            const v4 q = ld4(cell + L::OQ + r * 4);
+            v4 x = {0, 0, 0, 0};
+#pragma unroll
+            for (int f = 0; f < NF1; ++f)
+#pragma unroll
+                for (int c = 0; c < N1; ++c) x[f] += (real)tab[K::O_C2FC + f * N1 + c] * q[c];
+            st4(cell + L::OX + r * 4, x);
+        }
+        __syncthreads();
+        // 2. coarse -> fine along (a, b): wave w takes the fine rows w, w + NW, ...
+        tab = (uni)fresh()->tab;
+        if (con && lc < nc) {
+            real* cell = s_w + lc * PER;
+            real x[NAB];
+#pragma unroll
+            for (int ab = 0; ab < NAB; ++ab) x[ab] = cell[L::OX + (ab * 5 + lv) * 4 + cf];
+            for (int f = w; f < NABF; f += NW) {
+                real acc = 0;
+#pragma unroll
+                for (int ab = 0; ab < NAB; ++ab) acc += (real)tab[K::O_C2FAB + f * NAB + ab] * x[ab];
+                cell[L::OF + (f * NF1 + cf) * 5 + lv] = acc;
+            }
+        }
+        __syncthreads();
+        // 3. contravariant flux perturbation at the fine points: F~_m = adj_m . (F(q_ref + dq) -
+        //    F(q_ref)) by the exact algebraic expansion about q_ref (every term carries a
+        //    perturbation factor, so nothing cancels in the storage precision)
+        if (fon && fc < nc) {
+            a = fresh();
+            const real r0 = (real)a->qref[0], u0 = (real)a->qref[1], v0 = (real)a->qref[2], w0 = (real)a->qref[3];
+            const real p0 = (real)a->qref[4];
+            const real H0 = (real)(kGamma / (kGamma - 1.0) * a->qref[4] * recip(a->qref[0]) +
+                                   0.5 * (a->qref[1] * a->qref[1] + a->qref[2] * a->qref[2] + a->qref[3] * a->qref[3]));
+            real* cell = s_w + fc * PER;
+            const real* d = cell + L::OF + ff * 5;
+            const real dr = d[0], du = d[1], dv = d[2], dw = d[3], dp = d[4];
+            const real dpr = (dp * r0 - p0 * dr) * recip(r0 * (r0 + dr));
+            const real dH = real(kGamma / (kGamma - 1.0)) * dpr + (u0 * du + v0 * dv + w0 * dw) +
+                            real(0.5) * (du * du + dv * dv + dw * dw);
+            real* o = cell + L::OT + (ff % NF1) * 5 * RS + ff / NF1;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                const real a0 = ad[m * 3], a1 = ad[m * 3 + 1], a2 = ad[m * 3 + 2];
+                const real un0 = u0 * a0 + v0 * a1 + w0 * a2;
+                const real dun = du * a0 + dv * a1 + dw * a2;
+                const real m0 = r0 * un0;
+                const real dm = r0 * dun + dr * (un0 + dun);
+                real* om = o + m * NF1 * 5 * RS;
+                om[0] = dm;
+                om[RS] = m0 * du + dm * (u0 + du) + dp * a0;
+                om[2 * RS] = m0 * dv + dm * (v0 + dv) + dp * a1;
+                om[3 * RS] = m0 * dw + dm * (w0 + dw) + dp * a2;
+                om[4 * RS] = m0 * dH + dm * (H0 + dH);
+            }
+        }
+        __syncthreads();
+        tab = (uni)fresh()->tab;
+        // 4. Y (rows ab of group w) and W (c = w)
+        if (con && lc < nc) {
+            real* cell = s_w + lc * PER;
+            real acc[N1];
+#pragma unroll
+            for (int r = 0; r < N1; ++r) acc[r] = 0;
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const real* f = cell + L::OT + ((m * NF1 + cf) * 5 + lv) * RS;
+#pragma unroll
+                for (int qa = 0; qa < QB; ++qa) {
+                    const v4 x = ld4(f + 4 * qa);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (4 * qa + e < NABF) {
+#pragma unroll
+                            for (int r = 0; r < N1; ++r)
+                                acc[r] += (real)tab[(m == 0 ? K::O_AA : K::O_AB) + (w * N1 + r) * NABF + 4 * qa + e] * x[e];
+                        }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < N1; ++r) cell[L::OY + ((w * N1 + r) * 5 + lv) * 4 + cf] = acc[r];
+            // here the lane's cf is the quad index of the fine (a, b) points
+            v4 s4 = {0, 0, 0, 0};
+#pragma unroll
+            for (int q = 0; q < NF1; ++q)
+                s4 += (real)tab[K::O_BC + w * NF1 + q] * ld4(cell + L::OT + ((2 * NF1 + q) * 5 + lv) * RS + 4 * cf);
+            st4(cell + L::OW + (w * 5 + lv) * RS + 4 * cf, s4);
+        }
+        __syncthreads();
+        a = fresh();
+        tab = (uni)a->tab;
+        // 5. divergence at the solution points of the rows ab of group w
+        if (oon && oc < nc) {
+            const real* cell = s_w + oc * PER;
+            const int64_t p0s = (c0 + oc) * NS;
+            real acc[N1];
+#pragma unroll
+            for (int r = 0; r < N1; ++r) {
+                const v4 y = ld4(cell + L::OY + ((w * N1 + r) * 5 + lv) * 4);
+                acc[r] = 0;
+#pragma unroll
+                for (int q = 0; q < NF1; ++q) acc[r] += fcc[q] * y[q];
+            }
+#pragma unroll
+            for (int qa = 0; qa < QB; ++qa) {
+                const v4 x = ld4(cell + L::OW + (ocl * 5 + lv) * RS + 4 * qa);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (4 * qa + e < NABF) {
+#pragma unroll
+                        for (int r = 0; r < N1; ++r)
+                            acc[r] += (real)tab[K::O_F2CAB + (w * N1 + r) * NABF + 4 * qa + e] * x[e];
+                    }
+            }
+#pragma unroll
+            for (int r = 0; r < N1; ++r) {
+                const int64_t pt = p0s + (w * N1 + r) * N1 + ocl;
+                GlobalPtr<real> g = (GlobalPtr<real>)a->gcl + pt * 3;
+                typedef __attribute__((address_space(1))) real GlobalReal;
+                ((GlobalReal*)a->R)[pt * 5 + lv] = acc[r] + g[0] * fr[0] + g[1] * fr[1] + g[2] * fr[2];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// ------------------------------------------------------------------ inviscid volume kernel (tets)
+// Dense operators (the collapsed tet basis does not factor).  A workgroup of 4 waves takes 12 cells;
+// lane = (cell, variable), 60 of 64, holds the 12 x 5 columns of dQ in registers, and every wave
+// applies its own rows of c2f and Op to all of them with the row entries from scalar loads (one
+// operator entry serves 60 products, no operator table in LDS).  The flux of one contravariant
+// direction at a time passes through LDS, lane = (cell, fine point), 12 x NF of them.
+// Measured, FP64: P2 70 us (546 with the jumps before, when every cell was one workgroup's pass over
+// operators in LDS), P3 329 us (1618 with jumps).
+template <int P, typename real> struct IT {
+    static constexpr int N1 = P + 1, NS = N1 * N1 * N1, OV = (2 * P < 3 ? 2 * P : 3), NF = (OV + 1) * (OV + 1) * (OV + 1);
+    static constexpr int CPT = 12, NW = 4, NT = 64 * NW;
+    static constexpr int RW = (NS + NW - 1) / NW;               // Op rows of a wave
+    static constexpr int NI = (CPT * NF + NT - 1) / NT;         // fine points of a thread
+    static constexpr int KB = sizeof(real) == 8 ? 4 : 8;        // operator columns per scalar load
+    static constexpr int FS = (NF * 5 + 3) / 4 * 4;
+    static constexpr int QS = (NS * 5) | 1;                     // LDS stride of a cell's dQ
+    static constexpr int N_Q = CPT * QS > CPT * FS ? CPT * QS : CPT * FS;
+};
+
+template <int P, typename real>
+__global__ void __launch_bounds__(256) k_inv_volume_tet(MeanArgs<real> a) {
+    using L = IT<P, real>;
+    using uni = typename Uni<real>::type;
+    constexpr int NS = L::NS, NF = L::NF, CPT = L::CPT, NW = L::NW, NT = L::NT, RW = L::RW, NI = L::NI, FS = L::FS;
+    constexpr int QS = L::QS;
+    __shared__ real s_q[L::N_Q];         // dQ [c][s][5], then Qf [c][j][5]
+    __shared__ real s_f[CPT * FS];       // F~_m [c][j][5]
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = tid & 63;
+    const int lc = t / 5, lv = t % 5;
+    const uni c2f = (uni)a.c2f, op = (uni)a.op;
+    const int64_t n_tiles = (a.n_cells + CPT - 1) / CPT;
+    for (CellWalk cw(n_tiles, 1, 0); cw.it < cw.hi; cw.it += cw.step) {
+        const int64_t c0 = a.cell_begin + cw.it * CPT;
+        const int nc = (int)(a.n_cells - cw.it * CPT < CPT ? a.n_cells - cw.it * CPT : CPT);
+        const bool on = t < 5 * CPT && lc < nc;
+        for (int o = tid; o < nc * NS; o += NT) {
+            const int c = o / NS, s = o % NS;
+            real* x = s_q + c * QS + s * 5;
+            if (a.dQ) {
+#pragma unroll
+                for (int v = 0; v < 5; ++v) x[v] = a.dQ[(c0 * NS + o) * 5 + v];
+            } else {
+                double u[5], q[5];
+                load_state(a.U, c0 * NS + o, a.so, c0 + c, u);
+                cons2prim(u, q);
+#pragma unroll
+                for (int v = 0; v < 5; ++v) x[v] = (real)(q[v] - a.qref[v]);
+            }
+        }
+        __syncthreads();
+        real x[NS];
+        if (on) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) x[s] = s_q[lc * QS + s * 5 + lv];
+        }
+        __syncthreads();
+        if (on) {
+            for (int j = w; j < NF; j += NW) {
+                real acc = 0;
+#pragma unroll
+                for (int s = 0; s < NS; ++s) acc += (real)c2f[j * NS + s] * x[s];
+                s_q[lc * FS + j * 5 + lv] = acc;
+            }
+        }
+        __syncthreads();
+        // point flux in FP64 about the reference state, one contravariant direction m at a time
+        real acc[RW];
+#pragma unroll
+        for (int r = 0; r < RW; ++r) acc[r] = 0;
+        for (int m = 0; m < 3; ++m) {
+#pragma unroll
+            for (int q = 0; q < NI; ++q) {
+                const int o = tid + NT * q, c = o / NF, j = o % NF;
+                if (o < nc * NF) {
+                    const real* ad = a.adjf + ((c0 + c) * NF + j) * 9 + m * 3;
+                    const real A[3] = {ad[0], ad[1], ad[2]};
+                    const real* dq = s_q + c * FS + j * 5;
+                    double q5[5], F[3][5];
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) q5[v] = a.qref[v] + (double)dq[v];
+                    euler_flux(q5, F);
+                    real f[5];
+#pragma unroll
+                    for (int v = 0; v < 5; ++v)
+                        f[v] = A[0] * (real)(F[0][v] - a.fref[v]) + A[1] * (real)(F[1][v] - a.fref[5 + v]) +
+                               A[2] * (real)(F[2][v] - a.fref[10 + v]);
+                    real* o5 = s_f + c * FS + j * 5;
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) o5[v] = f[v];
+                }
+            }
+            __syncthreads();
+            if (on) {
+                const real* f = s_f + lc * FS + lv;
+                const int s0 = w * RW;
+#pragma unroll 1
+                for (int j0 = 0; j0 < NF; j0 += L::KB) {
+                    real y[L::KB];
+#pragma unroll
+                    for (int e = 0; e < L::KB; ++e) y[e] = j0 + e < NF ? f[(j0 + e < NF ? j0 + e : 0) * 5] : real(0);
+#pragma unroll
+                    for (int r = 0; r < RW; ++r) {
+                        const int s = s0 + r < NS ? s0 + r : NS - 1;
+#pragma unroll
+                        for (int e = 0; e < L::KB; ++e)
+                            acc[r] += (real)op[s * 3 * NF + m * NF + (j0 + e < NF ? j0 + e : NF - 1)] * y[e];
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        if (on) {
+            const real g0 = (real)a.fref[lv], g1 = (real)a.fref[5 + lv], g2 = (real)a.fref[10 + lv];
+#pragma unroll
+            for (int r = 0; r < RW; ++r) {
+                const int s = w * RW + r;
+                if (s < NS) {
+                    const int64_t pt = (c0 + lc) * NS + s;
+                    const real* g = a.gcl + pt * 3;
+                    a.R[pt * 5 + lv] = acc[r] + g[0] * g0 + g[1] * g1 + g[2] * g2;
+                }
+            }
+        }
+    }
+}
+
+template <int P, int CT, typename real>
+int launch_inv_volume(const MeanArgs<real>& a, hipStream_t st) {
+    if (a.n_cells <= 0) return 0;
+    if constexpr (CT == 0) {
+        using L = IV<P, real>;
+        const int64_t tiles = (a.n_cells + L::CPT - 1) / L::CPT;
+        const int grid = walk_grid(tiles, 1, a.grid_cap > 0 ? a.grid_cap : 8192);
+        hipLaunchKernelGGL((k_inv_volume<P, real>), dim3(grid), dim3(64 * L::NW), 0, st, a);
+    } else {
+        using L = IT<P, real>;
+        const int64_t tiles = (a.n_cells + L::CPT - 1) / L::CPT;
+        const int grid = walk_grid(tiles, 1, a.grid_cap > 0 ? a.grid_cap : 4096);
+        hipLaunchKernelGGL((k_inv_volume_tet<P, real>), dim3(grid), dim3(L::NT), 0, st, a);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+#define AFR_VOL_INST(P, CT, T)                                                       \
+    template int launch_visc_volume<P, CT, T>(const MeanArgs<T>&, hipStream_t);      \
+    template int launch_inv_volume<P, CT, T>(const MeanArgs<T>&, hipStream_t);
+AFR_VOL_INST(1, 0, float)
+AFR_VOL_INST(2, 0, float)
+AFR_VOL_INST(1, 0, double)
+AFR_VOL_INST(2, 0, double)
+AFR_VOL_INST(1, 1, float)
+AFR_VOL_INST(2, 1, float)
+AFR_VOL_INST(1, 1, double)
+AFR_VOL_INST(2, 1, double)
+AFR_VOL_INST(3, 1, double)
+
+}  // namespace afr_mean

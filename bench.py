@@ -113,6 +113,13 @@ def algorithmic_bytes_visc_iface(n_sp, n_cells, nfp, w=4):
     return n_sp * (18 + 5 + 1 + 10) * w + n_cells * (5 * (nfp * 3 + 3) * w + 5 * 6 * 4 + 6 * w)
 
 
+def algorithmic_bytes_mean_flow(n_sp, n_fine_pts, n_faces, nfp, w=4):
+    """Compulsory traffic of the mean-flow residual as one pass: read U (5) and mu_t, write R (5),
+    det and adj (9) per solution point, adj(J) at the fine points, per physical face the flux-point
+    normals and face ids/codes."""
+    return n_sp * (5 + 1 + 5 + 1 + 9) * w + n_fine_pts * 9 * w + n_faces * (nfp * 3 * w + 16)
+
+
 def _cpu_sample(order, n_sample, budget_s, seed):
     """One single-threaded worker of the CPU baseline: (solution points, median seconds, evaluations)
     of the FP64 oracle's full P2 SST RANS residual on an n_sample^3-hex graded wall box."""
@@ -176,18 +183,17 @@ def cpu_baseline(order, n_sample=6, budget_s=20.0, workers=None):
                       f"({res[0][1]:.3f} s each on one core)"}
 
 
-def residual_kernel_names(P, knz, ns, v_inv=0, v_sst=0):
+def residual_kernel_names(P, knz, ns, v_sst=0):
     """{phase: [kernel names as the profiler prints them]} of one prism-mesh residual evaluation at
     order P with knz-wide interpolation rows, ns stored points per cell and the tile variants in
-    force (afr_mesh_set_variant: prism variant v stages the slot sources when v = 1; SST cell
-    variant v pairs prisms when v = 0)."""
+    force (afr_mesh_set_variant: SST cell variant v pairs prisms when v = 0)."""
     return {
         "dt_local": [f"afr_step::k_dt_cells<{ns}, float>" if ns in (1, 8, 27, 64) else "afr_step::k_dt_local<float>"],
         "sst": [f"afr_sst::k_sst_cell<{P}, 0, float, {1 - v_sst}>", f"afr_sst::k_sst_face<{P}, {knz}, float>",
                 f"afr_sst::k_sst_update<{P}, 0, float>"],
-        "visc_volume": [f"afr_visc::k_visc_volume<{P}, 0, float>"],
-        "inviscid": [f"afr_prism::k_prism_inviscid<{P}, {knz}, float, {v_inv}>"],
-        "visc_interface": [f"afr_visc::k_visc_iface<{P}, 0, {knz}, float>"],
+        "visc_volume": [f"afr_mean::k_visc_volume<{P}, 0, float>"],
+        "inviscid": [f"afr_mean::k_inv_volume<{P}, float>"],
+        "visc_interface": [f"afr_mean::k_iface<{P}, 0, {knz}, float, true, true, false>"],
     }
 
 
@@ -384,8 +390,9 @@ def tgv_p3_leg(args):
     def diagnostics():
         U = s.U
         ke = float((0.5 * (U[..., 1:4] ** 2).sum(-1) / U[..., 0]).mean().item())
-        s.dm.viscous_volume(U, None, mu=mu)
-        g = s.dm.work_vpack[..., 5:14].reshape(U.shape[0], U.shape[1], 3, 3)   # [i][j] = du_i/dx_j
+        # du_i/dx_j = (D u_i)_m adj[m][j] / det at the solution points
+        d = torch.einsum("mst,cti->csim", s.dm.D[1], U[..., 1:4] / U[..., :1])
+        g = torch.einsum("csim,csmj->csij", d, s.dm.adj) / s.dm.det[..., None, None]
         om2 = (g[..., 2, 1] - g[..., 1, 2]) ** 2 + (g[..., 0, 2] - g[..., 2, 0]) ** 2 + (g[..., 1, 0] - g[..., 0, 1]) ** 2
         ens = float((0.5 * U[..., 0] * om2).mean().item())
         return ke, ens, bool(torch.isfinite(U).all().item())
@@ -525,7 +532,7 @@ def main():
             residual_step()
         torch.cuda.synchronize()
 
-    n_ev = 6
+    n_ev = 4
     ev = [[torch.cuda.Event(enable_timing=True) for _ in range(n_ev)] for _ in range(args.steps)]
     torch.cuda.synchronize()
     t_start = time.perf_counter()
@@ -536,17 +543,13 @@ def main():
         e[1].record()
         dm.sst_step(U, k, w, dt, nut, mut, mu=MU, rates=rates)
         e[2].record()
-        dm.viscous_volume(U, mut, mu=MU)
+        dm.residual(U, mut, R, mu=MU)
         e[3].record()
-        dm.inviscid_from_primitives(dm.work_q, dm.work_umean, R)
-        e[4].record()
-        dm.viscous_interface(U, mut, R, mu=MU)
-        e[5].record()
     torch.cuda.synchronize()
     wall = time.perf_counter() - t_start
     ph = np.array([[ev[i][j].elapsed_time(ev[i][j + 1]) for j in range(n_ev - 1)] for i in range(args.steps)]).mean(0)
     ms_per_step = wall / args.steps * 1e3
-    names = ["dt_local", "sst", "visc_volume", "inviscid", "visc_interface"]
+    names = ["dt_local", "sst", "mean_flow"]
     log("[bench] residual: %.3f ms/step (%s)" % (ms_per_step, ", ".join(f"{n} {t:.3f}" for n, t in zip(names, ph))))
     if not bool(torch.isfinite(R).all()):
         raise RuntimeError("non-finite residual")
@@ -565,17 +568,15 @@ def main():
     fr = mesh.faces
     is_quad = np.isin(fr.owner_code, (0, 1, 2)) & (fr.owner < mesh.n_prism)
     n_phys_faces = int(fr.n_faces - is_quad.sum() // 2)
-    b_inv = algorithmic_bytes_inviscid(n_sp, mesh.n_cells * dm.nf, n_phys_faces, dm.nfp)
-    # per-phase rooflines (prism-only mesh: one launch per phase, three for SST), timed with HIP
+    # per-phase rooflines (prism-only mesh: one launch for dt, three each for SST and the mean flow), timed with HIP
     # events on the launch stream; PMC traffic from the committed rocprofv3 summary
     P, knz = args.order, dm.rows_knz
     from autoflowcfd_amd.autotune import get_variant
-    v_inv, v_sst = get_variant(dm, "prism_inviscid"), get_variant(dm, "sst_cell")
-    kn = residual_kernel_names(P, knz, dm.ns, v_inv, v_sst)
+    kn = residual_kernel_names(P, knz, dm.ns, get_variant(dm, "sst_cell"))
+    kn["mean_flow"] = kn.pop("visc_volume") + kn.pop("inviscid") + kn.pop("visc_interface")
     phase_bytes = {"dt_local": algorithmic_bytes_dt_local(n_sp, mesh.n_cells),
                    "sst": algorithmic_bytes_sst(n_sp, mesh.n_cells, fr.n_faces),
-                   "visc_volume": algorithmic_bytes_visc_volume(n_sp, mesh.n_cells), "inviscid": b_inv,
-                   "visc_interface": algorithmic_bytes_visc_iface(n_sp, mesh.n_cells, dm.nfp)}
+                   "mean_flow": algorithmic_bytes_mean_flow(n_sp, mesh.n_cells * dm.nf, n_phys_faces, dm.nfp)}
     kr = {}
     for phase, parts in kn.items():
         kname, b = " + ".join(parts), phase_bytes[phase]

@@ -79,14 +79,16 @@ enum { AFR_F32 = 0, AFR_F64 = 1 };
  *                                      dQ = Q - Q_ref in the storage precision and evaluate
  *                                      point fluxes / Riemann fluxes in FP64
  *   work_q     (C, ns, 5)              scratch for dQ = primitive - Q_ref
- *   work_grad  (C, ns, 12)             scratch for grad u (9, [i][j] = du_i/dx_j) and grad T (3)
+ *   work_grad  (C, ns, 12)             kept for callers that lay it out; the kernels keep gradients on chip
  *   work_umean (C, 5)                  scratch for the per-cell mean |U| (outlier reference)
- *   work_rvol  (C, ns, 5)              scratch for the viscous volume term
- *   work_vpack (C, ns, 20)             scratch: per-point (dQ, grad u, grad T, mu_t, pad) pack
+ *   work_rvol  (C, ns, 5)              scratch for the viscous volume term: 4 values (momentum, energy) per
+ *                                      point, not yet divided by det J, at stride 4
+ *   work_vpack (C, ns, 20)             scratch: per-point pack at stride 16: dQ (5), grad u + (grad u)^T
+ *                                      (xx, yy, zz, xy, xz, yz), grad T (3), mu_t, pad
  *   dsp_w[t], dsp_i[t] (3, ns, W_t)    sparse rows of D[t] (W = 9 prism / 27 tet at P2; row m of
  *                                      direction m holds its non-zeros first, zero-padded)
  *   esp_w[t], esp_i[t] (5, nfp, K_t)   sparse rows of E[t] in slot order (K = nfp prism / ns tet)
- *   work_h     (C)                     scratch for the interior-penalty length mean(det)^(1/3)
+ *   work_h     (C)                     kept for callers that lay it out; computed where it is needed
  *   metric_flux_scale (C, ns)          sum_m |adj(J)[m, :]| (geometric time-step limit)
  *   volume     (C)                     cell volumes (GL quadrature)
  *   work_r, work_s1, work_s2 (C, ns, 5) pseudo-step scratch: residual, stage states
@@ -262,16 +264,15 @@ int afr_inviscid_from_primitives(const AfrMesh *mesh, const void *dQ, const void
 
 /* Viscous BR1 FR residual dU/dt (C, ns, 5); mu_t (C, ns) or NULL.
  * mu, Pr, Pr_t as in the reference (1.8e-5, 0.72, 0.9 by default).  Uses the
- * work buffers work_q, work_umean, work_grad, work_rvol and work_h; on return
- * work_q / work_umean hold the prepared state of U and work_grad its gradients. */
+ * work buffers work_q, work_umean, work_rvol and work_vpack; on return work_q /
+ * work_umean hold the prepared state of U. */
 int afr_viscous_residual(const AfrMesh *mesh, const void *U, const void *mu_t, void *R, double mu,
                          double Pr, double Pr_t, int32_t suppress, void *stream);
 
 /* The two phases of afr_viscous_residual, for callers that interleave other work:
- * afr_viscous_volume writes the prepared state (work_q, work_umean), the gradients
- * (work_grad), the viscous volume term (work_rvol) and work_h from U;
- * afr_viscous_interface adds the BR1 interface correction to work_rvol, applies the
- * outlier zeroing when suppress != 0 and writes (accumulate == 0) or adds
+ * afr_viscous_volume writes the prepared state (work_q, work_umean), the interface
+ * pack (work_vpack) and the viscous volume term (work_rvol) from U;
+ * afr_viscous_interface adds the BR1 interface correction, applies the outlier zeroing when suppress != 0 and writes (accumulate == 0) or adds
  * (accumulate != 0) the result to R. */
 int afr_viscous_volume(const AfrMesh *mesh, const void *U, const void *mu_t, double mu, double Pr, double Pr_t,
                        void *stream);
@@ -376,9 +377,8 @@ int afr_mesh_set_grid(AfrMesh *mesh, int32_t kernel, int32_t grid_cap);
 int afr_mesh_get_grid(const AfrMesh *mesh, int32_t kernel);
 
 /* Tile shape of one kernel on this mesh (no reference counterpart; picked by the autotuner with
- * the grid size).  AFR_K_PRISM_INVISCID: 0 = the own cell's state staged in LDS, the slot sources
- * read from global memory; 1 = the own cell and its five slot sources staged in LDS (more LDS per
- * wavefront, fewer waves per SIMD).  AFR_K_SST_CELL: 0 = two prisms per wavefront (half-waves of
+ * the grid size).  AFR_K_PRISM_INVISCID: 0 and 1 are accepted and are the same tile shape (its
+ * volume kernel reads no neighbours).  AFR_K_SST_CELL: 0 = two prisms per wavefront (half-waves of
  * 32 lanes, P <= 2 prisms), 1 = one cell per wavefront.  Other kernels: 0 only.  Every variant
  * computes the same values bit for bit. */
 int afr_mesh_set_variant(AfrMesh *mesh, int32_t kernel, int32_t variant);

@@ -1,9 +1,8 @@
 """Autotuner of the launch shapes of the residual kernels on one mesh.
 
 Every residual kernel walks its cells with a persistent grid; how many workgroups that grid
-has trades latency hiding against tail effects and L2 sharing, and the SST cell kernel also comes in
-two tile shapes (``VARIANTS``: two prisms or one cell per wavefront, which trade LDS and lanes
-against occupancy; the prism inviscid kernel takes both codes for one shape).  The best choice depends on the kernel, the order, the precision and the
+has trades latency hiding against tail effects and L2 sharing (``VARIANTS``: tile-shape codes that a
+kernel takes; both codes of either kernel are one shape).  The best choice depends on the kernel, the order, the precision and the
 mesh size.  ``autotune`` times each kernel's phase with HIP events on the launch stream for every
 (tile variant, grid size) candidate (results do not depend on either: only the time does) and
 leaves the fastest set on the mesh (``afr_mesh_set_variant``, ``afr_mesh_set_grid``).  Choices

@@ -9,38 +9,6 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-// Occupancy targets (waves per SIMD) of the heavy kernels, as build parameters: 0 leaves the
-// register allocation to the compiler; n > 0 asks for at least n waves per SIMD (the compiler
-// then budgets registers for it, spilling if it must).  Measured on the 82^3 P2 SST residual:
-// the interface kernel 3.52 (7 waves, 28 B/lane spilled), 3.22 (6 waves, no spill), 3.55 ms
-// (compiler's choice, 5 waves); the SST update 3.90 (8 waves, 56 B/lane spilled), 3.83 (7 waves,
-// 20 B), 3.88 ms (6 waves, no spill) for the whole SST phase; the SST cell, inviscid and viscous
-// volume kernels are bounded by LDS or already at their register limit.
-#ifndef AFR_WPE_SST_CELL
-#define AFR_WPE_SST_CELL 0
-#endif
-#ifndef AFR_WPE_SST_UPDATE
-#define AFR_WPE_SST_UPDATE 7
-#endif
-#ifndef AFR_WPE_VISC_IFACE
-#define AFR_WPE_VISC_IFACE 6
-#endif
-#ifndef AFR_WPE_VISC_VOLUME
-#define AFR_WPE_VISC_VOLUME 0
-#endif
-#ifndef AFR_WPE_PRISM
-#define AFR_WPE_PRISM 0
-#endif
-#define AFR_WPE_ATTR_0
-#define AFR_WPE_ATTR_N(n) __attribute__((amdgpu_waves_per_eu(n, 8)))
-#define AFR_WPE_SEL(n) AFR_WPE_SEL2(n)
-#define AFR_WPE_SEL2(n) AFR_WPE_ATTR_##n
-#define AFR_WPE_ATTR_4 AFR_WPE_ATTR_N(4)
-#define AFR_WPE_ATTR_5 AFR_WPE_ATTR_N(5)
-#define AFR_WPE_ATTR_6 AFR_WPE_ATTR_N(6)
-#define AFR_WPE_ATTR_7 AFR_WPE_ATTR_N(7)
-#define AFR_WPE_ATTR_8 AFR_WPE_ATTR_N(8)
-
 namespace afr {
 
 template <typename real> struct Tiny;
@@ -391,11 +359,12 @@ __host__ __device__ __forceinline__ void viscous_flux_dot(const real q[5], const
 struct CellWalk {
     int64_t it, hi, step;
     __device__ __forceinline__ CellWalk(int64_t n, int waves_per_block, int wid) {
-        const int nxcd = gridDim.x >= 8 ? 8 : 1;
-        const int xcd = blockIdx.x % nxcd, lb = blockIdx.x / nxcd;
-        step = (int64_t)(gridDim.x / nxcd) * waves_per_block;
-        it = n * xcd / nxcd + (int64_t)lb * waves_per_block + wid;
-        hi = n * (xcd + 1) / nxcd;
+        // shifts: a 64-bit division takes some 150 instructions at the start of every kernel
+        const int sh = gridDim.x >= 8 ? 3 : 0;
+        const int xcd = blockIdx.x & ((1 << sh) - 1), lb = blockIdx.x >> sh;
+        step = (int64_t)(gridDim.x >> sh) * waves_per_block;
+        it = (n * xcd >> sh) + (int64_t)lb * waves_per_block + wid;
+        hi = n * (xcd + 1) >> sh;
     }
 };
 

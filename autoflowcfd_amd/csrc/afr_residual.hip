@@ -691,8 +691,6 @@ int run_sst(const AfrMeshDesc& d, const StateOff& so, const void* U, void* k, vo
     a.crec = (real*)d.work_crec;
     a.det = (const real*)d.det;
     a.adj = (const real*)d.adj;
-    a.E0 = (const real*)d.E[0];
-    a.E1 = (const real*)d.E[1];
     a.slot_nb = d.slot_nb;
     a.slot_blk = d.slot_blk;
     a.slot_mask = d.slot_mask;
@@ -724,13 +722,9 @@ int run_sst(const AfrMeshDesc& d, const StateOff& so, const void* U, void* k, vo
             b.cell_begin = ct == 0 ? 0 : d.n_prism;
             b.n_cells = ct == 0 ? d.n_prism : d.n_cells - d.n_prism;
             b.D = (const real*)d.D[ct];
-            b.Dsp_w = (const real*)d.dsp_w[ct];
-            b.Dsp_i = d.dsp_i[ct];
-            b.Esp_w = (const real*)d.esp_w[ct];
-            b.Esp_i = d.esp_i[ct];
+            b.E = (const real*)d.E[ct];
             b.schedule = ct == 0 ? d.prism_schedule : nullptr;
             b.grid_cap = d.grid_cap[phase == 0 ? AFR_K_SST_CELL : AFR_K_SST_UPDATE];
-            b.variant = phase == 0 ? d.variant[AFR_K_SST_CELL] : 0;
             if (b.n_cells <= 0) continue;
             int rc;
             if (phase == 0)

@@ -20,7 +20,10 @@
 //                 (src/autoflowcfd/core/fr_solver/turbulence.py:112-121 uses a KD-tree)
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "../../include/afr.h"
+#include "afr_meanflow.hpp"
 #include "afr_physics.hpp"
 #include "afr_sst.hpp"
 #include "afr_sst_point.hpp"
@@ -32,270 +35,305 @@ namespace afr_sst {
 
 constexpr int kWaves = 4;
 
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+using afr_mean::V4;
+using afr_mean::ld4;
+using afr_mean::st4;
+using afr_mean::wave_sync;
+template <typename real> struct V2;
+template <> struct V2<float> { typedef float type __attribute__((ext_vector_type(2))); };
+template <> struct V2<double> { typedef double type __attribute__((ext_vector_type(2))); };
+
+// acc += w x by components: a vector product would keep w splatted over as many registers
+template <typename V, typename real> __device__ __forceinline__ void fma_to(V& acc, real w, V x) {
+    if constexpr (std::is_same<V, real>::value) acc += w * x;
+    else {
+#pragma unroll
+        for (int q = 0; q < (int)(sizeof(V) / sizeof(real)); ++q) acc[q] += w * x[q];
+    }
 }
 
-__device__ __forceinline__ int slot_code(int slot) { return slot < 3 ? slot : (slot == 3 ? 4 : 5); }
-
+// Lanes of a wavefront: (cell, solution point), LW lanes per cell: 8 cells at P1, 2 (27 of 32 lanes) at P2
 template <int P, int CT> struct SO {
     static constexpr int N1 = P + 1, NS = N1 * N1 * N1, NFP = N1 * N1, NSLOT = CT == 0 ? 5 : 4;
+    static constexpr int LW = NS <= 8 ? 8 : 32, CPW = 64 / LW;
 };
 
 // ------------------------------------------------------------------ per-cell sources and volume terms
-// One wave per cell.  The contractions (gradients D x, face traces E x, volume divergence D F)
-// run in the storage precision on per-cell perturbations x - x_0 (x_0: the value at the cell's
-// first solution point; D rows sum to zero and E rows to one, so D x = D (x - x_0) and
-// E x = x_0 + E (x - x_0)), which keeps FP32 contractions as accurate as FP64 ones on FP32
-// data.  The SST source terms are FP64 (the blend functions FP32 on the FP32 path).
-// non-zeros per sparse derivative row (prism: N1, N1^2, N1; tet: N1, N1^2, N1^3) and per
-// face-trace row (prism N1^2, tet N1^3): the widths of the mesh's sparse D / E tables
-template <int P, int CT> struct SW {
-    static constexpr int N1 = P + 1, NS = N1 * N1 * N1;
-    static constexpr int W0 = N1, W1 = N1 * N1, W2 = CT == 0 ? N1 : NS;
-    static constexpr int WM = W2 > W1 ? W2 : W1;
-    static constexpr int KE = CT == 0 ? N1 * N1 : NS;
-};
-
-// cells per wavefront of the cell kernel (its tile variant, PAIR): two half-waves of 32 lanes when
-// a cell has at most 32 solution points, so the per-point phases (FP64 sources) keep 54 of 64
-// lanes busy at P2 (PAIR 1), or one cell per wavefront (PAIR 0); the autotuner picks per mesh
-template <int P, int CT, int PAIR> struct SstCellPlan {
-    static constexpr int NS = (P + 1) * (P + 1) * (P + 1);
-    static constexpr int CPW = (PAIR && CT == 0 && NS <= 32) ? 2 : 1;   // cells per wave (prisms)
-    static constexpr int LW = 64 / CPW;                             // lanes per cell
-};
-
-template <int P, int CT, typename real, int PAIR>
-__global__ void __launch_bounds__(64 * kWaves) AFR_WPE_SEL(AFR_WPE_SST_CELL) k_sst_cell(SstArgs<real> a) {
+// The contractions (gradients D x, face traces E x, volume divergence D F) run in the storage
+// precision on per-cell perturbations x - x_0 (x_0: the value at the cell's first solution point; D
+// rows sum to zero and E rows to one, so D x = D (x - x_0) and E x = x_0 + E (x - x_0)), which keeps
+// FP32 contractions as accurate as FP64 ones on FP32 data.  The SST source terms are FP64 (the blend
+// functions FP32 on the FP32 path).
+//
+// A lane keeps the non-zeros of its derivative rows in registers for the whole kernel (d/da: an a
+// line, d/db: an (a, b) plane, d/dc: a c line of a prism, every point of a tet from LDS), and those
+// of XX are dealt out with the N1^2-wide b face last, so that
+// only the last round is wide).  Fields lie in LDS as 16-byte vectors of perturbations, so a non-zero
+// costs one or two LDS reads and no subtraction.  Traces are written for slots that own a face
+// record only: no other is read.
+//
+// Bound: FP64 source arithmetic and HBM together (4.3 GB at 82^3 P2 FP32).  Measured there 1165 us,
+// before (rows as index / weight tables in LDS, one 4-byte read and one subtraction per product, every
+// slot's trace) 1938; 152k P1 prisms FP32 95 us (252, 24 of 64 lanes busy).
+template <int P, int CT> struct SC {
     using O = SO<P, CT>;
-    using W = SW<P, CT>;
-    using L = SstCellPlan<P, CT, PAIR>;
-    constexpr int NS = O::NS, WM = W::WM, KE = W::KE, CPW = L::CPW, LW = L::LW;
-    constexpr int WD[3] = {W::W0, W::W1, W::W2};
-    // per-SP record (12): rho, u, v, w, k, omega, Gk, Gw (the face-trace fields, contiguous),
-    // m1, m2, m3 (the momentum gradient fields), pad
-    constexpr int NF = 12, G_ = 16;  // gradient record: grad m (9), grad k (3), grad omega (3), pad
-    constexpr int NFP = O::NFP, NSLOT = O::NSLOT;
-    constexpr int PER_CELL = NS * NF + NS * G_ + NS * 8;
-    // sparse derivative and face-trace rows (the D / E non-zeros only)
-    __shared__ real s_Dw[3 * NS * WM];
-    __shared__ int s_Di[3 * NS * WM];
-    __shared__ real s_Ew[5 * NFP * KE];
-    __shared__ int s_Ei[5 * NFP * KE];
-    __shared__ __attribute__((aligned(16))) real s_w[kWaves][CPW * PER_CELL];
-    for (int i = threadIdx.x; i < 3 * NS * WM; i += 64 * kWaves) {
-        s_Dw[i] = a.Dsp_w[i];
-        s_Di[i] = a.Dsp_i[i];
+    static constexpr int NS = O::NS, NI = O::NSLOT * O::NFP, RD = (NI + O::LW - 1) / O::LW;
+    static constexpr int PER = (NS * 14 + 3) / 4 * 4;           // two 4-vectors and three pairs per point
+    static constexpr int DT = CT == 1 ? NS * (NS | 1) : 1;      // d/dc rows of a tet
+    // flux points in the order they are dealt out: prism slots 0, 1, 3, 4, 2
+    static constexpr __device__ int slot(int o) {
+        const int q = o / O::NFP;
+        return CT == 1 ? q : (q < 2 ? q : (q == 4 ? 2 : q + 1));
     }
-    for (int i = threadIdx.x; i < 5 * NFP * KE; i += 64 * kWaves) {
-        s_Ew[i] = a.Esp_w[i];
-        s_Ei[i] = a.Esp_i[i];
+    // non-zeros of a prism's trace rows in round r
+    static constexpr int nnz(int r) { return (r + 1) * O::LW > 4 * O::NFP ? O::N1 * O::N1 : O::N1; }
+    static constexpr int first(int r) { return r == 0 ? 0 : first(r - 1) + nnz(r - 1); }
+    static constexpr int ET = CT == 1 ? NI * (NS | 1) : first(RD) * O::LW;   // trace rows: tets (row, point)
+    template <typename real> static constexpr int wpe() { return sizeof(real) == 4 ? (P == 2 && CT == 0 ? 3 : 4) : (P == 2 && CT == 1 ? 1 : 2); }
+};
+
+template <int P, int CT, typename real>
+__global__ void __launch_bounds__(64 * kWaves)
+    __attribute__((amdgpu_waves_per_eu(SC<P, CT>::template wpe<real>()))) k_sst_cell(SstArgs<real> a) {
+    using O = SO<P, CT>;
+    using L = SC<P, CT>;
+    using v4 = typename V4<real>::type;
+    using v2 = typename V2<real>::type;
+    constexpr int N1 = O::N1, NS = O::NS, NFP = O::NFP, LW = O::LW, CPW = O::CPW, RS = NS | 1;
+    __shared__ __attribute__((aligned(16))) real s_w[kWaves][CPW * L::PER];
+    __shared__ real s_dc[L::DT], s_e[L::ET];
+    __shared__ int s_eb[L::RD * LW];
+    const int tid = threadIdx.x, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t0 = tid & 63;
+    if constexpr (CT == 1) {
+        for (int q = tid; q < NS * NS; q += 64 * kWaves) s_dc[(q / NS) * RS + q % NS] = a.D[2 * NS * NS + q];
+        for (int q = tid; q < L::NI * NS; q += 64 * kWaves) s_e[(q / NS) * RS + q % NS] = a.E[q];
+        __syncthreads();
     }
-    __syncthreads();
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = threadIdx.x & 63;
-    const int h = t / LW, tl = t % LW;               // cell of the wave, lane within the cell
-    real* sv = s_w[wid] + h * PER_CELL;  // [s][NF]
-    real* sg = sv + NS * NF;             // [s][G_]
-    real* sF = sg + NS * G_;             // [j][f][4]: contravariant convective + diffusive flux of k (f=0), omega (f=1), m = 0..2
+    real wa[N1], wb[N1 * N1], wc[N1];
+    {
+    const int tl = t0 % LW, sp = tl < NS ? tl : 0, i = sp / (N1 * N1), j = (sp / N1) % N1, k = sp % N1;
+#pragma unroll
+    for (int q = 0; q < N1; ++q) {
+        wa[q] = a.D[sp * NS + (q * N1 + j) * N1 + k];
+        wc[q] = CT == 0 ? a.D[(2 * NS + sp) * NS + (i * N1 + j) * N1 + q] : real(0);
+    }
+#pragma unroll
+    for (int q = 0; q < N1 * N1; ++q) wb[q] = a.D[(NS + sp) * NS + q * N1 + k];
+    }
+    // trace rows of the lanes' flux points: weights and first point
+    if constexpr (CT == 0) {
+        for (int x = tid; x < L::RD * LW; x += 64 * kWaves) {
+            const int r = x / LW, o = x < L::NI ? x : 0, slot = L::slot(o), fp = o % NFP;
+            const int y = fp / N1, z = fp % N1;      // a: (b, c), b: (a, c), c: (a, b)
+            const int n = slot == 2 ? N1 * N1 : N1, st = slot < 2 ? N1 * N1 : (slot == 2 ? N1 : 1);
+            const int b = slot < 2 ? y * N1 + z : (slot == 2 ? z : (y * N1 + z) * N1);
+            s_eb[x] = b;
+            for (int q = 0; q < L::nnz(r); ++q)
+                s_e[(L::first(r) + q) * LW + x % LW] = q < n ? a.E[(slot * NFP + fp) * NS + b + q * st] : real(0);
+        }
+        __syncthreads();
+    }
     const double mu = a.mu_molecular;
     const int64_t n_units = (a.n_cells + CPW - 1) / CPW;
     for (CellWalk cw(n_units, kWaves, wid); cw.it < cw.hi; cw.it += cw.step) {
-        // list positions CPW it + h; a missing second cell leaves its half-wave idle
-        const int64_t pos0 = cw.it * CPW;
-        const int64_t c0 = walk_cell(a.schedule, pos0);
-        const int64_t c1 = (CPW == 2 && pos0 + 1 < a.n_cells) ? walk_cell(a.schedule, pos0 + 1) : c0;
-        const bool live = h == 0 || pos0 + 1 < a.n_cells;
-        const int64_t cell = a.cell_begin + (h == 0 ? c0 : c1);
-        const int64_t cb = cell * NS;                // first solution point of the cell
-        // the lane's wall distance and adjugate (used by the same lane in the point phase) are
-        // loaded here with the state
-        real d_s = real(0), adj_s[9];
+        const int64_t c0 = cw.it * CPW;
+        // the lane's indexes are formed anew for every cell: held over the loop, the addresses made from
+        // them would take the registers that the contractions need
+        const int t = afr_mean::lane_fresh(t0);
+        const int h = t / LW, tl = t % LW;               // cell of the wave, lane within the cell
+        const int sp = tl < NS ? tl : 0, i = sp / (N1 * N1), j = (sp / N1) % N1, k = sp % N1;
+        real* const sA = s_w[wid] + h * L::PER;          // m1, m2, m3, k, then rho, u, v, w
+        real* const sB = sA + NS * 4;                    // k, omega, Gamma_k, Gamma_omega
+        real* const sV = sA + NS * 8;                    // omega, then the contravariant fluxes [m][s][k, omega]
+        // row m of this lane's point applied to a 4-vector field / a field of stride 1 / of pairs
+        auto apply = [&](int m, auto zero, auto get) {
+            auto acc = zero;
+            if (m == 0) {
+    #pragma unroll
+                for (int q = 0; q < N1; ++q) fma_to(acc, wa[q], get(q * N1 * N1 + j * N1 + k));
+            } else if (m == 1) {
+    #pragma unroll
+                for (int q = 0; q < N1 * N1; ++q) fma_to(acc, wb[q], get(q * N1 + k));
+            } else if constexpr (CT == 0) {
+    #pragma unroll
+                for (int q = 0; q < N1; ++q) fma_to(acc, wc[q], get((i * N1 + j) * N1 + q));
+            } else {
+    #pragma unroll 4
+                for (int q = 0; q < NS; ++q) fma_to(acc, s_dc[sp * RS + q], get(q));
+            }
+            return acc;
+        };
+        auto at0 = [&](real x) { return __shfl(x, h * LW); };   // the value at the cell's first point
+        const int nc = (int)(a.n_cells - c0 < CPW ? a.n_cells - c0 : CPW);
+        const bool live = tl < NS && h < nc;
+        const int64_t cell = a.cell_begin + c0 + (h < nc ? h : 0);
+        const int64_t pt = cell * NS + sp;
+        // codes of the faces whose records this cell owns
+        int own = 0;
+        if (tl < kInc) {
+            const int e = a.inc[cell * kInc + tl];
+            own = e >= 0 && !(e & 8) ? 1 << (e & 7) : 0;
+        }
 #pragma unroll
-        for (int q = 0; q < 9; ++q) adj_s[q] = real(0);
-        if (live && tl < NS) {
-            const int64_t i = cb + tl;
-            d_s = a.d_wall[i];
+        for (int m = 1; m < kInc; m <<= 1) own |= __shfl_xor(own, m);
+        if constexpr (LW > kInc) own = __shfl(own, h * LW);
+        real ad[9], u5[5];
 #pragma unroll
-            for (int q = 0; q < 9; ++q) adj_s[q] = a.adj[i * 9 + q];
-            real u5[5];
+        for (int q = 0; q < 9; ++q) ad[q] = a.adj[pt * 9 + q];
+        const real ks0 = a.k[pt], ws0 = a.w[pt], dw = a.d_wall[pt], idet = recip(a.det[pt]);
+        {
             double off[5];
             a.so.row(cell, off);
 #pragma unroll
             for (int v = 0; v < 5; ++v)
-                u5[v] = a.so.mode ? (real)((double)a.U[i * 5 + v] + off[v]) : a.U[i * 5 + v];
-            const real rho = u5[0] > real(1e-10) ? u5[0] : real(1e-10);
-            real* r = sv + tl * NF;
-            r[0] = rho;
-            r[1] = u5[1] / rho;
-            r[2] = u5[2] / rho;
-            r[3] = u5[3] / rho;
-            r[4] = a.k[i];
-            r[5] = a.w[i];
-            r[8] = u5[1];
-            r[9] = u5[2];
-            r[10] = u5[3];
+                u5[v] = a.so.mode ? (real)((double)a.U[pt * 5 + v] + off[v]) : a.U[pt * 5 + v];
+        }
+        const real rr = u5[0] > real(1e-10) ? u5[0] : real(1e-10);
+        const real k0 = at0(ks0), w0 = at0(ws0);
+        {
+            const real m0[3] = {at0(u5[1]), at0(u5[2]), at0(u5[3])};
+            if (live) {
+                st4(sA + sp * 4, (v4){u5[1] - m0[0], u5[2] - m0[1], u5[3] - m0[2], ks0 - k0});
+                sV[sp] = ws0 - w0;
+            }
         }
         wave_sync();
-        // gradients of m1, m2, m3, k, omega: lane (s, field), sparse rows, perturbations about SP 0
-        for (int o = tl; o < 5 * NS; o += LW) {
-            if (!live) break;
-            const int s = o / 5, f = o % 5;
-            const int src = f < 3 ? 8 + f : 4 + (f - 3);
-            const real x0 = sv[src];
-            real d[3];
+        real gm[3][3], gk[3], gw[3];
+        {
+            v4 d[3];
+            real e[3];
 #pragma unroll
             for (int m = 0; m < 3; ++m) {
-                real acc = 0;
-#pragma unroll
-                for (int k = 0; k < WD[m]; ++k) {
-                    const int idx = (m * NS + s) * WM + k;
-                    acc += s_Dw[idx] * (sv[s_Di[idx] * NF + src] - x0);
-                }
-                d[m] = acc;
+                d[m] = apply(m, (v4){0, 0, 0, 0}, [&](int q) { return ld4(sA + q * 4); });
+                e[m] = apply(m, real(0), [&](int q) { return sV[q]; });
+                __builtin_amdgcn_sched_barrier(0);   // one row's loads in flight at a time: registers
             }
-            const real* ad = a.adj + (cb + s) * 9;
-            const real idet = real(1) / a.det[cb + s];
-            const int base = f < 3 ? f * 3 : 9 + (f - 3) * 3;
-#pragma unroll
-            for (int n = 0; n < 3; ++n) sg[s * G_ + base + n] = (ad[0 * 3 + n] * d[0] + ad[1 * 3 + n] * d[1] + ad[2 * 3 + n] * d[2]) * idet;
-        }
-        wave_sync();
-        if (live && tl < NS) {
-            const int s = tl;
-            const int64_t i = cb + s;
-            const real* r = sv + s * NF;
-            const real* gs = sg + s * G_;
-            const double rho = (double)r[0], k = (double)r[4], w = (double)r[5];
-            const double d = (double)d_s;
-            // strain rate of the momentum gradient
-            double S2 = 0.0;
-#pragma unroll
-            for (int p = 0; p < 3; ++p)
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    const double sij = 0.5 * ((double)gs[p * 3 + q] + (double)gs[q * 3 + p]);
-                    S2 += sij * sij;
-                }
-            const double S = sqrt(2.0 * S2);
-            // clipped gradients of k and omega
-            double gk[3], gw[3];
 #pragma unroll
             for (int n = 0; n < 3; ++n) {
-                gk[n] = (double)gs[9 + n];
-                gw[n] = (double)gs[12 + n];
+                const v4 g = (ad[n] * d[0] + ad[3 + n] * d[1] + ad[6 + n] * d[2]) * idet;
+                gm[0][n] = g[0];
+                gm[1][n] = g[1];
+                gm[2][n] = g[2];
+                gk[n] = g[3];
+                gw[n] = (ad[n] * e[0] + ad[3 + n] * e[1] + ad[6 + n] * e[2]) * idet;
             }
-            const double mk = sqrt(gk[0] * gk[0] + gk[1] * gk[1] + gk[2] * gk[2]);
-            const double mw = sqrt(gw[0] * gw[0] + gw[1] * gw[1] + gw[2] * gw[2]);
-            if (mk > 1e6) {
-                const double f = dmin(dmax(1e6 / dmax(mk, 1e-10), 0.0), 1.0);
-                gk[0] *= f; gk[1] *= f; gk[2] *= f;
+        }
+        // sources of the point (FP64), mu = 1.8e-5 as the reference's source terms
+        const double rho = (double)rr, kd = (double)ks0, wd = (double)ws0, dd = (double)dw;
+        const double irho = recip(dmax(rho, 1e-10));
+        real Gk, Gw;
+        {
+            double S2 = 0.0;
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                const double q = (double)gm[p][p], o = (double)gm[p][(p + 1) % 3] + (double)gm[(p + 1) % 3][p];
+                S2 += q * q + 0.5 * (o * o);
             }
-            if (mw > 1e6) {
-                const double f = dmin(dmax(1e6 / dmax(mw, 1e-10), 0.0), 1.0);
-                gw[0] *= f; gw[1] *= f; gw[2] *= f;
+            const double SS2 = 2.0 * S2, S = sqrt(SS2);
+            // clipped gradients of k and omega
+            double fk = 1.0, fw = 1.0, mk = 0.0, mw = 0.0, gd = 0.0;
+#pragma unroll
+            for (int n = 0; n < 3; ++n) {
+                mk += (double)gk[n] * (double)gk[n];
+                mw += (double)gw[n] * (double)gw[n];
             }
-            const double gdot = gk[0] * gw[0] + gk[1] * gw[1] + gk[2] * gw[2];
-            // sources (mu = 1.8e-5 as the reference's source terms)
+            if (mk > 1e12) fk = dmin(dmax(1e6 / dmax(sqrt(mk), 1e-10), 0.0), 1.0);
+            if (mw > 1e12) fw = dmin(dmax(1e6 / dmax(sqrt(mw), 1e-10), 0.0), 1.0);
+#pragma unroll
+            for (int n = 0; n < 3; ++n) gd += (fk * (double)gk[n]) * (fw * (double)gw[n]);
             const double musrc = 1.8e-5;
-            const double irho = recip(dmax(rho, 1e-10));   // one reciprocal for the four uses
-            const double nu = musrc * irho;
-            const double ks = dmin(k, 1e40), wsf = dmax(dmin(w, 1e40), 1e-10);
-            const double CD = dmax(2.0 * rho * SW2 / wsf * gdot, 1e-10);
-            const double F1 = Blend<real>::F1(ks, wsf, d, nu, rho, CD);
-            const double F2 = Blend<real>::F2(ks, wsf, d, nu);
+            const double ks = dmin(kd, 1e40), wsf = dmax(dmin(wd, 1e40), 1e-10);
+            const double cross = 2.0 * rho * SW2 * recip(wsf) * gd;
+            double F1, F2;
+            __builtin_amdgcn_sched_barrier(0);
+            Blend<real>::both(ks, wsf, dd, musrc * irho, rho, dmax(cross, 1e-10), F1, F2);
             const double beta = F1 * B1 + (1.0 - F1) * B2;
-            double nut;
-            {
-                const double kk = dmax(ks, 1e-10), ww = dmax(wsf, 1e-10), SS = dmax(S, 1e-10);
-                nut = A1 * kk / dmax(A1 * ww, F2 * SS);
-                nut = dmin(nut, 1.0e5 * musrc * irho);
-                nut = isfinite(nut) ? nut : 0.0;
-            }
-            const double Pk = dmin(nut * rho * S * S, 10.0 * BSTAR * rho * ks * wsf);
-            double Sk = Pk - rho * BSTAR * ks * wsf;
+            const double kk = dmax(ks, 1e-10), SS = dmax(S, 1e-10);
+            double nut = A1 * kk * recip(dmax(A1 * wsf, F2 * SS));
+            nut = dmin(nut, 1.0e5 * musrc * irho);
+            nut = isfinite(nut) ? nut : 0.0;
+            const double rnut = rho * nut, Dk = BSTAR * rho * ks * wsf;
+            double Sk = dmin(rnut * S * S, 10.0 * Dk) - Dk;
             const double g1 = B1 / BSTAR - SW1 * KAP * KAP / sqrt(BSTAR);
             const double g2 = B2 / BSTAR - SW2 * KAP * KAP / sqrt(BSTAR);
             const double gam = F1 * g1 + (1.0 - F1) * g2;
-            double Sw = rho * gam * S * S - rho * beta * wsf * wsf + 2.0 * rho * (1.0 - F1) * SW2 / wsf * gdot;
+            double Sw = rho * gam * S * S - rho * beta * wsf * wsf + (1.0 - F1) * cross;
             Sk = finite_or(Sk, 0.0);
             Sw = finite_or(Sw, 0.0);
-            const double ir = irho;
-            a.src[i * 3 + 0] = (real)(Sk * ir);
-            a.src[i * 3 + 1] = (real)(Sw * ir);
-            a.src[i * 3 + 2] = (real)beta;
-            a.nu_t[i] = (real)nut;
-            a.mu_t[i] = (real)(rho * nut);
-            // diffusivities with the transport's own F1 (molecular mu, raw k / omega)
-            const double wsaf = dmax(w, 1e-10);
-            const double CDt = dmax(2.0 * rho * SW2 / wsaf * gdot, 1e-10);
-            const double F1t = Blend<real>::F1(k, w, d, mu * irho, rho, CDt);
-            const double rnut = rho * nut;
-            const double Gk = mu + (F1t * SK1 + (1.0 - F1t) * SK2) * rnut;
-            const double Gw = mu + (F1t * SW1 + (1.0 - F1t) * SW2) * rnut;
-            real* rw = sv + s * NF;
-            rw[6] = (real)Gk;
-            rw[7] = (real)Gw;
-            real* nbp = a.nbp + i * 4;
-            nbp[0] = (real)k;
-            nbp[1] = (real)w;
-            nbp[2] = (real)Gk;
-            nbp[3] = (real)Gw;
-            // contravariant transport fluxes (raw gradients in the diffusion), convective +
-            // diffusive summed per field: sF[s][f][m]
-            const real* ad = adj_s;
-            const real rr = r[0];
-            const real ru[3] = {rr * r[1], rr * r[2], rr * r[3]};
-            const real gkr = (real)Gk, gwr = (real)Gw, kr = r[4], wr = r[5];
-            real* fo = sF + s * 8;
-#pragma unroll
-            for (int m = 0; m < 3; ++m) {
-                const real am[3] = {ad[m * 3 + 0], ad[m * 3 + 1], ad[m * 3 + 2]};
-                const real fr = am[0] * ru[0] + am[1] * ru[1] + am[2] * ru[2];
-                fo[0 * 4 + m] = fr * kr + gkr * (am[0] * gs[9] + am[1] * gs[10] + am[2] * gs[11]);
-                fo[1 * 4 + m] = fr * wr + gwr * (am[0] * gs[12] + am[1] * gs[13] + am[2] * gs[14]);
+            // diffusivities with the transport's own F1 (molecular mu, raw k / omega): the same
+            // arguments as the sources' F1 unless mu differs or k, omega were clipped
+            double F1t = F1;
+            if (!(mu == musrc && kd <= 1e40 && wd <= 1e40)) {
+                const double CDt = dmax(2.0 * rho * SW2 / dmax(wd, 1e-10) * gd, 1e-10);
+                F1t = Blend<real>::F1(kd, wd, dd, mu * irho, rho, CDt);
             }
+            Gk = (real)(mu + (F1t * SK1 + (1.0 - F1t) * SK2) * rnut);
+            Gw = (real)(mu + (F1t * SW1 + (1.0 - F1t) * SW2) * rnut);
+            if (live) {
+                a.src[pt * 3 + 0] = (real)(Sk * irho);
+                a.src[pt * 3 + 1] = (real)(Sw * irho);
+                a.src[pt * 3 + 2] = (real)beta;
+                a.nu_t[pt] = (real)nut;
+                a.mu_t[pt] = (real)rnut;
+                st4(a.nbp + pt * 4, (v4){ks0, ws0, Gk, Gw});
+            }
+        }
+        const v4 xa = {rr, (real)((double)u5[1] * irho), (real)((double)u5[2] * irho), (real)((double)u5[3] * irho)};
+        const v4 xb = {ks0, ws0, Gk, Gw};
+        const v4 a0 = {at0(xa[0]), at0(xa[1]), at0(xa[2]), at0(xa[3])};
+        const v4 b0 = {k0, w0, at0(Gk), at0(Gw)};
+        wave_sync();
+        // contravariant transport fluxes (raw gradients in the diffusion), convective + diffusive
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const real fr = ad[m * 3] * (rr * xa[1]) + ad[m * 3 + 1] * (rr * xa[2]) + ad[m * 3 + 2] * (rr * xa[3]);
+            const real fk = fr * ks0 + Gk * (ad[m * 3] * gk[0] + ad[m * 3 + 1] * gk[1] + ad[m * 3 + 2] * gk[2]);
+            const real fw = fr * ws0 + Gw * (ad[m * 3] * gw[0] + ad[m * 3 + 1] * gw[1] + ad[m * 3 + 2] * gw[2]);
+            const v2 f = {fk - at0(fk), fw - at0(fw)};
+            if (live) *reinterpret_cast<v2*>(sV + (m * NS + sp) * 2) = f;
+        }
+        if (live) {
+            st4(sA + sp * 4, xa - a0);
+            st4(sB + sp * 4, xb - b0);
         }
         wave_sync();
-        // owner-side face traces of (rho, u, v, w, k, omega, Gamma_k, Gamma_omega): lane (slot, flux point)
-        for (int o = tl; o < NSLOT * NFP; o += LW) {
-            if (!live) break;
-            const int slot = o / NFP, fp = o % NFP;
-            real x0[kPack], tr[kPack];
+        // owner-side face traces of (rho, u, v, w, k, omega, Gamma_k, Gamma_omega)
 #pragma unroll
-            for (int q = 0; q < kPack; ++q) {
-                x0[q] = sv[q];
-                tr[q] = 0;
-            }
+        for (int r = 0; r < L::RD; ++r) {
+            const int o = tl + r * LW, slot = L::slot(o), fp = o % NFP;
+            if (o < L::NI && h < nc && (own >> (slot < 3 ? slot : slot + 1) & 1)) {
+                v4 ta = a0, tb = b0;
+                if constexpr (CT == 0) {
+                    const int b = s_eb[o], st = slot < 2 ? N1 * N1 : (slot == 2 ? N1 : 1);
 #pragma unroll
-            for (int k = 0; k < KE; ++k) {
-                const int e = (slot * NFP + fp) * KE + k;
-                const real ej = s_Ew[e];
-                const real* x = sv + s_Ei[e] * NF;
-#pragma unroll
-                for (int q = 0; q < kPack; ++q) tr[q] += ej * (x[q] - x0[q]);
-            }
-            real* ov = a.pack + ((cell * 5 + slot) * NFP + fp) * kPack;
-#pragma unroll
-            for (int q = 0; q < kPack; ++q) ov[q] = x0[q] + tr[q];
-        }
-        // volume terms: -(D.F)/det for k and omega, perturbations about SP 0
-        for (int o = tl; o < 2 * NS; o += LW) {
-            if (!live) break;
-            const int s = o >> 1, f = o & 1;
-            real acc = 0;
-#pragma unroll
-            for (int m = 0; m < 3; ++m) {
-                const real f0 = sF[f * 4 + m];
-#pragma unroll
-                for (int k = 0; k < WD[m]; ++k) {
-                    const int idx = (m * NS + s) * WM + k;
-                    acc += s_Dw[idx] * (sF[s_Di[idx] * 8 + f * 4 + m] - f0);
+                    for (int q = 0; q < L::nnz(r); ++q) {
+                        const int x = q < N1 || slot == 2 ? b + q * st : 0;   // narrow rows: padding
+                        const real w = s_e[(L::first(r) + q) * LW + tl];
+                        fma_to(ta, w, ld4(sA + x * 4));
+                        fma_to(tb, w, ld4(sB + x * 4));
+                    }
+                } else {
+#pragma unroll 2
+                    for (int q = 0; q < NS; ++q) {
+                        const real e = s_e[o * RS + q];
+                        fma_to(ta, e, ld4(sA + q * 4));
+                        fma_to(tb, e, ld4(sB + q * 4));
+                    }
                 }
+                real* ov = a.pack + ((cell * 5 + slot) * NFP + fp) * kPack;
+                st4(ov, ta);
+                st4(ov + 4, tb);
             }
-            a.vol[(cb + s) * 2 + f] = -acc / a.det[cb + s];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // volume terms: -(D.F)/det for k and omega
+        {
+            v2 acc = {0, 0};
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+                acc += apply(m, (v2){0, 0}, [&](int q) { return *reinterpret_cast<const v2*>(sV + (m * NS + q) * 2); });
+            if (live) *reinterpret_cast<v2*>(a.vol + pt * 2) = -acc * idet;
         }
         wave_sync();
     }
@@ -381,98 +419,140 @@ __global__ void __launch_bounds__(256) k_sst_face(SstArgs<real> a) {
 }
 
 // ------------------------------------------------------------------ gather, outlier zeroing, update
-template <int P, int CT, typename real>
-__global__ void __launch_bounds__(64 * kWaves) AFR_WPE_SEL(AFR_WPE_SST_UPDATE) k_sst_update(SstArgs<real> a) {
-    using O = SO<P, CT>;
-    constexpr int N1 = O::N1, NS = O::NS, NFP = O::NFP;
-    __shared__ double s_t[kWaves][2 * NS];
-    __shared__ double s_fld[kWaves][2 * NS];
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = threadIdx.x & 63;
-    // per-point tables of the three cube axes (flux point of the point on each axis and the
-    // correction-function values at its coordinate), the same for every cell: staged once
-    __shared__ int s_fps[3 * NS];
-    __shared__ real s_gl[3 * NS], s_gr[3 * NS];
-    for (int q = threadIdx.x; q < 3 * NS; q += 64 * kWaves) {
-        s_fps[q] = a.fp_of_sp[q];
-        const int cs = a.coord_of_sp[q];
-        s_gl[q] = a.gL[cs];
-        s_gr[q] = a.gR[cs];
+// One lane per solution point takes both fields through gather, zeroing and update in registers.  The
+// outlier rule's certificate (at most (NS - 1) / 2 values below 1e-4 of the largest: then the median
+// is too large for any value to be zeroed) takes the maximum over the cell's lanes and counts in a
+// ballot, on values rounded to FP32: its margin of 1e-4 of the threshold covers the rounding, and
+// values that FP32 could not tell from zero or infinity go the exact way.
+// Bound: HBM and the gather of record corrections.  Measured (82^3 P2 FP32): 621 us, 1298 with one cell
+// per wavefront and the FP64 certificate through LDS; 152k P1 prisms 51 us (308).
+template <int LW> __device__ __forceinline__ float cell_max(float x) {
+    x = fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, false)));    // xor 1
+    x = fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xf, 0xf, false)));    // xor 2
+    x = fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x141, 0xf, 0xf, false)));   // half row
+    if constexpr (LW > 8) {
+        x = fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x140, 0xf, 0xf, false)));   // row
+        x = fmaxf(x, __shfl_xor(x, 16));
     }
-    __syncthreads();
-    double* st = s_t[wid];
-    double* sf = s_fld[wid];
-    for (CellWalk cw(a.n_cells, kWaves, wid); cw.it < cw.hi; cw.it += cw.step) {
-        const int64_t cell = a.cell_begin + walk_cell(a.schedule, cw.it);
-        if (t < 2 * NS) {
-            const int s = t >> 1, f = t & 1;
-            const int64_t i = cell * NS + s;
-            const double det = (double)a.det[i];
-            int fps[3];
-            double gl[3], gr[3];
+    return x;
+}
+
+template <int P, int CT, typename real>
+__global__ void __launch_bounds__(64 * kWaves) k_sst_update(SstArgs<real> a) {
+    using O = SO<P, CT>;
+    using v2 = typename V2<real>::type;
+    constexpr int NS = O::NS, NFP = O::NFP, LW = O::LW, CPW = O::CPW;
+    constexpr int k1 = (NS - 1) / 2, k2 = NS / 2;
+    __shared__ double s_x[kWaves][CPW * NS * 2], s_med[kWaves][CPW * 4];
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = threadIdx.x & 63;
+    const int h = t / LW, tl = t % LW, s = tl < NS ? tl : 0;
+    const uint64_t group = (LW == 64 ? ~0ull : ((1ull << LW) - 1)) << (h * LW);
+    // flux point of the point on each axis, correction-function values at its coordinate
+    int fps[3];
+    real gl[3], gr[3];
 #pragma unroll
-            for (int ax = 0; ax < 3; ++ax) {
-                fps[ax] = s_fps[ax * NS + s];
-                gl[ax] = (double)s_gl[ax * NS + s];
-                gr[ax] = (double)s_gr[ax * NS + s];
-            }
-            int ev[kInc];
+    for (int ax = 0; ax < 3; ++ax) {
+        fps[ax] = a.fp_of_sp[ax * NS + s];
+        const int cs = a.coord_of_sp[ax * NS + s];
+        gl[ax] = a.gL[cs];
+        gr[ax] = a.gR[cs];
+    }
+    const int64_t n_units = (a.n_cells + CPW - 1) / CPW;
+    for (CellWalk cw(n_units, kWaves, wid); cw.it < cw.hi; cw.it += cw.step) {
+        const int64_t c0 = cw.it * CPW;
+        const int nc = (int)(a.n_cells - c0 < CPW ? a.n_cells - c0 : CPW);
+        const bool live = tl < NS && h < nc;
+        const int64_t pos = c0 + (h < nc ? h : 0);
+        const int64_t cell = a.cell_begin + (a.schedule ? a.schedule[pos] : pos);
+        const int64_t i = cell * NS + s;
+        int ev[kInc];
 #pragma unroll
-            for (int q = 0; q < kInc; ++q) ev[q] = a.inc[cell * kInc + q];
-            double cv[kInc];
+        for (int q = 0; q < kInc; ++q) ev[q] = a.inc[cell * kInc + q];
+        v2 cv[kInc];
 #pragma unroll
-            for (int q = 0; q < kInc; ++q) {
-                const int e = ev[q];
-                const int axis = (e & 7) >> 1;
-                const int fp = axis == 0 ? fps[0] : (axis == 1 ? fps[1] : fps[2]);
-                cv[q] = e < 0 ? 0.0 : (double)a.crec[((int64_t)(e >> 4) * NFP + fp) * 2 + f];
-            }
-            double acc = 0.0;
-#pragma unroll
-            for (int q = 0; q < kInc; ++q) {
-                const int e = ev[q];
-                if (e < 0) continue;
-                const int role = (e >> 3) & 1;
-                const int code = e & 7;
-                const int axis = code >> 1;
-                const double g = (code & 1) ? (axis == 0 ? gr[0] : (axis == 1 ? gr[1] : gr[2]))
-                                            : (axis == 0 ? gl[0] : (axis == 1 ? gl[1] : gl[2]));
-                acc += (role == 0 ? -1.0 : 1.0) * g * cv[q];
-            }
-            double off[5];
-            a.so.row(cell, off);
-            const double rho = dmax((double)a.U[i * 5] + off[0], 1e-10);
-            st[t] = ((double)a.vol[i * 2 + f] + acc / det) / rho;
-            sf[t] = fabs((double)(f == 0 ? a.k[i] : a.w[i]));
+        for (int q = 0; q < kInc; ++q) {
+            const int e = ev[q], axis = (e & 7) >> 1;
+            const int fp = axis == 0 ? fps[0] : (axis == 1 ? fps[1] : fps[2]);
+            cv[q] = (v2){0, 0};
+            if (e >= 0) cv[q] = *reinterpret_cast<const v2*>(a.crec + ((int64_t)(e >> 4) * NFP + fp) * 2);
         }
-        wave_sync();
+        const v2 vol = *reinterpret_cast<const v2*>(a.vol + i * 2);
+        const real det = a.det[i], u0 = a.U[i * 5], kr = a.k[i], wr = a.w[i], dtr = a.dt[i];
+        const real s0 = a.src[i * 3], s1 = a.src[i * 3 + 1], s2 = a.src[i * 3 + 2];
+        double off[5];
+        a.so.row(cell, off);
+        double ak = 0.0, aw = 0.0;
+#pragma unroll
+        for (int q = 0; q < kInc; ++q) {
+            const int e = ev[q], axis = (e & 7) >> 1;
+            const real gm = axis == 0 ? gl[0] : (axis == 1 ? gl[1] : gl[2]);
+            const real gp = axis == 0 ? gr[0] : (axis == 1 ? gr[1] : gr[2]);
+            double g = (double)((e & 1) ? gp : gm);
+            g = e < 0 ? 0.0 : ((e & 8) ? g : -g);
+            ak += g * (double)cv[q][0];
+            aw += g * (double)cv[q][1];
+        }
+        const double irho = recip(dmax((double)u0 + off[0], 1e-10)), idet = recip((double)det);
+        double tk = ((double)vol[0] + ak * idet) * irho, tw = ((double)vol[1] + aw * idet) * irho;
         // outlier zeroing per field (troubled_cell.py:339-408 with n_vars = 1, once for k and once
         // for omega, each field's own mean |value| as the reference magnitude), then non-finite
         // transport values -> 0 (transport.py:509-515)
-        outlier_zeroing<NS, 2, double>(st, [sf](int f) {
-            double m = 0.0;
-            for (int s2 = 0; s2 < NS; ++s2) m += sf[s2 * 2 + f];
-            return m / NS;
-        }, t);
-        wave_sync();
-        if (t < 2 * NS && !isfinite(st[t])) st[t] = 0.0;
-        wave_sync();
-        if (t < NS) {
-            const int s = t;
-            const int64_t i = cell * NS + s;
-            const double dt = (double)a.dt[i];
-            const double k = (double)a.k[i], w = (double)a.w[i];
+        {
+            const float xk = live ? (float)fabs(tk) : 0.0f, xw = live ? (float)fabs(tw) : 0.0f;
+            const float mk = cell_max<LW>(xk), mw = cell_max<LW>(xw);
+            const int nk = __popcll(__ballot(live && xk < mk * 1.0001e-4f) & group);
+            const int nw = __popcll(__ballot(live && xw < mw * 1.0001e-4f) & group);
+            const bool tiny = live && ((tk != 0.0 && mk < 1e-30f) || (tw != 0.0 && mw < 1e-30f));
+            if (__any(nk > k1 || nw > k1 || tiny)) {
+                double* const sx = s_x[wid] + h * NS * 2;
+                double* const sm = s_med[wid] + h * 4;
+                if (live) {
+                    sx[s * 2] = fabs(tk);
+                    sx[s * 2 + 1] = fabs(tw);
+                }
+                if (tl < 4) sm[tl] = -1.0;
+                wave_sync();
+                if (live) {   // rank of the lane's two values among the finite ones of their field
+                    for (int f = 0; f < 2; ++f) {
+                        const double x = fabs(f ? tw : tk);
+                        int lt = 0, le = 0;
+                        for (int q = 0; q < NS; ++q) {
+                            lt += sx[q * 2 + f] < x;
+                            le += sx[q * 2 + f] <= x;
+                        }
+                        if (lt <= k1 && k1 < le) sm[f * 2] = x;         // equal values write the same
+                        if (lt <= k2 && k2 < le) sm[f * 2 + 1] = x;
+                    }
+                }
+                wave_sync();
+                if (live) {
+                    for (int f = 0; f < 2; ++f) {
+                        const double m1 = sm[f * 2], m2 = sm[f * 2 + 1];
+                        if (m1 < 0.0 || m2 < 0.0) continue;             // NaN median: nothing zeroed
+                        double um = 0.0;
+                        for (int q = 0; q < NS; ++q) um += fabs((double)(f ? a.w : a.k)[cell * NS + q]);
+                        double ref = nan_max((NS % 2) ? m1 : 0.5 * (m1 + m2), 1e-9 * (um / NS));
+                        ref = nan_max(ref, Tiny<double>::v);
+                        if (fabs(f ? tw : tk) > 1e4 * ref) (f ? tw : tk) = 0.0;
+                    }
+                }
+                wave_sync();   // k and omega are read by every lane before any is updated
+            }
+        }
+        if (!isfinite(tk)) tk = 0.0;
+        if (!isfinite(tw)) tw = 0.0;
+        if (live) {
+            const double dt = (double)dtr, k = (double)kr, w = (double)wr;
             const double wsafe = dmax(w, 1e-10);
-            const double beta = (double)a.src[i * 3 + 2];
-            double dk = (double)a.src[i * 3 + 0] / (1.0 + dt * BSTAR * wsafe);
-            double dw = (double)a.src[i * 3 + 1] / (1.0 + dt * beta * wsafe);
-            dk = finite_or(dk, 0.0) + st[s * 2 + 0];
-            dw = finite_or(dw, 0.0) + st[s * 2 + 1];
+            double dk = (double)s0 / (1.0 + dt * BSTAR * wsafe);
+            double dw = (double)s1 / (1.0 + dt * (double)s2 * wsafe);
+            dk = finite_or(dk, 0.0) + tk;
+            dw = finite_or(dw, 0.0) + tw;
             dk = finite_or(dk, 0.0);
             dw = finite_or(dw, 0.0);
             if (a.rates) {
                 // residual evaluation only: dk/dt and domega/dt of the update, fields untouched
-                a.rates[i * 2 + 0] = (real)dk;
-                a.rates[i * 2 + 1] = (real)dw;
+                *reinterpret_cast<v2*>(a.rates + i * 2) = (v2){(real)dk, (real)dw};
             } else {
                 double kn = k + dt * dk, wn = w + dt * dw;
                 kn = isfinite(kn) ? kn : 1e-12;
@@ -481,7 +561,6 @@ __global__ void __launch_bounds__(64 * kWaves) AFR_WPE_SEL(AFR_WPE_SST_UPDATE) k
                 a.w[i] = (real)dmax(wn, 1e-12);
             }
         }
-        wave_sync();
     }
 }
 
@@ -518,22 +597,13 @@ __global__ void __launch_bounds__(256) k_wall_distance(const double* __restrict_
     }
 }
 
-template <int P, int CT, typename real, int PAIR>
-int launch_sst_cell_t(const SstArgs<real>& a, hipStream_t st) {
-    constexpr int CPW = SstCellPlan<P, CT, PAIR>::CPW;
-    const int64_t units = (a.n_cells + CPW - 1) / CPW;
-    hipLaunchKernelGGL((k_sst_cell<P, CT, real, PAIR>),
-                       dim3((unsigned)walk_grid(units, kWaves, a.grid_cap > 0 ? a.grid_cap : 4096)), dim3(64 * kWaves),
-                       0, st, a);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
 template <int P, int CT, typename real>
 int launch_sst_cell(const SstArgs<real>& a, hipStream_t st) {
     if (a.n_cells <= 0) return 0;
-    if (a.variant == 0) return launch_sst_cell_t<P, CT, real, 1>(a, st);
-    if (a.variant == 1) return launch_sst_cell_t<P, CT, real, 0>(a, st);
-    return -1;
+    const int64_t units = (a.n_cells + SO<P, CT>::CPW - 1) / SO<P, CT>::CPW;
+    hipLaunchKernelGGL((k_sst_cell<P, CT, real>), dim3((unsigned)walk_grid(units, kWaves, a.grid_cap > 0 ? a.grid_cap : 4096)),
+                       dim3(64 * kWaves), 0, st, a);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 template <int P, typename real>
@@ -556,8 +626,9 @@ int launch_sst_face(const SstArgs<real>& a, hipStream_t st) {
 template <int P, int CT, typename real>
 int launch_sst_update(const SstArgs<real>& a, hipStream_t st) {
     if (a.n_cells <= 0) return 0;
-    hipLaunchKernelGGL((k_sst_update<P, CT, real>), dim3((unsigned)walk_grid(a.n_cells, kWaves, a.grid_cap > 0 ? a.grid_cap : 4096)), dim3(64 * kWaves), 0,
-                       st, a);
+    const int64_t units = (a.n_cells + SO<P, CT>::CPW - 1) / SO<P, CT>::CPW;
+    hipLaunchKernelGGL((k_sst_update<P, CT, real>), dim3((unsigned)walk_grid(units, kWaves, a.grid_cap > 0 ? a.grid_cap : 4096)),
+                       dim3(64 * kWaves), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

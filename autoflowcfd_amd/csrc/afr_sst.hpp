@@ -22,7 +22,7 @@ struct SstArgs {
     const real* dt;               // (C, NS)
     real* nu_t;                   // (C, NS) out
     real* mu_t;                   // (C, NS) out: rho(U) nu_t
-    real* pack;                   // (C, 5, NFP, kPack) scratch: owner-side face traces of the pack
+    real* pack;                   // (C, 5, NFP, kPack) scratch: face traces of the pack, slots that own a record
     real* nbp;                    // (C, NS, 4) scratch: k, omega, Gamma_k, Gamma_omega at the solution points
     real* rates;                  // (C, NS, 2) out when non-null: dk/dt, domega/dt instead of the update
     real* vol;                    // (C, NS, 2) scratch: volume transport terms of k, omega
@@ -31,12 +31,7 @@ struct SstArgs {
     const real* det;
     const real* adj;              // (C, NS, 3, 3)
     const real* D;                // (3, NS, NS) of the cell type
-    const real* Dsp_w;            // (3, NS, WM) sparse derivative rows of the cell type: weights
-    const int* Dsp_i;             //                                                     point indices
-    const real* Esp_w;            // (5, NFP, KE) sparse face-trace rows of the cell type (slot order)
-    const int* Esp_i;
-    const real* E0;               // (5, NFP, NS) prism, slot order
-    const real* E1;               // (5, NFP, NS) tet, slot order
+    const real* E;                // (5, NFP, NS) face-trace rows of the cell type, slot order
     const int* slot_nb;
     const int* slot_blk;
     const int* slot_mask;
@@ -57,7 +52,6 @@ struct SstArgs {
     const int* schedule;          // null, or the locality order of the cells of this type
     int grid_cap = 0;     // persistent grid size (workgroups); 0: built-in default
     int grid_cap_face = 0;  // same for the face-record kernel
-    int variant = 0;        // cell kernel: 0 two prisms per wavefront, 1 one cell per wavefront
 };
 
 template <int P, int CT, typename real>

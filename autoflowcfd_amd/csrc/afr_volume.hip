@@ -19,6 +19,12 @@ using namespace afr;
 
 namespace afr_mean {
 
+// acc += w x by components: a vector product would keep w splatted over four registers
+template <typename V, typename real> __device__ __forceinline__ void fma4(V& acc, real w, V x) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[q] += w * x[q];
+}
+
 // ------------------------------------------------------------------ viscous volume kernel
 // Lanes of a wavefront: (cell, solution point), LW lanes per cell (P1: 8 cells of 8 lanes, P2: 2
 // cells of 27 of 32 lanes).  A lane keeps the non-zeros of its derivative rows in registers for the
@@ -73,19 +79,19 @@ __global__ void __launch_bounds__((64 * VV<P, CT, real>::WAVES)) k_visc_volume(M
         if constexpr (L::DENSE) {
             const real* row = a.D + ((int64_t)m * NS + sp) * NS;
 #pragma unroll 4
-            for (int q = 0; q < NS; ++q) acc += row[q] * ld4(x + q * 4);
+            for (int q = 0; q < NS; ++q) fma4(acc, row[q], ld4(x + q * 4));
         } else if (m == 0) {
 #pragma unroll
-            for (int q = 0; q < N1; ++q) acc += wa[q] * ld4(x + (q * N1 * N1 + j * N1 + k) * 4);
+            for (int q = 0; q < N1; ++q) fma4(acc, wa[q], ld4(x + (q * N1 * N1 + j * N1 + k) * 4));
         } else if (m == 1) {
 #pragma unroll
-            for (int q = 0; q < N1 * N1; ++q) acc += wb[q] * ld4(x + (q * N1 + k) * 4);
+            for (int q = 0; q < N1 * N1; ++q) fma4(acc, wb[q], ld4(x + (q * N1 + k) * 4));
         } else if constexpr (CT == 0) {
 #pragma unroll
-            for (int q = 0; q < N1; ++q) acc += wc[q] * ld4(x + ((i * N1 + j) * N1 + q) * 4);
+            for (int q = 0; q < N1; ++q) fma4(acc, wc[q], ld4(x + ((i * N1 + j) * N1 + q) * 4));
         } else {
 #pragma unroll
-            for (int q = 0; q < NS; ++q) acc += s_dc[sp * RS + q] * ld4(x + q * 4);
+            for (int q = 0; q < NS; ++q) fma4(acc, s_dc[sp * RS + q], ld4(x + q * 4));
         }
         return acc;
     };

@@ -183,13 +183,12 @@ def cpu_baseline(order, n_sample=6, budget_s=20.0, workers=None):
                       f"({res[0][1]:.3f} s each on one core)"}
 
 
-def residual_kernel_names(P, knz, ns, v_sst=0):
+def residual_kernel_names(P, knz, ns):
     """{phase: [kernel names as the profiler prints them]} of one prism-mesh residual evaluation at
-    order P with knz-wide interpolation rows, ns stored points per cell and the tile variants in
-    force (afr_mesh_set_variant: SST cell variant v pairs prisms when v = 0)."""
+    order P with knz-wide interpolation rows, ns stored points per cell."""
     return {
         "dt_local": [f"afr_step::k_dt_cells<{ns}, float>" if ns in (1, 8, 27, 64) else "afr_step::k_dt_local<float>"],
-        "sst": [f"afr_sst::k_sst_cell<{P}, 0, float, {1 - v_sst}>", f"afr_sst::k_sst_face<{P}, {knz}, float>",
+        "sst": [f"afr_sst::k_sst_cell<{P}, 0, float>", f"afr_sst::k_sst_face<{P}, {knz}, float>",
                 f"afr_sst::k_sst_update<{P}, 0, float>"],
         "visc_volume": [f"afr_mean::k_visc_volume<{P}, 0, float>"],
         "inviscid": [f"afr_mean::k_inv_volume<{P}, float>"],
@@ -571,8 +570,7 @@ def main():
     # per-phase rooflines (prism-only mesh: one launch for dt, three each for SST and the mean flow), timed with HIP
     # events on the launch stream; PMC traffic from the committed rocprofv3 summary
     P, knz = args.order, dm.rows_knz
-    from autoflowcfd_amd.autotune import get_variant
-    kn = residual_kernel_names(P, knz, dm.ns, get_variant(dm, "sst_cell"))
+    kn = residual_kernel_names(P, knz, dm.ns)
     kn["mean_flow"] = kn.pop("visc_volume") + kn.pop("inviscid") + kn.pop("visc_interface")
     phase_bytes = {"dt_local": algorithmic_bytes_dt_local(n_sp, mesh.n_cells),
                    "sst": algorithmic_bytes_sst(n_sp, mesh.n_cells, fr.n_faces),

@@ -377,10 +377,8 @@ int afr_mesh_set_grid(AfrMesh *mesh, int32_t kernel, int32_t grid_cap);
 int afr_mesh_get_grid(const AfrMesh *mesh, int32_t kernel);
 
 /* Tile shape of one kernel on this mesh (no reference counterpart; picked by the autotuner with
- * the grid size).  AFR_K_PRISM_INVISCID: 0 and 1 are accepted and are the same tile shape (its
- * volume kernel reads no neighbours).  AFR_K_SST_CELL: 0 = two prisms per wavefront (half-waves of
- * 32 lanes, P <= 2 prisms), 1 = one cell per wavefront.  Other kernels: 0 only.  Every variant
- * computes the same values bit for bit. */
+ * the grid size).  AFR_K_PRISM_INVISCID and AFR_K_SST_CELL: 0 and 1 are accepted and are the same
+ * tile shape.  Other kernels: 0 only.  Every variant computes the same values bit for bit. */
 int afr_mesh_set_variant(AfrMesh *mesh, int32_t kernel, int32_t variant);
 int afr_mesh_get_variant(const AfrMesh *mesh, int32_t kernel);
 

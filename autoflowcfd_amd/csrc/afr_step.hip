@@ -10,7 +10,10 @@
 //                  fixed summation order: deterministic)
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "../../include/afr.h"
+#include "afr_meanflow.hpp"
 #include "afr_physics.hpp"
 #include "afr_step.hpp"
 
@@ -88,80 +91,151 @@ __global__ void __launch_bounds__(kThreads) k_dt_cells(const real* __restrict__ 
 }
 
 // U_out = c0 U0 + c1 Ua + c2 dt R, then positivity (rho >= 1e-6, |u| <= 1e4,
-// p >= p_floor) per solution point and the modal filter per cell.  A workgroup
-// takes CPB = 256 / NS consecutive cells at a time: one thread per solution point
-// forms the stage value and its projection into LDS, then one thread per output
-// value applies the cell's filter row and writes it (consecutive threads,
-// consecutive addresses).  Ua may alias U_out, U0 may alias U_out (the cells of a
-// pass are read completely before any of them is written).  With a state offset
-// the three states are offsets from the cell's reference: the stage combination
-// is the same (c0 + c1 = 1), the positivity test sees the absolute state, a
-// projected component is stored back as its offset, and the filter (which keeps
-// constants) acts on the offset.
+// p >= p_floor) per solution point and the modal filter per cell.  Ua may alias U_out, U0 may
+// alias U_out (the cells of a pass are read completely before any of them is written).  With a
+// state offset the three states are offsets from the cell's reference: the stage combination is the
+// same (c0 + c1 = 1), the positivity test sees the absolute state, a projected component is stored
+// back as its offset, and the filter (which keeps constants) acts on the offset.
+//
+// A wavefront takes whole cells (lane = (cell, point): 8 cells at P1, 2 at P2, 1 at P3) and needs no
+// barrier.  Values cross HBM in consecutive order; a lane holds its filter row in registers for the
+// whole kernel (again when the wave passes from prisms to tets) and reads each point's five values
+// from LDS at once.  Bound: HBM (5 values from 3 arrays and dt in, 5 out, per point).  1024 workgroups
+// are what the device holds at once at P2; 2048 and 4096 cost 2 and 5% (weights loaded by more waves).
+// Measured, 88k P2 prisms FP32: 36.8 us, 58.6 with one thread per filtered value and the filter in LDS;
+// 12k P2 tets FP64 15.6 us (25.4), P1 tets FP64 8.4 (11.8).
+template <int NS> struct RK {
+    static constexpr int LW = NS <= 8 ? 8 : (NS <= 32 ? 32 : 64), CPW = 64 / LW, WAVES = 4, PS = 8;
+    static constexpr int NE = CPW * NS * 5, IT = (NE + 63) / 64;   // values of a pass, per lane
+    static constexpr bool REG = NS <= 27;   // filter row in registers; P3: columns in LDS
+    template <typename real> static constexpr int wpe() { return !REG ? 2 : (NS <= 8 ? (sizeof(real) == 4 ? 5 : 4) : (sizeof(real) == 4 ? 4 : 3)); }
+};
+
 template <int NS, typename real>
-__global__ void __launch_bounds__(kThreads) k_rk_stage(const real* U0, const real* Ua, const real* __restrict__ R,
-                                                       const real* __restrict__ dt, real* U_out, StateOff so,
-                                                       const real* __restrict__ filt0, const real* __restrict__ filt1,
-                                                       int64_t n_cells, int64_t n_prism, double c0, double c1,
-                                                       double c2, double p_floor) {
-    constexpr int NSV = NS * 5, CPB = kThreads / NS;
-    __shared__ real s_f[2][NS * NS];
-    __shared__ real s_x[CPB * NSV];
-    for (int i = threadIdx.x; i < NS * NS; i += kThreads) {
-        s_f[0][i] = filt0[i];
-        s_f[1][i] = filt1[i];
+__global__ void __launch_bounds__((64 * RK<NS>::WAVES))
+    __attribute__((amdgpu_waves_per_eu(RK<NS>::template wpe<real>())))
+    k_rk_stage(const real* U0, const real* Ua, const real* __restrict__ R, const real* __restrict__ dt, real* U_out,
+               StateOff so, const real* __restrict__ filt0, const real* __restrict__ filt1, int64_t n_cells,
+               int64_t n_prism, double c0, double c1, double c2, double p_floor) {
+    using L = RK<NS>;
+    using v4 = typename afr_mean::V4<real>::type;
+    constexpr int LW = L::LW, CPW = L::CPW, PS = L::PS;
+    __shared__ __attribute__((aligned(16))) real s_w[L::WAVES][CPW * NS * PS];
+    __shared__ real s_f[2][L::REG ? 1 : NS * NS];
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t0 = threadIdx.x & 63;
+    if constexpr (!L::REG) {
+        for (int q = threadIdx.x; q < NS * NS; q += 64 * L::WAVES) {
+            s_f[0][q % NS * NS + q / NS] = filt0[q];
+            s_f[1][q % NS * NS + q / NS] = filt1[q];
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    const int t = threadIdx.x;
-    for (int64_t cb = (int64_t)blockIdx.x * CPB; cb < n_cells; cb += (int64_t)gridDim.x * CPB) {
-        const int nc = (int)(n_cells - cb < CPB ? n_cells - cb : CPB);
-        if (t < nc * NS) {
-            const int64_t cell = cb + t / NS;
-            const int64_t i = cb * NS + t;
-            const double d = (double)dt[i];
-            double q[5], qa[5], off[5];
-            so.row(cell, off);
+#pragma unroll 1
+    for (int ct = 0; ct < 2; ++ct) {
+        const int64_t begin = ct == 0 ? 0 : n_prism, end = ct == 0 ? n_prism : n_cells;
+        real f[L::REG ? NS : 1];
+        if constexpr (L::REG) {
+            const real* row = (ct == 0 ? filt0 : filt1) + (t0 % LW < NS ? t0 % LW : 0) * NS;
 #pragma unroll
-            for (int v = 0; v < 5; ++v) {
-                double val = c0 * (double)U0[i * 5 + v] + c2 * d * (double)R[i * 5 + v];
-                if (c1 != 0.0) val += c1 * (double)Ua[i * 5 + v];
-                q[v] = (double)(real)val;  // stage value in the storage precision
-                qa[v] = so.mode ? q[v] + off[v] : q[v];
-            }
-            const bool low_rho = !(qa[0] > 1e-6);
-            const double rho = low_rho ? 1e-6 : qa[0];
-            double vx = qa[1] / rho, vy = qa[2] / rho, vz = qa[3] / rho;
-            const double vm = sqrt(vx * vx + vy * vy + vz * vz);
-            const bool fast = vm > 1e4;
-            double m1 = qa[1], m2 = qa[2], m3 = qa[3];
-            if (fast) {
-                const double f = 1e4 / vm;
-                vx *= f; vy *= f; vz *= f;
-                m1 = rho * vx; m2 = rho * vy; m3 = rho * vz;
-            }
-            const double ke = 0.5 * rho * (vx * vx + vy * vy + vz * vz);
-            double E = qa[4];
-            const bool low_p = 0.4 * (E - ke) < p_floor;
-            if (low_p) E = p_floor / 0.4 + ke;
-            // a component the projection left alone is stored as it was (exact); a projected one
-            // as its (absolute) value less the offset
-            real* x = s_x + t * 5;
-            x[0] = low_rho ? (real)(rho - off[0]) : (real)q[0];
-            x[1] = fast ? (real)(m1 - off[1]) : (real)q[1];
-            x[2] = fast ? (real)(m2 - off[2]) : (real)q[2];
-            x[3] = fast ? (real)(m3 - off[3]) : (real)q[3];
-            x[4] = low_p ? (real)(E - off[4]) : (real)q[4];
+            for (int j = 0; j < NS; ++j) f[j] = row[j];
         }
-        __syncthreads();
-        for (int o = t; o < nc * NSV; o += kThreads) {
-            const int cc = o / NSV, r = o % NSV, s = r / 5, v = r % 5;
-            const real* F = s_f[cb + cc < n_prism ? 0 : 1];
-            const real* x = s_x + cc * NSV;
-            real acc = 0;
-            for (int j = 0; j < NS; ++j) acc += F[s * NS + j] * x[j * 5 + v];
-            U_out[cb * NSV + o] = acc;
+        for (CellWalk cw((end - begin + CPW - 1) / CPW, L::WAVES, wid); cw.it < cw.hi; cw.it += cw.step) {
+            const int t = afr_mean::lane_fresh(t0), h = t / LW, s = t % LW < NS ? t % LW : 0;
+            real* const sx = s_w[wid];
+            real* const sc = sx + h * NS * PS;
+            const int64_t cb = begin + cw.it * CPW;
+            const int nc = (int)(end - cb < CPW ? end - cb : CPW);
+            const int64_t i0 = cb * NS;
+            real x0[L::IT], xr[L::IT], xa[L::IT], xd[L::IT];
+#pragma unroll
+            for (int q = 0; q < L::IT; ++q) {
+                const int o = t + q * 64;
+                if (o < nc * NS * 5) {
+                    x0[q] = U0[i0 * 5 + o];
+                    xr[q] = R[i0 * 5 + o];
+                    xd[q] = dt[i0 + o / 5];
+                    xa[q] = c1 != 0.0 ? Ua[i0 * 5 + o] : real(0);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < L::IT; ++q) {
+                const int o = t + q * 64;
+                if (o < nc * NS * 5) {
+                    double val = c0 * (double)x0[q] + c2 * (double)xd[q] * (double)xr[q];
+                    if (c1 != 0.0) val += c1 * (double)xa[q];
+                    sx[o / 5 * PS + o % 5] = (real)val;   // stage value in the storage precision
+                }
+            }
+            afr_mean::wave_sync();
+            const bool live = t % LW < NS && h < nc;
+            if (live) {
+                real* x = sc + s * PS;
+                double off[5], qa[5];
+                so.row(cb + h, off);
+#pragma unroll
+                for (int v = 0; v < 5; ++v) qa[v] = so.mode ? (double)x[v] + off[v] : (double)x[v];
+                const bool low_rho = !(qa[0] > 1e-6);
+                const double rho = low_rho ? 1e-6 : qa[0];
+                const double mm = qa[1] * qa[1] + qa[2] * qa[2] + qa[3] * qa[3];
+                if (low_rho || mm > 1e8 * rho * rho || 0.4 * (qa[4] - 0.5 * mm * recip(rho)) < p_floor) {
+                    double vx = qa[1] / rho, vy = qa[2] / rho, vz = qa[3] / rho;
+                    const double vm = sqrt(vx * vx + vy * vy + vz * vz);
+                    const bool fast = vm > 1e4;
+                    double m1 = qa[1], m2 = qa[2], m3 = qa[3];
+                    if (fast) {
+                        const double g = 1e4 / vm;
+                        vx *= g; vy *= g; vz *= g;
+                        m1 = rho * vx; m2 = rho * vy; m3 = rho * vz;
+                    }
+                    const double ke = 0.5 * rho * (vx * vx + vy * vy + vz * vz);
+                    // a component the projection left alone stays as it was (exact); a projected one is
+                    // stored as its (absolute) value less the offset
+                    if (low_rho) x[0] = (real)(rho - off[0]);
+                    if (fast) {
+                        x[1] = (real)(m1 - off[1]);
+                        x[2] = (real)(m2 - off[2]);
+                        x[3] = (real)(m3 - off[3]);
+                    }
+                    if (0.4 * (qa[4] - ke) < p_floor) x[4] = (real)(p_floor / 0.4 + ke - off[4]);
+                }
+            }
+            afr_mean::wave_sync();
+            v4 acc = {0, 0, 0, 0};
+            real acc4 = 0;
+            auto add = [&](int j, real w) {
+                const v4 y = afr_mean::ld4(sc + j * PS);
+                const real z = sc[j * PS + 4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[v] += w * y[v];
+                acc4 += w * z;
+            };
+            if constexpr (L::REG) {
+#pragma unroll
+                for (int j = 0; j < NS; ++j) {
+                    add(j, f[j]);
+                    if (j % 5 == 4) __builtin_amdgcn_sched_barrier(0);   // five points in flight: registers
+                }
+            } else {
+#pragma unroll 4
+                for (int j = 0; j < NS; ++j) add(j, s_f[ct][j * NS + s]);
+            }
+            // formed here: sunk into the branch below, the sums would keep all their operands alive
+            real out[5] = {acc[0], acc[1], acc[2], acc[3], acc4};
+#pragma unroll
+            for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(out[v]));
+            afr_mean::wave_sync();
+            if (live) {
+#pragma unroll
+                for (int v = 0; v < 5; ++v) sc[s * PS + v] = out[v];
+            }
+            afr_mean::wave_sync();
+#pragma unroll
+            for (int q = 0; q < L::IT; ++q) {
+                const int o = t + q * 64;
+                if (o < nc * NS * 5) U_out[i0 * 5 + o] = sx[o / 5 * PS + o % 5];
+            }
+            afr_mean::wave_sync();
         }
-        __syncthreads();
     }
 }
 
@@ -231,18 +305,18 @@ template <typename real>
 int launch_rk_stage(int ns, const real* U0, const real* Ua, const real* R, const real* dt, real* U_out,
                     StateOff so, const real* filt0, const real* filt1, int64_t n_cells, int64_t n_prism,
                     double c0, double c1, double c2, double p_floor, hipStream_t st) {
-    const int grid = grid_for(n_cells, ns > 0 ? kThreads / ns : 1);
-    if (ns == 8)
-        hipLaunchKernelGGL((k_rk_stage<8, real>), dim3(grid), dim3(kThreads), 0, st, U0, Ua, R, dt, U_out, so,
-                           filt0, filt1, n_cells, n_prism, c0, c1, c2, p_floor);
-    else if (ns == 27)
-        hipLaunchKernelGGL((k_rk_stage<27, real>), dim3(grid), dim3(kThreads), 0, st, U0, Ua, R, dt, U_out, so,
-                           filt0, filt1, n_cells, n_prism, c0, c1, c2, p_floor);
-    else if (ns == 64)
-        hipLaunchKernelGGL((k_rk_stage<64, real>), dim3(grid), dim3(kThreads), 0, st, U0, Ua, R, dt, U_out, so,
-                           filt0, filt1, n_cells, n_prism, c0, c1, c2, p_floor);
-    else
-        return -1;
+    auto go = [&](auto NS) {
+        using L = RK<decltype(NS)::value>;
+        const int64_t units = (n_prism + L::CPW - 1) / L::CPW + (n_cells - n_prism + L::CPW - 1) / L::CPW;
+        hipLaunchKernelGGL((k_rk_stage<decltype(NS)::value, real>), dim3(walk_grid(units, L::WAVES, 1024)),
+                           dim3(64 * L::WAVES), 0, st, U0, Ua, R, dt, U_out, so, filt0, filt1, n_cells, n_prism, c0, c1,
+                           c2, p_floor);
+    };
+    using std::integral_constant;
+    if (ns == 8) go(integral_constant<int, 8>());
+    else if (ns == 27) go(integral_constant<int, 27>());
+    else if (ns == 64) go(integral_constant<int, 64>());
+    else return -1;
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -591,18 +591,21 @@ int afr_residual_norm_cases(const AfrMesh* mesh, const void* R, int32_t n_vars_t
     const int64_t cv = (int64_t)ns_of(d) * 5;
     const auto& po = mesh->case_prism_off;
     const auto& to = mesh->case_tet_off;
+    std::vector<afr_step::NormCase> cases(d.n_cases);
     for (int i = 0; i < d.n_cases; ++i) {
-        // the work_part buffer is reused case after case (stream order)
-        const int64_t a0 = po[i] * cv, n0 = (po[i + 1] - po[i]) * cv;
-        const int64_t a1 = (d.n_prism + to[i]) * cv, n1 = (to[i + 1] - to[i]) * cv;
-        const double n_total = (double)((n0 + n1) / 5) * n_vars_total;
-        const int rc = d.dtype == AFR_F32
-                           ? afr_step::launch_norm2<float>((const float*)R, a0, n0, a1, n1, n_total, d.work_part,
-                                                           afr_step::kNormParts, out + i, st)
-                           : afr_step::launch_norm2<double>((const double*)R, a0, n0, a1, n1, n_total, d.work_part,
-                                                            afr_step::kNormParts, out + i, st);
-        if (rc) return fail("residual norm launch failed");
+        afr_step::NormCase& c = cases[i];
+        c.a0 = po[i] * cv;
+        c.n0 = (po[i + 1] - po[i]) * cv;
+        c.a1 = (d.n_prism + to[i]) * cv;
+        c.n1 = (to[i + 1] - to[i]) * cv;
+        c.n_total = (double)((c.n0 + c.n1) / 5) * n_vars_total;
     }
+    const int rc = d.dtype == AFR_F32
+                       ? afr_step::launch_norm_cases<float>((const float*)R, cases.data(), d.n_cases, d.work_part,
+                                                            afr_step::kNormParts, out, st)
+                       : afr_step::launch_norm_cases<double>((const double*)R, cases.data(), d.n_cases, d.work_part,
+                                                             afr_step::kNormParts, out, st);
+    if (rc) return fail("residual norm launch failed");
     return 0;
 }
 

@@ -26,10 +26,22 @@ int launch_norm(const real* x, int64_t n, double n_total, double* part, int n_pa
 template <typename real>
 int launch_fill(real* x, int64_t n, double v, hipStream_t st);
 
-// norm of the logical array x[a0, a0 + n0) ++ x[a1, a1 + n1) (bit-identical to launch_norm of the
-// same values stored contiguously)
+// One case of a batch: the logical array x[a0, a0 + n0) ++ x[a1, a1 + n1), its norm's divisor, and (set
+// by the launcher) its workgroups and its first partial sum.  A group goes by value with the launch.
+constexpr int kNormGroup = 32;
+struct NormCase {
+    int64_t a0, n0, a1, n1;
+    double n_total;
+    int parts, first;
+};
+struct NormGroup {
+    int n;
+    NormCase c[kNormGroup];
+};
+
+// norms of n cases (each bit-identical to launch_norm of the same values stored contiguously)
 template <typename real>
-int launch_norm2(const real* x, int64_t a0, int64_t n0, int64_t a1, int64_t n1, double n_total, double* part,
-                 int n_part_max, double* out, hipStream_t st);
+int launch_norm_cases(const real* x, const NormCase* cases, int n, double* part, int n_part_max, double* out,
+                      hipStream_t st);
 
 }  // namespace afr_step

@@ -431,128 +431,222 @@ __global__ void __launch_bounds__((64 * IV<P, real>::NW))
 }
 
 // ------------------------------------------------------------------ inviscid volume kernel (tets)
-// Dense operators (the collapsed tet basis does not factor).  A workgroup of 4 waves takes 12 cells;
-// lane = (cell, variable), 60 of 64, holds the 12 x 5 columns of dQ in registers, and every wave
-// applies its own rows of c2f and Op to all of them with the row entries from scalar loads (one
-// operator entry serves 60 products, no operator table in LDS).  The flux of one contravariant
-// direction at a time passes through LDS, lane = (cell, fine point), 12 x NF of them.
-// Measured, FP64: P2 70 us (546 with the jumps before, when every cell was one workgroup's pass over
-// operators in LDS), P3 329 us (1618 with jumps).
+// Dense operators (the collapsed tet basis does not factor).  A workgroup takes 12 cells; in the two
+// contractions lane = (cell, variable), 60 of 64, with the operand column in registers and the
+// operator entries from scalar loads (one entry serves 60 products; no operator in LDS).  The fluxes are formed once per fine point, lane = (cell, fine point), in FP64,
+// and all three contravariant components of a chunk of CH points pass through LDS.
+// P1: three waves, wave m takes direction m of all rows (a value read from LDS serves eight rows) and
+// the three parts meet in LDS.  P2, P3: four waves, each its own rows, chunks of 16 points.
+// Bound: the waits for scalar operands (an operator of P2 and P3 is larger than the scalar cache) at
+// two or three waves per SIMD.  Measured: P1 FP32, 98k tets 50 us (76 with a flux pass per direction and
+// split rows), P1 FP64 24.6k tets 25 (32; 31 with all 27 points at once: half the waves in flight), P2
+// FP64 60 (70), P3 FP64 285 (329).  Slower: the next row's scalars requested while one is used (their
+// waits are for both: P3 540), P2 in chunks of 8 points (63).
 template <int P, typename real> struct IT {
     static constexpr int N1 = P + 1, NS = N1 * N1 * N1, OV = (2 * P < 3 ? 2 * P : 3), NF = (OV + 1) * (OV + 1) * (OV + 1);
-    static constexpr int CPT = 12, NW = 4, NT = 64 * NW;
-    static constexpr int RW = (NS + NW - 1) / NW;               // Op rows of a wave
-    static constexpr int NI = (CPT * NF + NT - 1) / NT;         // fine points of a thread
-    static constexpr int KB = sizeof(real) == 8 ? 4 : 8;        // operator columns per scalar load
-    static constexpr int FS = (NF * 5 + 3) / 4 * 4;
-    static constexpr int QS = (NS * 5) | 1;                     // LDS stride of a cell's dQ
-    static constexpr int N_Q = CPT * QS > CPT * FS ? CPT * QS : CPT * FS;
+    static constexpr bool SPLIT = P == 1;                       // waves split directions instead of rows
+    static constexpr int CPT = 12, NW = SPLIT ? 3 : 4, NT = 64 * NW;
+    static constexpr int RW = SPLIT ? NS : (NS + NW - 1) / NW;  // Op rows of a wave
+    static constexpr int CH = SPLIT ? (sizeof(real) == 8 ? 9 : NF) : 16, NCH = NF / CH;   // fine points at a time
+    // scalars of one wait (scalar loads return out of order: a wait is for all of them): RG rows of KB
+    // columns of Op, KA columns of c2f, about 60 of the wave's 102 scalar registers
+    static constexpr int KB = SPLIT ? 9 : (sizeof(real) == 8 ? 4 : 8);
+    static constexpr int RG = NS == 64 ? 8 : (SPLIT && sizeof(real) == 8 ? 4 : RW);
+    static constexpr int KA = NS == 64 ? 32 : NS;
+    // sums per direction at P2 and P3, where the three cancel (operators of 4e5 and more)
+    static constexpr int AD = P == 1 || (P == 2 && sizeof(real) == 8) ? 1 : 3;
+    static constexpr int NP = (CPT * CH + NT - 1) / NT;         // fine points of a thread and chunk
+    static constexpr int QS = (NS * 5) | 1, FS = (NF * 5) | 1, CS = (CH * 5) | 1;
+    static constexpr int N_Q = CPT * (QS > FS ? QS : FS), N_F = 3 * CPT * CS;
+    static_assert(NF % CH == 0 && CH % KB == 0 && NS % KA == 0 && RW % RG == 0, "whole chunks");
+    static_assert(NS * 5 <= FS && (!SPLIT || 3 * CPT * NS * 5 <= N_F), "results over the work areas");
 };
 
 template <int P, typename real>
-__global__ void __launch_bounds__(256) k_inv_volume_tet(MeanArgs<real> a) {
+__global__ void __launch_bounds__((IT<P, real>::NT)) k_inv_volume_tet(MeanArgs<real> args) {
     using L = IT<P, real>;
     using uni = typename Uni<real>::type;
-    constexpr int NS = L::NS, NF = L::NF, CPT = L::CPT, NW = L::NW, NT = L::NT, RW = L::RW, NI = L::NI, FS = L::FS;
-    constexpr int QS = L::QS;
-    __shared__ real s_q[L::N_Q];         // dQ [c][s][5], then Qf [c][j][5]
-    __shared__ real s_f[CPT * FS];       // F~_m [c][j][5]
+    constexpr int NS = L::NS, NF = L::NF, CPT = L::CPT, NW = L::NW, NT = L::NT, RW = L::RW, NP = L::NP, FS = L::FS;
+    constexpr int QS = L::QS, CH = L::CH, CS = L::CS, KA = L::KA, KB = L::KB;
+    __shared__ real s_q[L::N_Q];         // dQ [c][s][5], then Qf [c][j][5], then (rows split) the result
+    __shared__ real s_f[L::N_F];         // F~ [m][c][j][5] of a chunk, then (directions split) the parts of the result
+    typedef const __attribute__((address_space(4))) MeanArgs<real> Args;
+    Args* const kernarg = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+    auto fresh = [&]() -> Args* {        // arguments read anew in every stage instead of held in registers
+        Args* p = kernarg;
+        asm volatile("" : "+s"(p));
+        return p;
+    };
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = tid & 63;
     const int lc = t / 5, lv = t % 5;
-    const uni c2f = (uni)a.c2f, op = (uni)a.op;
-    const int64_t n_tiles = (a.n_cells + CPT - 1) / CPT;
+    const int64_t n_cells = args.n_cells, n_tiles = (n_cells + CPT - 1) / CPT;
     for (CellWalk cw(n_tiles, 1, 0); cw.it < cw.hi; cw.it += cw.step) {
-        const int64_t c0 = a.cell_begin + cw.it * CPT;
-        const int nc = (int)(a.n_cells - cw.it * CPT < CPT ? a.n_cells - cw.it * CPT : CPT);
+        Args* a = fresh();
+        const int64_t c0 = a->cell_begin + cw.it * CPT;
+        const int nc = (int)(n_cells - cw.it * CPT < CPT ? n_cells - cw.it * CPT : CPT);
         const bool on = t < 5 * CPT && lc < nc;
+        // adjugates of this thread's fine points of chunk k
+        real ad[NP][9];
+        auto take_adj = [&](int k) {
+            GlobalPtr<real> src = (GlobalPtr<real>)fresh()->adjf;
+#pragma unroll
+            for (int q = 0; q < NP; ++q) {
+                const int o = tid + NT * q, c = o / CH, j = k * CH + o % CH;
+                if (o < nc * CH) {
+#pragma unroll
+                    for (int e = 0; e < 9; ++e) ad[q][e] = src[((c0 + c) * NF + j) * 9 + e];
+                }
+            }
+        };
+        take_adj(0);
         for (int o = tid; o < nc * NS; o += NT) {
             const int c = o / NS, s = o % NS;
             real* x = s_q + c * QS + s * 5;
-            if (a.dQ) {
+            if (a->dQ) {
 #pragma unroll
-                for (int v = 0; v < 5; ++v) x[v] = a.dQ[(c0 * NS + o) * 5 + v];
+                for (int v = 0; v < 5; ++v) x[v] = ((GlobalPtr<real>)a->dQ)[(c0 * NS + o) * 5 + v];
             } else {
+                StateOff so;
+                so.table = a->so.table;
+                so.cell_case = a->so.cell_case;
+#pragma unroll
+                for (int v = 0; v < 5; ++v) so.one[v] = a->so.one[v];
+                so.mode = a->so.mode;
+                so.sorted = a->so.sorted;
+                so.split = a->so.split;
                 double u[5], q[5];
-                load_state(a.U, c0 * NS + o, a.so, c0 + c, u);
+                load_state(a->U, c0 * NS + o, so, c0 + c, u);
                 cons2prim(u, q);
 #pragma unroll
-                for (int v = 0; v < 5; ++v) x[v] = (real)(q[v] - a.qref[v]);
+                for (int v = 0; v < 5; ++v) x[v] = (real)(q[v] - a->qref[v]);
             }
         }
         __syncthreads();
-        real x[NS];
-        if (on) {
+        {
+            real x[NS];
 #pragma unroll
-            for (int s = 0; s < NS; ++s) x[s] = s_q[lc * QS + s * 5 + lv];
-        }
-        __syncthreads();
-        if (on) {
+            for (int s = 0; s < NS; ++s) x[s] = s_q[(on ? lc : 0) * QS + s * 5 + lv];
+            __syncthreads();
+            const uni c2f = (uni)fresh()->c2f;
+#pragma unroll 1
             for (int j = w; j < NF; j += NW) {
                 real acc = 0;
 #pragma unroll
-                for (int s = 0; s < NS; ++s) acc += (real)c2f[j * NS + s] * x[s];
-                s_q[lc * FS + j * 5 + lv] = acc;
+                for (int k = 0; k < NS; k += KA) {
+                    real c[KA];
+#pragma unroll
+                    for (int e = 0; e < KA; ++e) c[e] = (real)c2f[j * NS + k + e];
+#pragma unroll
+                    for (int e = 0; e < KA; ++e) acc += c[e] * x[k + e];
+                    if (KA < NS) __builtin_amdgcn_sched_barrier(0);
+                }
+                if (on) s_q[lc * FS + j * 5 + lv] = acc;
             }
         }
         __syncthreads();
-        // point flux in FP64 about the reference state, one contravariant direction m at a time
-        real acc[RW];
+        constexpr int AD = L::AD;
+        real acc[AD][RW];
 #pragma unroll
-        for (int r = 0; r < RW; ++r) acc[r] = 0;
-        for (int m = 0; m < 3; ++m) {
+        for (int m = 0; m < AD; ++m)
 #pragma unroll
-            for (int q = 0; q < NI; ++q) {
-                const int o = tid + NT * q, c = o / NF, j = o % NF;
-                if (o < nc * NF) {
-                    const real* ad = a.adjf + ((c0 + c) * NF + j) * 9 + m * 3;
-                    const real A[3] = {ad[0], ad[1], ad[2]};
-                    const real* dq = s_q + c * FS + j * 5;
+            for (int r = 0; r < RW; ++r) acc[m][r] = 0;
+#pragma unroll 1
+        for (int k = 0; k < L::NCH; ++k) {
+            // point flux in FP64 about the reference state, its three contravariant components
+            a = fresh();
+#pragma unroll
+            for (int q = 0; q < NP; ++q) {
+                const int o = tid + NT * q, c = o / CH, j = o % CH;
+                if (o < nc * CH) {
+                    const real* dq = s_q + c * FS + (k * CH + j) * 5;
                     double q5[5], F[3][5];
 #pragma unroll
-                    for (int v = 0; v < 5; ++v) q5[v] = a.qref[v] + (double)dq[v];
+                    for (int v = 0; v < 5; ++v) q5[v] = a->qref[v] + (double)dq[v];
                     euler_flux(q5, F);
-                    real f[5];
+                    real f[3][5];
 #pragma unroll
-                    for (int v = 0; v < 5; ++v)
-                        f[v] = A[0] * (real)(F[0][v] - a.fref[v]) + A[1] * (real)(F[1][v] - a.fref[5 + v]) +
-                               A[2] * (real)(F[2][v] - a.fref[10 + v]);
-                    real* o5 = s_f + c * FS + j * 5;
+                    for (int i = 0; i < 3; ++i)
 #pragma unroll
-                    for (int v = 0; v < 5; ++v) o5[v] = f[v];
+                        for (int v = 0; v < 5; ++v) f[i][v] = (real)(F[i][v] - a->fref[i * 5 + v]);
+#pragma unroll
+                    for (int m = 0; m < 3; ++m)
+#pragma unroll
+                        for (int v = 0; v < 5; ++v)
+                            s_f[(m * CPT + c) * CS + j * 5 + v] =
+                                ad[q][m * 3] * f[0][v] + ad[q][m * 3 + 1] * f[1][v] + ad[q][m * 3 + 2] * f[2][v];
                 }
             }
+            if (k + 1 < L::NCH) take_adj(k + 1);
             __syncthreads();
-            if (on) {
-                const real* f = s_f + lc * FS + lv;
-                const int s0 = w * RW;
+            const uni op = (uni)fresh()->op;
+            auto row = [&](int r) { return L::SPLIT ? r : (w * RW + r < NS ? w * RW + r : NS - 1); };
+            auto columns = [&](int m, int j0, real* sum) {   // sum += op[rows][m][k CH + j0 ..] F~_m
+                real y[KB];
+                const real* f = s_f + (m * CPT + (on ? lc : 0)) * CS + j0 * 5 + lv;
+#pragma unroll
+                for (int e = 0; e < KB; ++e) y[e] = f[e * 5];
+                const uni o0 = op + m * NF + k * CH + j0;
+#pragma unroll
+                for (int r0 = 0; r0 < RW; r0 += L::RG) {
+                    real c[L::RG][KB];
+#pragma unroll
+                    for (int r = 0; r < L::RG; ++r)
+#pragma unroll
+                        for (int e = 0; e < KB; ++e) c[r][e] = (real)o0[row(r0 + r) * 3 * NF + e];
+#pragma unroll
+                    for (int r = 0; r < L::RG; ++r)
+#pragma unroll
+                        for (int e = 0; e < KB; ++e) sum[r0 + r] += c[r][e] * y[e];
+                    if (L::RG < RW) __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            if constexpr (L::SPLIT) {
 #pragma unroll 1
-                for (int j0 = 0; j0 < NF; j0 += L::KB) {
-                    real y[L::KB];
-#pragma unroll
-                    for (int e = 0; e < L::KB; ++e) y[e] = j0 + e < NF ? f[(j0 + e < NF ? j0 + e : 0) * 5] : real(0);
-#pragma unroll
-                    for (int r = 0; r < RW; ++r) {
-                        const int s = s0 + r < NS ? s0 + r : NS - 1;
-#pragma unroll
-                        for (int e = 0; e < L::KB; ++e)
-                            acc[r] += (real)op[s * 3 * NF + m * NF + (j0 + e < NF ? j0 + e : NF - 1)] * y[e];
-                    }
+                for (int j0 = 0; j0 < CH; j0 += KB) columns(w, j0, acc[0]);
+            } else {
+                auto direction = [&](int m, real* sum) {
+#pragma unroll 1
+                    for (int j0 = 0; j0 < CH; j0 += KB) columns(m, j0, sum);
+                };
+                if constexpr (AD == 1) {
+#pragma unroll 1
+                    for (int i = 0; i < 3 * (CH / KB); ++i) columns(i / (CH / KB), i % (CH / KB) * KB, acc[0]);
+                } else {
+                    direction(0, acc[0]);
+                    direction(1, acc[AD > 1 ? 1 : 0]);
+                    direction(2, acc[AD > 1 ? 2 : 0]);
                 }
             }
             __syncthreads();
         }
+        real* const out = L::SPLIT ? s_f + w * CPT * NS * 5 : s_q;
         if (on) {
-            const real g0 = (real)a.fref[lv], g1 = (real)a.fref[5 + lv], g2 = (real)a.fref[10 + lv];
 #pragma unroll
             for (int r = 0; r < RW; ++r) {
-                const int s = w * RW + r;
-                if (s < NS) {
-                    const int64_t pt = (c0 + lc) * NS + s;
-                    const real* g = a.gcl + pt * 3;
-                    a.R[pt * 5 + lv] = acc[r] + g[0] * g0 + g[1] * g1 + g[2] * g2;
-                }
+                const int s = L::SPLIT ? r : w * RW + r;
+                if (s < NS) out[(lc * NS + s) * 5 + lv] = AD == 1 ? acc[0][r] : acc[0][r] + acc[AD > 1 ? 1 : 0][r] + acc[AD > 1 ? 2 : 0][r];
             }
         }
+        __syncthreads();
+        a = fresh();
+        for (int o = tid; o < nc * NS * 5; o += NT) {
+            const int v = o % 5;
+            const int64_t pt = c0 * NS + o / 5;
+            GlobalPtr<real> g = (GlobalPtr<real>)a->gcl + pt * 3;
+            real r;
+            if constexpr (L::SPLIT) r = s_f[o] + s_f[CPT * NS * 5 + o] + s_f[2 * CPT * NS * 5 + o];
+            else r = s_q[o];
+            real fr[3];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                fr[m] = (real)a->fref[m * 5];
+#pragma unroll
+                for (int e = 1; e < 5; ++e) fr[m] = v == e ? (real)a->fref[m * 5 + e] : fr[m];
+            }
+            typedef __attribute__((address_space(1))) real GlobalReal;
+            ((GlobalReal*)a->R)[c0 * NS * 5 + o] = r + g[0] * fr[0] + g[1] * fr[1] + g[2] * fr[2];
+        }
+        __syncthreads();
     }
 }
 

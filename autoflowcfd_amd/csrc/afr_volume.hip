@@ -10,6 +10,8 @@
 //                      Y = A_a F~_a + A_b F~_b,  W = B_c F~_c,  div = f2c_c Y + f2c_ab W + gcl F(Q_ref)
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "../../include/afr.h"
 #include "afr_meanflow.hpp"
 #include "afr_physics.hpp"
@@ -430,31 +432,227 @@ __global__ void __launch_bounds__((64 * IV<P, real>::NW))
     }
 }
 
-// ------------------------------------------------------------------ inviscid volume kernel (tets)
-// Dense operators (the collapsed tet basis does not factor).  A workgroup takes 12 cells; in the two
-// contractions lane = (cell, variable), 60 of 64, with the operand column in registers and the
-// operator entries from scalar loads (one entry serves 60 products; no operator in LDS).  The fluxes are formed once per fine point, lane = (cell, fine point), in FP64,
-// and all three contravariant components of a chunk of CH points pass through LDS.
-// P1: three waves, wave m takes direction m of all rows (a value read from LDS serves eight rows) and
-// the three parts meet in LDS.  P2, P3: four waves, each its own rows, chunks of 16 points.
-// Bound: the waits for scalar operands (an operator of P2 and P3 is larger than the scalar cache) at
-// two or three waves per SIMD.  Measured: P1 FP32, 98k tets 50 us (76 with a flux pass per direction and
-// split rows), P1 FP64 24.6k tets 25 (32; 31 with all 27 points at once: half the waves in flight), P2
-// FP64 60 (70), P3 FP64 285 (329).  Slower: the next row's scalars requested while one is used (their
-// waits are for both: P3 540), P2 in chunks of 8 points (63).
-template <int P, typename real> struct IT {
+// ------------------------------------------------------------------ matrix cores, FP64 16 x 16 x 4
+// D += A B: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and D[4 i + l / 16][l % 16], i = 0 .. 3.
+typedef V4<double>::type d4;
+__device__ __forceinline__ d4 mma(double a, double b, d4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// ------------------------------------------------------------------ inviscid volume kernel (tets, FP64)
+// Dense operators (the collapsed tet basis does not factor): two matrix products per tile of 16 cells,
+// c2f x (16 cells x 5 variables) and Op x the contravariant fluxes, on the matrix cores.  Each wave keeps its operator fragments in registers for the whole kernel: a row tile of
+// c2f, and of Op a row tile (P1, P2: its share of the columns; the shares meet in LDS).  The operands
+// pass through LDS as [point][cell, variable], row stride 81: free of bank conflicts for the fragments
+// (16 columns of 4 rows) and for the point phases (16 points of a cell).  The flux is formed once per
+// fine point in FP64, lane = (cell, fine point), 16 fine points of all three directions at a time.
+// Bound: latency of the stages (barriers) at two or three workgroups per CU; the products take about a
+// quarter of the time.  Measured: P1, 24.6k tets 24.6 us, P2, 10.3k tets 42, P3, 24.6k tets 185; with
+// scalar operands and vector FMAs 25, 60 and 285 (waits for operators that the scalar cache does not hold).
+template <int P> struct IT {
+    static constexpr int N1 = P + 1, NS = N1 * N1 * N1, OV = (2 * P < 3 ? 2 * P : 3), NF = (OV + 1) * (OV + 1) * (OV + 1);
+    static constexpr int CPT = 16, NT = 256, LD = CPT * 5 + 1, CT = CPT * 5 / 16;   // columns: 5 tiles of 16
+    static constexpr int KS = (NS + 3) / 4;                     // steps of 4 over the solution points
+    static constexpr int RA = (NF + 15) / 16, WA = 4 / RA;      // row tiles of c2f, waves that share one
+    static constexpr int RC = (NS + 15) / 16, WC = 4 / RC;      // row tiles of Op, waves that share one
+    static constexpr int JS = 4 / WC;                           // steps of 4 fine points of a wave, chunk and direction
+    static constexpr int NQ = 16 * RA > 4 * KS ? 16 * RA : 4 * KS;   // rows of the first work area
+    static constexpr int N_LDS = (NQ + 48) * LD;
+    static_assert(RA * WA == 4 && RC * WC == 4 && NQ + 48 >= 64, "wave shares");
+};
+
+template <int P>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_inv_volume_tet_f64(MeanArgs<double> args) {
+    typedef double real;
+    using L = IT<P>;
+    constexpr int NS = L::NS, NF = L::NF, CPT = L::CPT, NT = L::NT, LD = L::LD, KS = L::KS, RA = L::RA, RC = L::RC;
+    constexpr int JS = L::JS, CT = L::CT;
+    // dQ [s][n], then Qf [j][n]; F~ [m][16 j][n]; then the shares of the result [part][s][n]
+    __shared__ double s_q[L::N_LDS];
+    double* const s_f = s_q + L::NQ * LD;
+    typedef const __attribute__((address_space(4))) MeanArgs<double> Args;
+    Args* const kernarg = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
+    auto fresh = [&]() -> Args* {        // arguments read anew in every stage instead of held in registers
+        Args* p = kernarg;
+        asm volatile("" : "+s"(p));
+        return p;
+    };
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = tid & 63;
+    const int ln = t % 16, lk = t / 16;
+    const int ra = w % RA, rc = w % RC, part = w / RC;
+    double fa[KS], fo[RA][3][JS];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const int j = ra * 16 + ln, s = 4 * k + lk;
+        fa[k] = j < NF && s < NS ? args.c2f[j * NS + s] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < RA; ++k)
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int q = 0; q < JS; ++q) {
+                const int s = rc * 16 + ln, j = k * 16 + (part * JS + q) * 4 + lk;
+                fo[k][m][q] = s < NS && j < NF ? args.op[(s * 3 + m) * NF + j] : 0.0;
+            }
+    const int64_t n_cells = args.n_cells, n_tiles = (n_cells + CPT - 1) / CPT;
+    for (CellWalk cw(n_tiles, 1, 0); cw.it < cw.hi; cw.it += cw.step) {
+        Args* a = fresh();
+        const int64_t c0 = a->cell_begin + cw.it * CPT;
+        const int nc = (int)(n_cells - cw.it * CPT < CPT ? n_cells - cw.it * CPT : CPT);
+        const int fc = tid / 16, fj = tid % 16;      // fine point of this thread: cell, point of the chunk
+        real ad[9];
+        auto take_adj = [&](int k) {
+            if (fc < nc && k * 16 + fj < NF) {
+                GlobalPtr<real> src = (GlobalPtr<real>)fresh()->adjf + ((c0 + fc) * NF + k * 16 + fj) * 9;
+#pragma unroll
+                for (int e = 0; e < 9; ++e) ad[e] = src[e];
+            }
+        };
+        take_adj(0);
+        if constexpr (4 * KS > NS) {     // rows past the points: zero
+            for (int o = tid; o < (4 * KS - NS) * LD; o += NT) s_q[NS * LD + o] = real(0);
+        }
+        for (int o = tid; o < nc * NS; o += NT) {
+            const int c = o / NS, s = o % NS;
+            real* x = s_q + s * LD + c * 5;
+            if (a->dQ) {
+#pragma unroll
+                for (int v = 0; v < 5; ++v) x[v] = ((GlobalPtr<real>)a->dQ)[(c0 * NS + o) * 5 + v];
+            } else {
+                StateOff so;
+                so.table = a->so.table;
+                so.cell_case = a->so.cell_case;
+#pragma unroll
+                for (int v = 0; v < 5; ++v) so.one[v] = a->so.one[v];
+                so.mode = a->so.mode;
+                so.sorted = a->so.sorted;
+                so.split = a->so.split;
+                double u[5], q[5];
+                load_state(a->U, c0 * NS + o, so, c0 + c, u);
+                cons2prim(u, q);
+#pragma unroll
+                for (int v = 0; v < 5; ++v) x[v] = (real)(q[v] - a->qref[v]);
+            }
+        }
+        __syncthreads();
+        {
+            constexpr int NC = (CT + L::WA - 1) / L::WA;
+            d4 q[NC];
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                const int ct = w / RA + i * L::WA;
+                q[i] = (d4){0, 0, 0, 0};
+                if (ct < CT) {
+#pragma unroll
+                    for (int k = 0; k < KS; ++k) q[i] = mma(fa[k], s_q[(4 * k + lk) * LD + ct * 16 + ln], q[i]);
+                }
+            }
+            __syncthreads();             // Qf takes the place of dQ
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                const int ct = w / RA + i * L::WA;
+                if (ct < CT) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s_q[(ra * 16 + 4 * e + lk) * LD + ct * 16 + ln] = (real)q[i][e];
+                }
+            }
+        }
+        __syncthreads();
+        d4 acc[CT];
+#pragma unroll
+        for (int i = 0; i < CT; ++i) acc[i] = (d4){0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < RA; ++k) {
+            // point flux in FP64 about the reference state, its three contravariant components
+            a = fresh();
+            if (fc < nc) {
+                real f[3][5];
+#pragma unroll
+                for (int i = 0; i < 15; ++i) f[i / 5][i % 5] = real(0);
+                if (k * 16 + fj < NF) {
+                    double q5[5], F[3][5];
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) q5[v] = a->qref[v] + (double)s_q[(k * 16 + fj) * LD + fc * 5 + v];
+                    euler_flux(q5, F);
+                    real d[3][5];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+#pragma unroll
+                        for (int v = 0; v < 5; ++v) d[i][v] = (real)(F[i][v] - a->fref[i * 5 + v]);
+#pragma unroll
+                    for (int m = 0; m < 3; ++m)
+#pragma unroll
+                        for (int v = 0; v < 5; ++v)
+                            f[m][v] = ad[m * 3] * d[0][v] + ad[m * 3 + 1] * d[1][v] + ad[m * 3 + 2] * d[2][v];
+                }
+#pragma unroll
+                for (int i = 0; i < 15; ++i) s_f[(i / 5 * 16 + fj) * LD + fc * 5 + i % 5] = f[i / 5][i % 5];
+            }
+            if (k + 1 < RA) take_adj(k + 1);
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+#pragma unroll
+                for (int q = 0; q < JS; ++q) {
+                    const real* x = s_f + (m * 16 + (part * JS + q) * 4 + lk) * LD + ln;
+#pragma unroll
+                    for (int i = 0; i < CT; ++i) acc[i] = mma(fo[k][m][q], x[i * 16], acc[i]);
+                }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int i = 0; i < CT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                s_q[((part * RC + rc) * 16 + 4 * e + lk) * LD + i * 16 + ln] = acc[i][e];
+        __syncthreads();
+        a = fresh();
+        for (int o = tid; o < nc * NS * 5; o += NT) {
+            const int v = o % 5, s = o / 5 % NS, c = o / (5 * NS);
+            GlobalPtr<real> g = (GlobalPtr<real>)a->gcl + (c0 * NS + o / 5) * 3;
+            double sum = s_q[s * LD + c * 5 + v];
+#pragma unroll
+            for (int q = 1; q < L::WC; ++q) sum += s_q[(q * RC * 16 + s) * LD + c * 5 + v];
+            const real r = (real)sum;
+            real fr[3];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                fr[m] = (real)a->fref[m * 5];
+#pragma unroll
+                for (int e = 1; e < 5; ++e) fr[m] = v == e ? (real)a->fref[m * 5 + e] : fr[m];
+            }
+            typedef __attribute__((address_space(1))) real GlobalReal;
+            ((GlobalReal*)a->R)[c0 * NS * 5 + o] = r + g[0] * fr[0] + g[1] * fr[1] + g[2] * fr[2];
+        }
+        __syncthreads();
+    }
+}
+
+// ------------------------------------------------------------------ inviscid volume kernel (tets, FP32)
+// Dense operators (the collapsed tet basis does not factor), vector FMAs: the FP32 matrix instruction
+// left 1.0e-6 against 64 bits on P1 tets where these sums leave 8e-7, and FP64 products on the matrix
+// cores took 67 us where this takes 50 (98k tets).  A workgroup takes 12 cells; in the two contractions
+// lane = (cell, variable), 60 of 64, with the operand column in registers and the operator entries from
+// scalar loads (one entry serves 60 products; no operator in LDS).  The fluxes are formed once per fine
+// point, lane = (cell, fine point), in FP64, and all three contravariant components of a chunk of CH
+// points pass through LDS.  P1: three waves, wave m takes direction m of all rows (a value read from LDS
+// serves eight rows) and the three parts meet in LDS.  P2: four waves, each its own rows.
+// Bound: the waits for scalar operands.  98k P1 tets 50 us (76 with a flux pass per direction and split
+// rows).
+template <int P> struct IV32 {
     static constexpr int N1 = P + 1, NS = N1 * N1 * N1, OV = (2 * P < 3 ? 2 * P : 3), NF = (OV + 1) * (OV + 1) * (OV + 1);
     static constexpr bool SPLIT = P == 1;                       // waves split directions instead of rows
     static constexpr int CPT = 12, NW = SPLIT ? 3 : 4, NT = 64 * NW;
     static constexpr int RW = SPLIT ? NS : (NS + NW - 1) / NW;  // Op rows of a wave
-    static constexpr int CH = SPLIT ? (sizeof(real) == 8 ? 9 : NF) : 16, NCH = NF / CH;   // fine points at a time
+    static constexpr int CH = SPLIT ? NF : 16, NCH = NF / CH;   // fine points at a time
     // scalars of one wait (scalar loads return out of order: a wait is for all of them): RG rows of KB
     // columns of Op, KA columns of c2f, about 60 of the wave's 102 scalar registers
-    static constexpr int KB = SPLIT ? 9 : (sizeof(real) == 8 ? 4 : 8);
-    static constexpr int RG = NS == 64 ? 8 : (SPLIT && sizeof(real) == 8 ? 4 : RW);
-    static constexpr int KA = NS == 64 ? 32 : NS;
-    // sums per direction at P2 and P3, where the three cancel (operators of 4e5 and more)
-    static constexpr int AD = P == 1 || (P == 2 && sizeof(real) == 8) ? 1 : 3;
+    static constexpr int KB = SPLIT ? 9 : 8;
+    static constexpr int RG = RW;
+    static constexpr int KA = NS;
+    // sums per direction at P2, where the three cancel (operators up to 4e5)
+    static constexpr int AD = P == 1 ? 1 : 3;
     static constexpr int NP = (CPT * CH + NT - 1) / NT;         // fine points of a thread and chunk
     static constexpr int QS = (NS * 5) | 1, FS = (NF * 5) | 1, CS = (CH * 5) | 1;
     static constexpr int N_Q = CPT * (QS > FS ? QS : FS), N_F = 3 * CPT * CS;
@@ -462,15 +660,16 @@ template <int P, typename real> struct IT {
     static_assert(NS * 5 <= FS && (!SPLIT || 3 * CPT * NS * 5 <= N_F), "results over the work areas");
 };
 
-template <int P, typename real>
-__global__ void __launch_bounds__((IT<P, real>::NT)) k_inv_volume_tet(MeanArgs<real> args) {
-    using L = IT<P, real>;
+template <int P>
+__global__ void __launch_bounds__((IV32<P>::NT)) k_inv_volume_tet_f32(MeanArgs<float> args) {
+    typedef float real;
+    using L = IV32<P>;
     using uni = typename Uni<real>::type;
     constexpr int NS = L::NS, NF = L::NF, CPT = L::CPT, NW = L::NW, NT = L::NT, RW = L::RW, NP = L::NP, FS = L::FS;
     constexpr int QS = L::QS, CH = L::CH, CS = L::CS, KA = L::KA, KB = L::KB;
     __shared__ real s_q[L::N_Q];         // dQ [c][s][5], then Qf [c][j][5], then (rows split) the result
     __shared__ real s_f[L::N_F];         // F~ [m][c][j][5] of a chunk, then (directions split) the parts of the result
-    typedef const __attribute__((address_space(4))) MeanArgs<real> Args;
+    typedef const __attribute__((address_space(4))) MeanArgs<float> Args;
     Args* const kernarg = (Args*)__builtin_amdgcn_kernarg_segment_ptr();
     auto fresh = [&]() -> Args* {        // arguments read anew in every stage instead of held in registers
         Args* p = kernarg;
@@ -659,10 +858,11 @@ int launch_inv_volume(const MeanArgs<real>& a, hipStream_t st) {
         const int grid = walk_grid(tiles, 1, a.grid_cap > 0 ? a.grid_cap : 8192);
         hipLaunchKernelGGL((k_inv_volume<P, real>), dim3(grid), dim3(64 * L::NW), 0, st, a);
     } else {
-        using L = IT<P, real>;
+        using L = std::conditional_t<sizeof(real) == 8, IT<P>, IV32<P>>;
         const int64_t tiles = (a.n_cells + L::CPT - 1) / L::CPT;
-        const int grid = walk_grid(tiles, 1, a.grid_cap > 0 ? a.grid_cap : 4096);
-        hipLaunchKernelGGL((k_inv_volume_tet<P, real>), dim3(grid), dim3(L::NT), 0, st, a);
+        const dim3 grid(walk_grid(tiles, 1, a.grid_cap > 0 ? a.grid_cap : 4096));
+        if constexpr (sizeof(real) == 8) hipLaunchKernelGGL((k_inv_volume_tet_f64<P>), grid, dim3(L::NT), 0, st, a);
+        else hipLaunchKernelGGL((k_inv_volume_tet_f32<P>), grid, dim3(L::NT), 0, st, a);
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

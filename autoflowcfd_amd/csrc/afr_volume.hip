@@ -27,6 +27,31 @@ template <typename V, typename real> __device__ __forceinline__ void fma4(V& acc
     for (int q = 0; q < 4; ++q) acc[q] += w * x[q];
 }
 
+// viscous flux of a point and its contravariant components g[m] = (momentum 3, energy); gr[n][f] = d f / dx_n
+template <typename real, typename V, typename Q>
+__device__ __forceinline__ void visc_flux(const V gr[3], const real* dq, real mt, const real* ad, real mu, real Pr, real Prt,
+                                          Q qref, V g[3]) {
+    const real mts = mu + mt;
+    const real lam = real(-2.0 / 3.0) * mts * (gr[0][0] + gr[1][1] + gr[2][2]);
+    const real cp = real(kGamma * kRair / (kGamma - 1.0));
+    const real kc = mu * cp / Pr + mt * cp / Prt;
+    real tau[3][3], e[3], vel[3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) tau[p][q] = mts * (gr[q][p] + gr[p][q]) + (p == q ? lam : real(0));
+#pragma unroll
+    for (int p = 0; p < 3; ++p) vel[p] = (real)(qref[1 + p] + (double)dq[1 + p]);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) e[p] = vel[0] * tau[0][p] + vel[1] * tau[1][p] + vel[2] * tau[2][p] - kc * gr[p][3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+#pragma unroll
+        for (int v = 0; v < 3; ++v) g[m][v] = ad[m * 3] * tau[0][v] + ad[m * 3 + 1] * tau[1][v] + ad[m * 3 + 2] * tau[2][v];
+        g[m][3] = ad[m * 3] * e[0] + ad[m * 3 + 1] * e[1] + ad[m * 3 + 2] * e[2];
+    }
+}
+
 // ------------------------------------------------------------------ viscous volume kernel
 // Lanes of a wavefront: (cell, solution point), LW lanes per cell (P1: 8 cells of 8 lanes, P2: 2
 // cells of 27 of 32 lanes).  A lane keeps the non-zeros of its derivative rows in registers for the
@@ -36,15 +61,14 @@ template <typename V, typename real> __device__ __forceinline__ void fma4(V& acc
 // gradients, stress and metrics in registers from the gradient to the flux.
 // Bound: HBM (reads U, mu_t, adj, det; writes the 16-value pack and the 4-value divergence: 4.5 GB at
 // 82^3 P2 FP32, 830 us = 5.4 TB/s).  Before: 2080 us with gradients staged through LDS, an 18-of-20-value
-// pack and a divided residual.  152k P1 prisms 57 us (285), P3 tets FP64 578 us (1168).
+// pack and a divided residual.  152k P1 prisms 57 us (285).
 template <int P, int CT, typename real> struct VV {
     static constexpr int N1 = P + 1, NS = N1 * N1 * N1;
-    static constexpr int LW = NS <= 8 ? 8 : (NS <= 32 ? 32 : 64), CPW = 64 / LW;
-    static constexpr bool DENSE = P >= 3;   // P3 tets: the round-off entries of their rows count
+    static constexpr int LW = NS <= 8 ? 8 : 32, CPW = 64 / LW;
     static constexpr int KP = kPack + 4;    // LDS stride of a pack point (bank-conflict-free 16-byte access)
     static constexpr int PER = NS * 4 + NS * KP;
-    static constexpr int WAVES = sizeof(real) == 8 && NS > 27 ? 2 : 4;
-    static constexpr int DT = CT == 1 && !DENSE ? NS * (NS | 1) : 4;   // d/dc rows of a tet
+    static constexpr int WAVES = 4;
+    static constexpr int DT = CT == 1 ? NS * (NS | 1) : 4;   // d/dc rows of a tet
 };
 
 template <int P, int CT, typename real>
@@ -59,30 +83,24 @@ __global__ void __launch_bounds__((64 * VV<P, CT, real>::WAVES)) k_visc_volume(M
     const int h = t / LW, s = t % LW;
     const bool on = s < NS;
     const int sp = on ? s : 0, i = sp / (N1 * N1), j = (sp / N1) % N1, k = sp % N1;
-    if constexpr (CT == 1 && !L::DENSE) {
+    if constexpr (CT == 1) {
         for (int q = tid; q < NS * NS; q += 64 * WAVES) s_dc[(q / NS) * RS + q % NS] = a.D[2 * NS * NS + q];
         __syncthreads();
     }
     real* const sF = s_w[wid] + h * L::PER;   // (du, dv, dw, dT) [s][4]
     real* const sP = sF + NS * 4;             // pack [s][KP], then G~ [m][s][4]
     real wa[N1], wb[N1 * N1], wc[N1];
-    if constexpr (!L::DENSE) {
 #pragma unroll
-        for (int q = 0; q < N1; ++q) {
-            wa[q] = a.D[sp * NS + (q * N1 + j) * N1 + k];
-            wc[q] = CT == 0 ? a.D[(2 * NS + sp) * NS + (i * N1 + j) * N1 + q] : real(0);
-        }
-#pragma unroll
-        for (int q = 0; q < N1 * N1; ++q) wb[q] = a.D[(NS + sp) * NS + q * N1 + k];
+    for (int q = 0; q < N1; ++q) {
+        wa[q] = a.D[sp * NS + (q * N1 + j) * N1 + k];
+        wc[q] = CT == 0 ? a.D[(2 * NS + sp) * NS + (i * N1 + j) * N1 + q] : real(0);
     }
+#pragma unroll
+    for (int q = 0; q < N1 * N1; ++q) wb[q] = a.D[(NS + sp) * NS + q * N1 + k];
     // sum_k row_m[k] x[k] over a field of 4 values per point
     auto apply = [&](int m, const real* x) -> v4 {
         v4 acc = {0, 0, 0, 0};
-        if constexpr (L::DENSE) {
-            const real* row = a.D + ((int64_t)m * NS + sp) * NS;
-#pragma unroll 4
-            for (int q = 0; q < NS; ++q) fma4(acc, row[q], ld4(x + q * 4));
-        } else if (m == 0) {
+        if (m == 0) {
 #pragma unroll
             for (int q = 0; q < N1; ++q) fma4(acc, wa[q], ld4(x + (q * N1 * N1 + j * N1 + k) * 4));
         } else if (m == 1) {
@@ -158,31 +176,10 @@ __global__ void __launch_bounds__((64 * VV<P, CT, real>::WAVES)) k_visc_volume(M
         }
         wave_sync();
         if (live) {
-            // viscous flux and its contravariant components
-            const real mu = (real)a.mu, mts = mu + mt;
-            const real lam = real(-2.0 / 3.0) * mts * (gr[0][0] + gr[1][1] + gr[2][2]);
-            const real cp = real(kGamma * kRair / (kGamma - 1.0));
-            const real kc = mu * cp / (real)a.Pr + mt * cp / (real)a.Prt;
-            real tau[3][3], e[3];
+            v4 g[3];
+            visc_flux(gr, dq, mt, ad, (real)a.mu, (real)a.Pr, (real)a.Prt, a.qref, g);
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
-#pragma unroll
-                for (int q = 0; q < 3; ++q) tau[p][q] = mts * (gr[q][p] + gr[p][q]) + (p == q ? lam : real(0));
-            real vel[3];
-#pragma unroll
-            for (int p = 0; p < 3; ++p) vel[p] = (real)(a.qref[1 + p] + (double)dq[1 + p]);
-#pragma unroll
-            for (int p = 0; p < 3; ++p)
-                e[p] = vel[0] * tau[0][p] + vel[1] * tau[1][p] + vel[2] * tau[2][p] - kc * gr[p][3];
-#pragma unroll
-            for (int m = 0; m < 3; ++m) {
-                v4 g;
-#pragma unroll
-                for (int v = 0; v < 3; ++v)
-                    g[v] = ad[m * 3] * tau[0][v] + ad[m * 3 + 1] * tau[1][v] + ad[m * 3 + 2] * tau[2][v];
-                g[3] = ad[m * 3] * e[0] + ad[m * 3 + 1] * e[1] + ad[m * 3 + 2] * e[2];
-                st4(sP + (m * NS + s) * 4, g);
-            }
+            for (int m = 0; m < 3; ++m) st4(sP + (m * NS + s) * 4, g[m]);
         }
         wave_sync();
         if (live) {
@@ -193,13 +190,149 @@ __global__ void __launch_bounds__((64 * VV<P, CT, real>::WAVES)) k_visc_volume(M
     }
 }
 
+// ------------------------------------------------------------------ matrix cores, FP64 16 x 16 x 4
+// D += A B: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and D[4 i + l / 16][l % 16], i = 0 .. 3.
+typedef V4<double>::type d4;
+__device__ __forceinline__ d4 mma(double a, double b, d4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// ------------------------------------------------------------------ viscous volume kernel (P3 tets, FP64)
+// Dense derivative rows (their round-off entries count): both contractions, D x fields and D x
+// contravariant fluxes, on the matrix cores.  A workgroup takes 8 cells x 4 fields = 2 x 16 columns; wave
+// w holds the fragments of rows 16 w .. 16 w + 15 of the three D for the whole kernel.  A quad of lanes
+// ends the first product with four rows of the four fields of one cell: transposed within the quad, each
+// lane has the gradients of one point, whose state and metrics it has held from the start.
+// Measured: 24.6k cells 179 us, 590 with a lane per point reading its dense rows from global memory.
+struct V3 {
+    static constexpr int NS = 64, CPT = 8, CT = 2, LD = CPT * 4 + 2, KS = NS / 4;
+};
+
+// x of the lane at quad position (lane ^ M)
+template <int M> __device__ __forceinline__ double quad_xor(double x) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), M == 1 ? 0xB1 : 0x4E, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), M == 1 ? 0xB1 : 0x4E, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// within each quad of lanes: entry g of lane f becomes entry f of lane g (all lanes take part)
+__device__ __forceinline__ d4 quad_transpose(d4 x, int lane) {
+    const bool b0 = lane & 1, b1 = lane & 2;
+    const double s0 = quad_xor<1>(b0 ? x[0] : x[1]), s1 = quad_xor<1>(b0 ? x[2] : x[3]);
+    const d4 y = {b0 ? s0 : x[0], b0 ? x[1] : s0, b0 ? s1 : x[2], b0 ? x[3] : s1};
+    const double t0 = quad_xor<2>(b1 ? y[0] : y[2]), t1 = quad_xor<2>(b1 ? y[1] : y[3]);
+    return (d4){b1 ? t0 : y[0], b1 ? t1 : y[1], b1 ? y[2] : t0, b1 ? y[3] : t1};
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_visc_volume_p3(MeanArgs<double> a) {
+    using L = V3;
+    constexpr int NS = L::NS, CPT = L::CPT, CT = L::CT, LD = L::LD, KS = L::KS;
+    __shared__ __attribute__((aligned(16))) double s_x[NS * LD];       // (du, dv, dw, dT) [s][cell, field]
+    __shared__ __attribute__((aligned(16))) double s_g[3 * NS * LD];   // contravariant fluxes [m][s][cell, component]
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), t = tid & 63;
+    const int ln = t % 16, lk = t / 16;
+    const int s = 16 * w + 4 * (t % 4) + lk;             // this lane's point, of the cells ct * 4 + ln / 4
+    double fd[3][KS];
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+        for (int k = 0; k < KS; ++k) fd[m][k] = a.D[(m * NS + 16 * w + ln) * NS + 4 * k + lk];
+    const double T0 = a.qref[4] / (rmax(a.qref[0], 1e-10) * kRair);
+    const int64_t n_tiles = (a.n_cells + CPT - 1) / CPT;
+    for (CellWalk cw(n_tiles, 1, 0); cw.it < cw.hi; cw.it += cw.step) {
+        const int64_t c0 = a.cell_begin + cw.it * CPT;
+        const int nc = (int)(a.n_cells - cw.it * CPT < CPT ? a.n_cells - cw.it * CPT : CPT);
+        double dq[CT][5];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int c = ct * 4 + ln / 4;
+            d4 f = {0, 0, 0, 0};
+#pragma unroll
+            for (int v = 0; v < 5; ++v) dq[ct][v] = 0.0;
+            if (c < nc) {
+                const int64_t pt = (c0 + c) * NS + s;
+                double u[5], q[5];
+                load_state(a.U, pt, a.so, c0 + c, u);
+                cons2prim(u, q);
+#pragma unroll
+                for (int v = 0; v < 5; ++v) dq[ct][v] = q[v] - a.qref[v];
+                f = (d4){dq[ct][1], dq[ct][2], dq[ct][3], q[4] / (rmax(q[0], 1e-10) * kRair) - T0};
+                if (a.dQ_out) {
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) {
+                        a.dQ_out[pt * 5 + v] = dq[ct][v];
+                        s_g[(c * NS + s) * 5 + v] = fabs(u[v]);
+                    }
+                }
+            }
+            st4(s_x + s * LD + c * 4, f);
+        }
+        __syncthreads();
+        if (a.dQ_out) {   // per-cell mean |U| (outlier reference) of callers that prepare the state
+            if (tid < nc * 5) {
+                double acc = 0;
+                for (int q = 0; q < NS; ++q) acc += s_g[(tid / 5 * NS + q) * 5 + tid % 5];
+                a.umean_out[(c0 + tid / 5) * 5 + tid % 5] = acc / NS;
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int c = ct * 4 + ln / 4;
+            const int64_t pt = (c0 + (c < nc ? c : 0)) * NS + s;
+            double ad[9];
+#pragma unroll
+            for (int q = 0; q < 9; ++q) ad[q] = a.adj[pt * 9 + q];
+            const double mt = a.mu_t ? a.mu_t[pt] : 0.0, idet = recip(a.det[pt]);
+            d4 d[3] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+                const double x = s_x[(4 * k + lk) * LD + ct * 16 + ln];
+#pragma unroll
+                for (int m = 0; m < 3; ++m) d[m] = mma(fd[m][k], x, d[m]);
+            }
+#pragma unroll
+            for (int m = 0; m < 3; ++m) d[m] = quad_transpose(d[m], t);
+            d4 gr[3], g[3];
+#pragma unroll
+            for (int n = 0; n < 3; ++n) gr[n] = (ad[n] * d[0] + ad[3 + n] * d[1] + ad[6 + n] * d[2]) * idet;
+            visc_flux(gr, dq[ct], mt, ad, a.mu, a.Pr, a.Prt, a.qref, g);
+            if (c < nc) {
+                double* vp = a.pack + pt * kPack;
+                st4(vp, (d4){dq[ct][0], dq[ct][1], dq[ct][2], dq[ct][3]});
+                st4(vp + 4, (d4){dq[ct][4], gr[0][0] + gr[0][0], gr[1][1] + gr[1][1], gr[2][2] + gr[2][2]});
+                st4(vp + 8, (d4){gr[1][0] + gr[0][1], gr[2][0] + gr[0][2], gr[2][1] + gr[1][2], gr[0][3]});
+                st4(vp + 12, (d4){gr[1][3], gr[2][3], mt, 0.0});
+            }
+#pragma unroll
+            for (int m = 0; m < 3; ++m) st4(s_g + (m * NS + s) * LD + c * 4, g[m]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int c = ct * 4 + ln / 4;
+            d4 r[3] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};   // per direction, as the sums were
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+#pragma unroll
+                for (int m = 0; m < 3; ++m) r[m] = mma(fd[m][k], s_g[(m * NS + 4 * k + lk) * LD + ct * 16 + ln], r[m]);
+            const d4 sum = quad_transpose(r[0] + r[1] + r[2], t);
+            if (c < nc) st4(a.rvisc + ((c0 + c) * NS + s) * 4, sum);
+        }
+        __syncthreads();
+    }
+}
+
 template <int P, int CT, typename real>
 int launch_visc_volume(const MeanArgs<real>& a, hipStream_t st) {
-    using L = VV<P, CT, real>;
     if (a.n_cells <= 0) return 0;
-    const int64_t units = (a.n_cells + L::CPW - 1) / L::CPW;
-    const int grid = walk_grid(units, L::WAVES, a.grid_cap > 0 ? a.grid_cap : 8192);
-    hipLaunchKernelGGL((k_visc_volume<P, CT, real>), dim3(grid), dim3(64 * L::WAVES), 0, st, a);
+    const int cap = a.grid_cap > 0 ? a.grid_cap : 8192;
+    if constexpr (P == 3) {
+        hipLaunchKernelGGL(k_visc_volume_p3, dim3(walk_grid((a.n_cells + V3::CPT - 1) / V3::CPT, 1, cap)), dim3(256), 0, st, a);
+    } else {
+        using L = VV<P, CT, real>;
+        const int grid = walk_grid((a.n_cells + L::CPW - 1) / L::CPW, L::WAVES, cap);
+        hipLaunchKernelGGL((k_visc_volume<P, CT, real>), dim3(grid), dim3(64 * L::WAVES), 0, st, a);
+    }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -430,13 +563,6 @@ __global__ void __launch_bounds__((64 * IV<P, real>::NW))
         }
         __syncthreads();
     }
-}
-
-// ------------------------------------------------------------------ matrix cores, FP64 16 x 16 x 4
-// D += A B: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and D[4 i + l / 16][l % 16], i = 0 .. 3.
-typedef V4<double>::type d4;
-__device__ __forceinline__ d4 mma(double a, double b, d4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
 // ------------------------------------------------------------------ inviscid volume kernel (tets, FP64)

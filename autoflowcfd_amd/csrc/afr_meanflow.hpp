@@ -57,6 +57,8 @@ struct MeanArgs {
     double qref[5];                // primitive reference state, its flux F(qref)[i][v]
     double fref[15];
     double mu, Pr, Prt;
+    real* work;                    // scratch for the interpolation rows as matrix fragments (FP64 tets)
+    int64_t work_len;
     int suppress;
     int accumulate;                // viscous-only interface: R += result instead of R = result
 };
@@ -85,6 +87,13 @@ __device__ __forceinline__ typename V4<real>::type ld4(const real* p) {
 template <typename real>
 __device__ __forceinline__ void st4(real* p, typename V4<real>::type v) {
     *reinterpret_cast<typename V4<real>::type*>(p) = v;
+}
+
+// ------------------------------------------------------------------ matrix cores, FP64 16 x 16 x 4
+// D += A B: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and D[4 i + l / 16][l % 16], i = 0 .. 3.
+typedef V4<double>::type d4;
+__device__ __forceinline__ d4 mma(double a, double b, d4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
 template <typename T> using GlobalPtr = const __attribute__((address_space(1))) T*;

@@ -307,6 +307,8 @@ int run_part(const AfrMesh* mesh, Part part, const void* U, const void* mu_t, co
     a.mu = mu;
     a.Pr = Pr;
     a.Prt = Prt;
+    a.work = (real*)d.work_grad;
+    a.work_len = d.work_grad ? d.n_cells * (d.order + 1) * (d.order + 1) * (d.order + 1) * 12 : 0;
     a.suppress = suppress;
     a.accumulate = accumulate;
     a.n_cells_mesh = d.n_cells;

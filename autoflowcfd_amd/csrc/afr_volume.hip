@@ -190,13 +190,6 @@ __global__ void __launch_bounds__((64 * VV<P, CT, real>::WAVES)) k_visc_volume(M
     }
 }
 
-// ------------------------------------------------------------------ matrix cores, FP64 16 x 16 x 4
-// D += A B: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and D[4 i + l / 16][l % 16], i = 0 .. 3.
-typedef V4<double>::type d4;
-__device__ __forceinline__ d4 mma(double a, double b, d4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
 // ------------------------------------------------------------------ viscous volume kernel (P3 tets, FP64)
 // Dense derivative rows (their round-off entries count): both contractions, D x fields and D x
 // contravariant fluxes, on the matrix cores.  A workgroup takes 8 cells x 4 fields = 2 x 16 columns; wave

@@ -79,7 +79,7 @@ enum { AFR_F32 = 0, AFR_F64 = 1 };
  *                                      dQ = Q - Q_ref in the storage precision and evaluate
  *                                      point fluxes / Riemann fluxes in FP64
  *   work_q     (C, ns, 5)              scratch for dQ = primitive - Q_ref
- *   work_grad  (C, ns, 12)             kept for callers that lay it out; the kernels keep gradients on chip
+ *   work_grad  (C, ns, 12)             scratch (FP64 tets: the interpolation rows as matrix fragments)
  *   work_umean (C, 5)                  scratch for the per-cell mean |U| (outlier reference)
  *   work_rvol  (C, ns, 5)              scratch for the viscous volume term: 4 values (momentum, energy) per
  *                                      point, not yet divided by det J, at stride 4
@@ -264,7 +264,7 @@ int afr_inviscid_from_primitives(const AfrMesh *mesh, const void *dQ, const void
 
 /* Viscous BR1 FR residual dU/dt (C, ns, 5); mu_t (C, ns) or NULL.
  * mu, Pr, Pr_t as in the reference (1.8e-5, 0.72, 0.9 by default).  Uses the
- * work buffers work_q, work_umean, work_rvol and work_vpack; on return work_q /
+ * work buffers work_q, work_umean, work_rvol, work_grad and work_vpack; on return work_q /
  * work_umean hold the prepared state of U. */
 int afr_viscous_residual(const AfrMesh *mesh, const void *U, const void *mu_t, void *R, double mu,
                          double Pr, double Pr_t, int32_t suppress, void *stream);

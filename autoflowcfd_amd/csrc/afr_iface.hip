@@ -765,7 +765,10 @@ template <int P, int CT, int KMAX, typename real, bool INV, bool VISC>
 int launch_iface_t(const MeanArgs<real>& a, hipStream_t st) {
     using L = IF<P, CT, real, INV, VISC>;
     const int64_t tiles = (a.n_cells + L::CPT - 1) / L::CPT;
-    const int grid = walk_grid(tiles, 1, a.grid_cap > 0 ? a.grid_cap : 4096);
+    // 2048 workgroups, twice what is resident, up to some 50 tiles each (whole mean-flow residual, us, 2048
+    // against 4096: 18k tiles P2 313 / 320, 25k P1 437 / 440, 6k P3 tets 700 / 712); 4096 for larger meshes
+    // (220k tiles P2: 4844 / 4823)
+    const int grid = walk_grid(tiles, 1, a.grid_cap > 0 ? a.grid_cap : (tiles <= 100000 ? 2048 : 4096));
     // 32-bit byte offsets while the pack of all cells (the largest array by cells) and the table of
     // distinct interpolation rows stay under 4 GiB
     const bool big = a.n_cells_mesh * L::NS * kPack * (int64_t)sizeof(real) >= ((int64_t)1 << 32) ||

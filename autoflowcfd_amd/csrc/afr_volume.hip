@@ -329,6 +329,19 @@ int launch_visc_volume(const MeanArgs<real>& a, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+// the state offset out of the kernel arguments, field by field (scalar loads where it is used)
+__device__ __forceinline__ StateOff state_off(const __attribute__((address_space(4))) StateOff& x) {
+    StateOff so;
+    so.table = x.table;
+    so.cell_case = x.cell_case;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) so.one[v] = x.one[v];
+    so.mode = x.mode;
+    so.sorted = x.sorted;
+    so.split = x.split;
+    return so;
+}
+
 // ------------------------------------------------------------------ inviscid volume kernel (prisms)
 // A workgroup of N1 wavefronts takes CPT cells at a time (P2: 3 waves, 3 cells; P1: 2 waves, 4
 // cells).  In every contraction the wave index is the output row group, so the operator entries are
@@ -421,7 +434,9 @@ __global__ void __launch_bounds__((64 * IV<P, real>::NW))
                 for (int v = 0; v < 5; ++v) x[v * 4] = ((GlobalPtr<real>)a->dQ)[(c0 * NS + o) * 5 + v];
             } else {
                 double u[5], q[5];
-                load_state(args.U, c0 * NS + o, args.so, c0 + c, u);
+                // (field by field at P1: 159 -> 153 us at 152k hexes, no scalar spills; P2: no gain, +0.3%)
+                if constexpr (P == 1) load_state(a->U, c0 * NS + o, state_off(a->so), c0 + c, u);
+                else load_state(args.U, c0 * NS + o, args.so, c0 + c, u);
                 cons2prim(u, q);
 #pragma unroll
                 for (int v = 0; v < 5; ++v) x[v * 4] = (real)(q[v] - a->qref[v]);
@@ -639,16 +654,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 #pragma unroll
                 for (int v = 0; v < 5; ++v) x[v] = ((GlobalPtr<real>)a->dQ)[(c0 * NS + o) * 5 + v];
             } else {
-                StateOff so;
-                so.table = a->so.table;
-                so.cell_case = a->so.cell_case;
-#pragma unroll
-                for (int v = 0; v < 5; ++v) so.one[v] = a->so.one[v];
-                so.mode = a->so.mode;
-                so.sorted = a->so.sorted;
-                so.split = a->so.split;
                 double u[5], q[5];
-                load_state(a->U, c0 * NS + o, so, c0 + c, u);
+                load_state(a->U, c0 * NS + o, state_off(a->so), c0 + c, u);
                 cons2prim(u, q);
 #pragma unroll
                 for (int v = 0; v < 5; ++v) x[v] = (real)(q[v] - a->qref[v]);
@@ -824,16 +831,8 @@ __global__ void __launch_bounds__((IV32<P>::NT)) k_inv_volume_tet_f32(MeanArgs<f
 #pragma unroll
                 for (int v = 0; v < 5; ++v) x[v] = ((GlobalPtr<real>)a->dQ)[(c0 * NS + o) * 5 + v];
             } else {
-                StateOff so;
-                so.table = a->so.table;
-                so.cell_case = a->so.cell_case;
-#pragma unroll
-                for (int v = 0; v < 5; ++v) so.one[v] = a->so.one[v];
-                so.mode = a->so.mode;
-                so.sorted = a->so.sorted;
-                so.split = a->so.split;
                 double u[5], q[5];
-                load_state(a->U, c0 * NS + o, so, c0 + c, u);
+                load_state(a->U, c0 * NS + o, state_off(a->so), c0 + c, u);
                 cons2prim(u, q);
 #pragma unroll
                 for (int v = 0; v < 5; ++v) x[v] = (real)(q[v] - a->qref[v]);

@@ -192,7 +192,7 @@ def residual_kernel_names(P, knz, ns):
                 f"afr_sst::k_sst_update<{P}, 0, float>"],
         "visc_volume": [f"afr_mean::k_visc_volume<{P}, 0, float>"],
         "inviscid": [f"afr_mean::k_inv_volume<{P}, float>"],
-        "visc_interface": [f"afr_mean::k_iface<{P}, 0, {knz}, float, true, true, false>"],
+        "visc_interface": [f"afr_mean::k_iface<{P}, 0, {knz}, float, true, true, false, false>"],
     }
 
 

@@ -12,14 +12,14 @@
 // interpolation rows.  The jumps meet in LDS, from where one thread per solution point distributes
 // them; the outlier test runs on the residual in LDS, one lane per (cell, variable).
 //
-// Bound: latency of the gathers (VALU issue takes about half of the time, HBM traffic 7.8 GB at 82^3 P2
+// Bound: latency of the gathers (VALU issue takes about half of the time, HBM traffic 8.4 GB at 82^3 P2
 // FP32).  What this form is there for: one set of traces, slot tables and one residual write serve both
 // jumps, four resident waves per SIMD at no spill, the next tile's tables and own points in flight while
 // this one computes.  Tried and slower: five waves per workgroup with one slot per wave (2 or 3 resident
 // workgroups, uneven SIMDs: 5.0 ms), a lane's gather of all 15 values on its own instead of four lanes
 // sharing 16-byte loads (4.1 ms), a budget of five waves per SIMD (spills).
 // Measured (82^3 hex, 1.1 M prisms, P2 FP32): 2.75 ms; two kernels before, 2.88 ms for the viscous jumps
-// and about half of 2.98 ms for the inviscid ones.  152k P1 prisms FP32 263 us (401 + half of 1014).
+// and about half of 2.98 ms for the inviscid ones.  304k P1 prisms FP32 263 us (401 + half of 1014).
 // P2 and P3 tets FP64: see the matrix products below.
 #include <hip/hip_runtime.h>
 
@@ -766,7 +766,7 @@ int launch_iface_t(const MeanArgs<real>& a, hipStream_t st) {
     using L = IF<P, CT, real, INV, VISC>;
     const int64_t tiles = (a.n_cells + L::CPT - 1) / L::CPT;
     // 2048 workgroups, twice what is resident, up to some 50 tiles each (whole mean-flow residual, us, 2048
-    // against 4096: 18k tiles P2 313 / 320, 25k P1 437 / 440, 6k P3 tets 700 / 712); 4096 for larger meshes
+    // against 4096: 13k tiles P2 313 / 320, 25k P1 437 / 440, 6k P3 tets 700 / 712); 4096 for larger meshes
     // (220k tiles P2: 4844 / 4823)
     const int grid = walk_grid(tiles, 1, a.grid_cap > 0 ? a.grid_cap : (tiles <= 100000 ? 2048 : 4096));
     // 32-bit byte offsets while the pack of all cells (the largest array by cells) and the table of

@@ -54,7 +54,7 @@ __device__ __forceinline__ void prim_at(const real* U, int64_t c, const double* 
 
 // Lane = (cell, incidence): a cell's up to eight records are fetched and their fluxes formed at the
 // same time, then summed over the eight lanes.  Bound: the latency of the dependent loads and of one
-// AUSM+up flux in FP64.  Measured on 23.5k cells, FP32 storage: 27 us, 50 us with one thread
+// AUSM+up flux in FP64.  Measured on 94k cells, FP32 storage: 27 us, 50 us with one thread
 // walking the records of a cell.
 template <typename real>
 __global__ void __launch_bounds__(kThreads) k_p0_residual(AfrP0Desc d, const real* __restrict__ U,

@@ -74,7 +74,7 @@ template <int P, int CT> struct SO {
 //
 // Bound: FP64 source arithmetic and HBM together (4.3 GB at 82^3 P2 FP32).  Measured there 1165 us,
 // before (rows as index / weight tables in LDS, one 4-byte read and one subtraction per product, every
-// slot's trace) 1938; 152k P1 prisms FP32 95 us (252, 24 of 64 lanes busy).
+// slot's trace) 1938; 304k P1 prisms FP32 95 us (252, 24 of 64 lanes busy).
 template <int P, int CT> struct SC {
     using O = SO<P, CT>;
     static constexpr int NS = O::NS, NI = O::NSLOT * O::NFP, RD = (NI + O::LW - 1) / O::LW;
@@ -425,7 +425,7 @@ __global__ void __launch_bounds__(256) k_sst_face(SstArgs<real> a) {
 // ballot, on values rounded to FP32: its margin of 1e-4 of the threshold covers the rounding, and
 // values that FP32 could not tell from zero or infinity go the exact way.
 // Bound: HBM and the gather of record corrections.  Measured (82^3 P2 FP32): 621 us, 1298 with one cell
-// per wavefront and the FP64 certificate through LDS; 152k P1 prisms 51 us (308).
+// per wavefront and the FP64 certificate through LDS; 304k P1 prisms 51 us (308).
 template <int LW> __device__ __forceinline__ float cell_max(float x) {
     x = fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, false)));    // xor 1
     x = fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xf, 0xf, false)));    // xor 2

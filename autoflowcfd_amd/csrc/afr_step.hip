@@ -102,8 +102,8 @@ __global__ void __launch_bounds__(kThreads) k_dt_cells(const real* __restrict__ 
 // whole kernel (again when the wave passes from prisms to tets) and reads each point's five values
 // from LDS at once.  Bound: HBM (5 values from 3 arrays and dt in, 5 out, per point).  1024 workgroups
 // are what the device holds at once at P2; 2048 and 4096 cost 2 and 5% (weights loaded by more waves).
-// Measured, 88k P2 prisms FP32: 36.8 us, 58.6 with one thread per filtered value and the filter in LDS;
-// 12k P2 tets FP64 15.6 us (25.4), P1 tets FP64 8.4 (11.8).
+// Measured, 66.5k P2 prisms FP32: 36.8 us, 58.6 with one thread per filtered value and the filter in LDS;
+// 10.3k P2 tets FP64 15.6 us (25.4), P1 tets FP64 8.4 (11.8).
 template <int NS> struct RK {
     static constexpr int LW = NS <= 8 ? 8 : (NS <= 32 ? 32 : 64), CPW = 64 / LW, WAVES = 4, PS = 8;
     static constexpr int NE = CPW * NS * 5, IT = (NE + 63) / 64;   // values of a pass, per lane

@@ -61,7 +61,7 @@ __device__ __forceinline__ void visc_flux(const V gr[3], const real* dq, real mt
 // gradients, stress and metrics in registers from the gradient to the flux.
 // Bound: HBM (reads U, mu_t, adj, det; writes the 16-value pack and the 4-value divergence: 4.5 GB at
 // 82^3 P2 FP32, 830 us = 5.4 TB/s).  Before: 2080 us with gradients staged through LDS, an 18-of-20-value
-// pack and a divided residual.  152k P1 prisms 57 us (285).
+// pack and a divided residual.  304k P1 prisms 57 us (285).
 template <int P, int CT, typename real> struct VV {
     static constexpr int N1 = P + 1, NS = N1 * N1 * N1;
     static constexpr int LW = NS <= 8 ? 8 : 32, CPW = 64 / LW;
@@ -352,7 +352,7 @@ __device__ __forceinline__ StateOff state_off(const __attribute__((address_space
 // Bound: waits (59% of the wave cycles: barriers between the stages, scalar loads of the operators);
 // VALU issue takes 0.86 ms of it, HBM 3.5 GB.  Measured (82^3 P2 FP32): 1.21 ms; with the arguments held
 // in registers over the tile loop 1.48 ms.  Before, jumps included: 2.98 ms (one wave per cell, LDS
-// operator tables).  152k P1 prisms 143 us (1014 with jumps).
+// operator tables).  304k P1 prisms 143 us (1014 with jumps).
 template <int P, typename real> struct IV {
     using K = afr_prism::PK<P>;
     static constexpr int N1 = K::N1, NAB = K::NAB, NF1 = K::NF1, NABF = K::NABF, NF = K::NF, NS = K::NS;
@@ -434,7 +434,7 @@ __global__ void __launch_bounds__((64 * IV<P, real>::NW))
                 for (int v = 0; v < 5; ++v) x[v * 4] = ((GlobalPtr<real>)a->dQ)[(c0 * NS + o) * 5 + v];
             } else {
                 double u[5], q[5];
-                // (field by field at P1: 159 -> 153 us at 152k hexes, no scalar spills; P2: no gain, +0.3%)
+                // (field by field at P1: 159 -> 153 us at 304k prisms, no scalar spills; P2: no gain, +0.3%)
                 if constexpr (P == 1) load_state(a->U, c0 * NS + o, state_off(a->so), c0 + c, u);
                 else load_state(args.U, c0 * NS + o, args.so, c0 + c, u);
                 cons2prim(u, q);
@@ -758,13 +758,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 // ------------------------------------------------------------------ inviscid volume kernel (tets, FP32)
 // Dense operators (the collapsed tet basis does not factor), vector FMAs: the FP32 matrix instruction
 // left 1.0e-6 against 64 bits on P1 tets where these sums leave 8e-7, and FP64 products on the matrix
-// cores took 67 us where this takes 50 (98k tets).  A workgroup takes 12 cells; in the two contractions
+// cores took 67 us where this takes 50 (70k tets).  A workgroup takes 12 cells; in the two contractions
 // lane = (cell, variable), 60 of 64, with the operand column in registers and the operator entries from
 // scalar loads (one entry serves 60 products; no operator in LDS).  The fluxes are formed once per fine
 // point, lane = (cell, fine point), in FP64, and all three contravariant components of a chunk of CH
 // points pass through LDS.  P1: three waves, wave m takes direction m of all rows (a value read from LDS
 // serves eight rows) and the three parts meet in LDS.  P2: four waves, each its own rows.
-// Bound: the waits for scalar operands.  98k P1 tets 50 us (76 with a flux pass per direction and split
+// Bound: the waits for scalar operands.  70k P1 tets 50 us (76 with a flux pass per direction and split
 // rows).
 template <int P> struct IV32 {
     static constexpr int N1 = P + 1, NS = N1 * N1 * N1, OV = (2 * P < 3 ? 2 * P : 3), NF = (OV + 1) * (OV + 1) * (OV + 1);

@@ -52,9 +52,15 @@ __device__ __forceinline__ void prim_at(const real* U, int64_t c, const double* 
     cons2prim(u, q);
 }
 
+template <int CTRL> __device__ __forceinline__ double lane_swap(double x) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xf, 0xf, true));
+}
+
 // Lane = (cell, incidence): a cell's up to eight records are fetched and their fluxes formed at the
 // same time, then summed over the eight lanes.  Bound: the latency of the dependent loads and of one
-// AUSM+up flux in FP64.  Measured on 94k cells, FP32 storage: 27 us, 50 us with one thread
+// AUSM+up flux in FP64.  Measured on 94k cells, FP32 storage: 24 us (25 with the sums by
+// shuffles through LDS, 27.5 with the cells dealt to the XCDs in turn), 50 us with one thread
 // walking the records of a cell.
 template <typename real>
 __global__ void __launch_bounds__(kThreads) k_p0_residual(AfrP0Desc d, const real* __restrict__ U,
@@ -64,7 +70,10 @@ __global__ void __launch_bounds__(kThreads) k_p0_residual(AfrP0Desc d, const rea
     const real* adj = (const real*)d.adj;
     const int k = threadIdx.x & 7;
     const int64_t n8 = (d.n_cells + 7) / 8 * 8;   // whole wavefronts: the sums below need every lane
-    for (int64_t cc = ((int64_t)blockIdx.x * kThreads + threadIdx.x) >> 3; cc < n8; cc += (int64_t)gridDim.x * (kThreads / 8)) {
+    // workgroups are dealt to the eight XCDs in turn: each XCD gets one contiguous range of the cells, whose
+    // neighbours its L2 then holds
+    const int nb8 = gridDim.x & ~7u, blk = (int)blockIdx.x < nb8 ? (blockIdx.x & 7) * (nb8 >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    for (int64_t cc = ((int64_t)blk * kThreads + threadIdx.x) >> 3; cc < n8; cc += (int64_t)gridDim.x * (kThreads / 8)) {
         const int64_t c = cc < d.n_cells ? cc : d.n_cells - 1;
         // the records of a cell come first in its list: nothing follows the first hole
         const int e0 = d.cell_inc[c * 8 + k];
@@ -122,8 +131,9 @@ __global__ void __launch_bounds__(kThreads) k_p0_residual(AfrP0Desc d, const rea
 #pragma unroll
         for (int v = 0; v < 5; ++v) {
             double x = res[v];
-#pragma unroll
-            for (int m = 1; m < 8; m <<= 1) x += __shfl_xor(x, m);
+            x += lane_swap<0xB1>(x);     // lane ^ 1
+            x += lane_swap<0x4E>(x);     // lane ^ 2
+            x += lane_swap<0x141>(x);    // the other quad of eight lanes
             out = k == v ? x : out;
         }
         if (k < 5 && cc < d.n_cells) R[c * 5 + k] = (real)out;

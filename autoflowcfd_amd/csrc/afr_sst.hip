@@ -303,7 +303,7 @@ __global__ void __launch_bounds__(64 * kWaves)
         for (int r = 0; r < L::RD; ++r) {
             const int o = tl + r * LW, slot = L::slot(o), fp = o % NFP;
             if (o < L::NI && h < nc && (own >> (slot < 3 ? slot : slot + 1) & 1)) {
-                v4 ta = a0, tb = b0;
+                v4 ta = {0, 0, 0, 0}, tb = ta;   // the perturbation alone: one rounding at the size of x_0
                 if constexpr (CT == 0) {
                     const int b = s_eb[o], st = slot < 2 ? N1 * N1 : (slot == 2 ? N1 : 1);
 #pragma unroll
@@ -322,8 +322,8 @@ __global__ void __launch_bounds__(64 * kWaves)
                     }
                 }
                 real* ov = a.pack + ((cell * 5 + slot) * NFP + fp) * kPack;
-                st4(ov, ta);
-                st4(ov + 4, tb);
+                st4(ov, a0 + ta);
+                st4(ov + 4, b0 + tb);
             }
             __builtin_amdgcn_sched_barrier(0);
         }

@@ -232,7 +232,7 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
     __shared__ real s_a[L::N_A];
     __shared__ real s_j[L::N_J];
     __shared__ real s_rw[ROWS_CAP * KMAX];
-    __shared__ uint8_t s_ri[ROWS_CAP * KMAX];
+    __shared__ uint8_t s_ri[ROWS_CAP * KMAX];   // bit 7 of a row's first: it has more than N1 non-zeros
     __shared__ real s_ew[DENSE ? 1 : NSLOT * NFP * KW];   // own-trace weights
     __shared__ real s_med[2][CPT * NR];
     __shared__ int s_list[CPT * NR], s_bad;    // columns (cell, value) that need their median, how many
@@ -251,11 +251,17 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
     // prism box; a batch of cases or a tet mesh has more and reads them from global memory)
     const int n_rows = args.n_rows;
     const bool rows_lds = ROWS_CAP > 1 && n_rows + 1 <= ROWS_CAP;
-    if (rows_lds)
-        for (int q = tid; q < (n_rows + 1) * KMAX; q += NT) {
-            s_rw[q] = args.rows_w[q];
-            s_ri[q] = (uint8_t)args.rows_idx[q];
+    if (rows_lds) {
+#pragma unroll
+        for (int u = 0; u < (ROWS_CAP * KMAX + NT - 1) / NT; ++u) {
+            const int q = tid + u * NT, r = q / KMAX;
+            if (q < (n_rows + 1) * KMAX) {
+                const int i = args.rows_idx[q], nnz = args.rows_nnz[r < n_rows ? r : 0];
+                s_rw[q] = args.rows_w[q];
+                s_ri[q] = (uint8_t)(i | (q == r * KMAX && r < n_rows && nnz > N1 ? 128 : 0));
+            }
         }
+    }
     if (tid == 0) s_bad = 0;
     // Lane role, packed: slot, cell of the tile, flux point, in use.  The prism blocks are ordered with
     // the b face last, so that the waves with its wider own rows are not those with the (usually) wider
@@ -301,7 +307,7 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
     }
 
     // Where a lane takes its other side from: the boundary code, the source cell and the interpolation
-    // row (-1: none; wide: more than N1 non-zeros).
+    // row (-1: none).
     struct Slot {
         int mask, bc, blk0, blk1, nb0, nb1;
     };
@@ -318,14 +324,12 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
         return x;
     };
     int bc = 0, nb = 0, row = -1;
-    bool wide = false;
     auto take_slot = [&](const Slot& x, int fp) {
         const bool second = (x.mask >> fp) & 1;
         bc = x.bc;
         nb = second ? x.nb1 : x.nb0;
         row = (second ? x.blk1 : x.blk0) * NFP + fp;
         if (bc != BC_INTERIOR || nb < 0 || row < 0 || row >= n_rows) row = -1;
-        wide = second || ((x.mask >> 30) & 1);
     };
     // cell of list position p (the last cell for lanes and tiles past the end)
     auto cell_at = [&](int64_t p) -> int {
@@ -476,7 +480,8 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
 #pragma unroll
                 for (int q = 0; q < 5; ++q) pn[q] = real(0);
             }
-            auto terms = [&](int k0) {
+            bool wide = false;    // more than N1 non-zeros (known with the first terms; rows of prism sources)
+            auto terms = [&](int k0, auto first) {
                 Idx pt[N1];
                 real w[N1];
 #pragma unroll
@@ -484,6 +489,10 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
                     const int kk = KMAX % N1 == 0 || k0 + k < KMAX ? k0 + k : KMAX - 1;
                     int i;
                     row_entry(kk, i, w[k]);
+                    if (decltype(first)::value && k == 0 && KMAX == N1 * N1) {
+                        wide = rows_lds ? i & 128 : have && at<BIG>(a->rows_nnz, (Idx)r) > N1;
+                        if (rows_lds) i &= 127;
+                    }
                     pt[k] = p0 + i;
                     if (kk != k0 + k) w[k] = real(0);
                 }
@@ -496,19 +505,19 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
                         for (int q = 0; q < 5; ++q) pn[q] += w[k] * at<BIG>(a->dQ, pt[k] * 5 + q);
                 }
             };
-            terms(0);
+            terms(0, std::true_type());
             // further terms: the quads with a wide row (prism sources), or every lane up to the widest
             // row of the wave (dense rows of tet sources)
             if constexpr (KMAX == N1 * N1) {
                 if ((__ballot(have && wide) >> (tid & 60)) & 15) {
 #pragma unroll 1
-                    for (int k0 = N1; k0 < KMAX; k0 += N1) terms(k0);
+                    for (int k0 = N1; k0 < KMAX; k0 += N1) terms(k0, std::false_type());
                 }
             } else {
                 const int nnz = have ? at<BIG>(a->rows_nnz, (Idx)r) : 0;
                 const int kn = __any(nnz > N1 * N1) ? KMAX : (__any(nnz > N1) ? N1 * N1 : N1);
 #pragma unroll 1
-                for (int k0 = N1; k0 < kn; k0 += N1) terms(k0);
+                for (int k0 = N1; k0 < kn; k0 += N1) terms(k0, std::false_type());
             }
             if constexpr (VISC) quad_transpose<real>(acc, pn, qi);
         }

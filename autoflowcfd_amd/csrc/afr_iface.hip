@@ -471,8 +471,8 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
                     i = s_ri[r * KMAX + kk];
                     w = s_rw[r * KMAX + kk];
                 } else {
-                    i = at<BIG>(a->rows_idx, (Idx)(r * KMAX + kk));
-                    w = at<BIG>(a->rows_w, (Idx)(r * KMAX + kk));
+                    i = at<BIG>(a->rows_idx, (Idx)r * KMAX + kk);
+                    w = at<BIG>(a->rows_w, (Idx)r * KMAX + kk);
                 }
             };
             v4 acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};

@@ -1,5 +1,8 @@
-"""GPU: the mean-flow residual takes the width of an interpolation row from the row tables; the hint bit of
-the slot masks (bit 30) changes nothing."""
+"""GPU: the interpolation row tables of the mean-flow residual.
+
+* The width of a row is that of the tables; the hint bit of the slot masks (bit 30) changes nothing.
+* Tables of more than 2^31 entries, with the rows in use at their end: the 64-bit form of the interface
+  kernel, the same bits as the 32-bit form on the rows alone."""
 
 import pytest
 
@@ -46,3 +49,31 @@ def test_wide_row_hint_changes_nothing(name, order, prec):
         dm.slot_mask.copy_(bits)
         for a, b in zip(_residuals(dm, U, mut), ref):
             assert torch.equal(a, b)
+
+
+def _with_tables(dm, n_rows, nnz, idx, w):
+    dm.lib.afr_mesh_destroy(dm.handle)
+    dm.rows_nnz, dm.rows_idx, dm.rows_w = nnz, idx, w
+    dm._create(n_rows, dm.mesh.n_prism)
+
+
+@pytest.mark.parametrize("name,order,prec", [("wallbox", 1, "f32"), ("wallbox", 2, "f32"), ("wallbox", 1, "f64"),
+                                             ("wallbox", 2, "f64"), ("rotated", 2, "f32"), ("mixed", 1, "f32"),
+                                             ("mixed", 2, "f32"), ("mixed", 2, "f64")])
+def test_row_tables_past_two_to_the_31_entries(name, order, prec):
+    import torch
+    print(f"[gpu] row table of 2^31 entries {name} P{order} {prec}", flush=True)
+    dm, U, mut = _device(MESHES[name](), order, torch.float32 if prec == "f32" else torch.float64)
+    ref = _residuals(dm, U, mut)
+    k, n = dm.rows_knz, dm.n_rows
+    skip = ((1 << 31) // k // dm.nfp + 1) * dm.nfp           # whole blocks of unused rows before the others
+    assert skip * k >= 1 << 31 and n % dm.nfp == 0
+
+    def shifted(x):
+        y = torch.zeros((skip + n + 1,) + tuple(x.shape[1:]), dtype=x.dtype, device="cuda")
+        y[skip:] = x
+        return y
+    dm.slot_blk[dm.slot_blk >= 0] += skip // dm.nfp
+    _with_tables(dm, skip + n, shifted(dm.rows_nnz), shifted(dm.rows_idx), shifted(dm.rows_w))
+    for a, b in zip(_residuals(dm, U, mut), ref):
+        assert torch.equal(a, b)

@@ -250,15 +250,18 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
     // the deduplicated interpolation rows in LDS when the mesh has few blocks (8 for a graded
     // prism box; a batch of cases or a tet mesh has more and reads them from global memory)
     const int n_rows = args.n_rows;
-    const bool rows_lds = ROWS_CAP > 1 && n_rows + 1 <= ROWS_CAP;
+    const bool rows_lds = ROWS_CAP > 1 && n_rows < ROWS_CAP;
     if (rows_lds) {
 #pragma unroll
         for (int u = 0; u < (ROWS_CAP * KMAX + NT - 1) / NT; ++u) {
             const int q = tid + u * NT, r = q / KMAX;
-            if (q < (n_rows + 1) * KMAX) {
-                const int i = args.rows_idx[q], nnz = args.rows_nnz[r < n_rows ? r : 0];
+            if (r < n_rows) {
+                const int i = args.rows_idx[q], nnz = args.rows_nnz[r];
                 s_rw[q] = args.rows_w[q];
-                s_ri[q] = (uint8_t)(i | (q == r * KMAX && r < n_rows && nnz > N1 ? 128 : 0));
+                s_ri[q] = (uint8_t)(i | (q == r * KMAX && nnz > N1 ? 128 : 0));
+            } else if (r == n_rows) {   // after them one of zeros
+                s_rw[q] = real(0);
+                s_ri[q] = 0;
             }
         }
     }
@@ -462,8 +465,9 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
 #pragma unroll
             for (int q = 0; q < 3; ++q) A[q] = at<BIG>(a->slot_adjrow, ai + q);
             if constexpr (INV) fb = (at<BIG>(a->slot_fb, sidx) >> fp) & 1;
-            // 1. the other side's trace (the rows hold their non-zeros first; the last row is all zero)
-            const int r = have ? row : n_rows;
+            // 1. the other side's trace (the rows hold their non-zeros first); lanes without a source join the
+            //    loads of their quad with weights of zero: the last row in LDS, or the first of the table masked
+            const int r = have ? row : (rows_lds ? n_rows : 0);
             const Idx p0 = times<BIG>(have ? nb : 0, NS);
             const int qi = tid & 3;
             auto row_entry = [&](int kk, int& i, real& w) {
@@ -472,7 +476,7 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
                     w = s_rw[r * KMAX + kk];
                 } else {
                     i = at<BIG>(a->rows_idx, (Idx)r * KMAX + kk);
-                    w = at<BIG>(a->rows_w, (Idx)r * KMAX + kk);
+                    w = have ? at<BIG>(a->rows_w, (Idx)r * KMAX + kk) : real(0);
                 }
             };
             v4 acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
@@ -505,7 +509,10 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
                         for (int q = 0; q < 5; ++q) pn[q] += w[k] * at<BIG>(a->dQ, pt[k] * 5 + q);
                 }
             };
-            terms(0, std::true_type());
+            // waves without any source skip the rows (a table without rows is not read).  As a branch it also
+            // keeps the loads before it out of the gather: kernel on 1.1 M P2 prisms FP32 2755 -> 2430 us, 304k
+            // P1 prisms 262 -> 264
+            if (__any(have)) terms(0, std::true_type());
             // further terms: the quads with a wide row (prism sources), or every lane up to the widest
             // row of the wave (dense rows of tet sources)
             if constexpr (KMAX == N1 * N1) {

@@ -2,7 +2,8 @@
 
 * The width of a row is that of the tables; the hint bit of the slot masks (bit 30) changes nothing.
 * Tables of more than 2^31 entries, with the rows in use at their end: the 64-bit form of the interface
-  kernel, the same bits as the 32-bit form on the rows alone."""
+  kernel, the same bits as the 32-bit form on the rows alone.
+* Nothing past the n_rows rows is used: the memory after them holds indexes and weights of no use."""
 
 import pytest
 
@@ -75,5 +76,31 @@ def test_row_tables_past_two_to_the_31_entries(name, order, prec):
         return y
     dm.slot_blk[dm.slot_blk >= 0] += skip // dm.nfp
     _with_tables(dm, skip + n, shifted(dm.rows_nnz), shifted(dm.rows_idx), shifted(dm.rows_w))
+    for a, b in zip(_residuals(dm, U, mut), ref):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("name", sorted(MESHES) + ["one"])
+@pytest.mark.parametrize("order", [1, 2])
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+def test_no_row_is_used_past_the_last(name, order, prec):
+    import numpy as np
+    import torch
+    from autoflowcfd_amd.mesh import BC_FARFIELD, mesh_from_cells
+    print(f"[gpu] end of the row table {name} P{order} {prec}", flush=True)
+    src = wall_box(seed=2)
+    mesh = (mesh_from_cells(src.nodes, src.prism_conn[:1], default_bc=BC_FARFIELD) if name == "one"
+            else MESHES[name]())
+    dm, U, mut = _device(mesh, order, torch.float32 if prec == "f32" else torch.float64)
+    ref = _residuals(dm, U, mut)
+    n = 0 if name == "one" else dm.n_rows                    # a lone cell needs no row
+    assert n > 0 or bool((dm.slot_bc >= 0).all())
+
+    def ended(x, fill):
+        y = torch.full((n + 64,) + tuple(x.shape[1:]), fill, dtype=x.dtype, device="cuda")
+        y[:n] = x[:n]
+        return y
+    _with_tables(dm, n, ended(dm.rows_nnz, dm.rows_knz), ended(dm.rows_idx, (1 << 30) - 1),
+                 ended(dm.rows_w, float(np.nan)))
     for a, b in zip(_residuals(dm, U, mut), ref):
         assert torch.equal(a, b)

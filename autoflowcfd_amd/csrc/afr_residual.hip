@@ -409,6 +409,8 @@ int afr_inviscid_residual(const AfrMesh* mesh, const void* U, void* R, int32_t s
 
 namespace {
 
+int ns_of(const AfrMeshDesc& d) { return (d.order + 1) * (d.order + 1) * (d.order + 1); }
+
 bool viscous_ready(const AfrMeshDesc& d) {
     return d.adj && d.work_grad && d.work_rvol && d.work_h && d.work_vpack && d.dsp_w[0] && d.dsp_w[1] && d.dsp_i[0] &&
            d.dsp_i[1] && d.esp_w[0] && d.esp_w[1] && d.esp_i[0] && d.esp_i[1] && d.D[0] && d.D[1] && d.E[0] && d.E[1];
@@ -452,10 +454,15 @@ int afr_residual(const AfrMesh* mesh, const void* U, const void* mu_t, void* R, 
     const AfrMeshDesc& d = mesh->d;
     if (!viscous_ready(d)) return fail("afr_residual: mesh has no viscous work buffers");
     hipStream_t st = (hipStream_t)stream;
-    // viscous pack and volume term, inviscid volume term (into R), then both interface terms at once
-    if (mean_part(mesh, VISC_VOLUME, U, mu_t, nullptr, nullptr, nullptr, mu, Pr, Pr_t, 0, 0, st)) return -1;
-    if (mean_part(mesh, INV_VOLUME, U, nullptr, nullptr, nullptr, R, mu, Pr, Pr_t, 0, 0, st)) return -1;
-    return mean_part(mesh, IFACE_FULL, U, mu_t, nullptr, nullptr, R, mu, Pr, Pr_t, suppress, 0, st);
+    // viscous pack and volume term, inviscid volume term (into R), then both interface terms at once.  Where R
+    // lies over U, the state is gone from the second part on: the first prepares dQ and mean |U| for them
+    const size_t bytes = (size_t)d.n_cells * ns_of(d) * 5 * (d.dtype == AFR_F32 ? sizeof(float) : sizeof(double));
+    const char *u = (const char*)U, *r = (const char*)R;
+    const bool over = u < r + bytes && r < u + bytes;
+    const void *dQ = over ? d.work_q : nullptr, *umean = over ? d.work_umean : nullptr;
+    if (mean_part(mesh, VISC_VOLUME, U, mu_t, dQ, umean, nullptr, mu, Pr, Pr_t, 0, 0, st)) return -1;
+    if (mean_part(mesh, INV_VOLUME, U, nullptr, dQ, nullptr, R, mu, Pr, Pr_t, 0, 0, st)) return -1;
+    return mean_part(mesh, IFACE_FULL, U, mu_t, nullptr, umean, R, mu, Pr, Pr_t, suppress, 0, st);
 }
 
 namespace {
@@ -464,8 +471,6 @@ bool step_ready(const AfrMeshDesc& d) {
     return d.metric_flux_scale && d.volume && d.work_r && d.work_s1 && d.work_s2 && d.work_dt && d.work_part &&
            d.filt[0] && d.filt[1];
 }
-
-int ns_of(const AfrMeshDesc& d) { return (d.order + 1) * (d.order + 1) * (d.order + 1); }
 
 }  // namespace
 

@@ -280,7 +280,7 @@ int afr_viscous_interface(const AfrMesh *mesh, const void *U, const void *mu_t, 
 
 /* Full Navier-Stokes FR residual dU/dt = inviscid + viscous (each with its own
  * outlier zeroing when suppress != 0), as the reference solver sums them
- * (src/autoflowcfd/core/fr_solver/solver.py:360-420).  mu_t may be NULL. */
+ * (src/autoflowcfd/core/fr_solver/solver.py:360-420).  mu_t may be NULL.  R may lie over U. */
 int afr_residual(const AfrMesh *mesh, const void *U, const void *mu_t, void *R, double mu, double Pr,
                  double Pr_t, int32_t suppress, void *stream);
 

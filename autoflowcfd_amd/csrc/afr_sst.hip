@@ -502,8 +502,8 @@ __global__ void __launch_bounds__(64 * kWaves) k_sst_update(SstArgs<real> a) {
             const float mk = cell_max<LW>(xk), mw = cell_max<LW>(xw);
             const int nk = __popcll(__ballot(live && xk < mk * 1.0001e-4f) & group);
             const int nw = __popcll(__ballot(live && xw < mw * 1.0001e-4f) & group);
-            const bool tiny = live && ((tk != 0.0 && mk < 1e-30f) || (tw != 0.0 && mw < 1e-30f));
-            if (__any(nk > k1 || nw > k1 || tiny)) {
+            const bool out = mk > 3e38f || mw > 3e38f || (tk != 0.0 && mk < 1e-30f) || (tw != 0.0 && mw < 1e-30f);
+            if (__any(nk > k1 || nw > k1 || (live && out))) {
                 double* const sx = s_x[wid] + h * NS * 2;
                 double* const sm = s_med[wid] + h * 4;
                 if (live) {

@@ -362,6 +362,16 @@ int mean_part(const AfrMesh* mesh, Part part, const void* U, const void* mu_t, c
                : run_part<double>(mesh, part, U, mu_t, dQ, umean, R, mu, Pr, Prt, suppress, accumulate, st);
 }
 
+// the operators that the kernels read are there for every cell type present: E (all), c2f and op (inviscid
+// volume term of tets), D (viscous and SST terms)
+bool operators_ready(const AfrMeshDesc& d, bool inviscid, bool derivatives) {
+    for (int ct = 0; ct < 2; ++ct) {
+        if ((ct == 0 ? d.n_prism : d.n_cells - d.n_prism) <= 0) continue;
+        if (!d.E[ct] || (derivatives && !d.D[ct]) || (inviscid && ct == 1 && (!d.c2f[1] || !d.op[1]))) return false;
+    }
+    return true;
+}
+
 }  // namespace
 
 extern "C" {
@@ -393,6 +403,7 @@ int afr_prepare_state(const AfrMesh* mesh, const void* U, void* dQ, void* umean,
 int afr_inviscid_from_primitives(const AfrMesh* mesh, const void* dQ, const void* umean, void* R,
                                  int32_t suppress, void* stream) {
     if (!mesh || !dQ || !umean || !R) return fail("afr_inviscid_from_primitives: null argument");
+    if (!operators_ready(mesh->d, true, false)) return fail("afr_inviscid_from_primitives: mesh has no operator tables");
     hipStream_t st = (hipStream_t)stream;
     if (mean_part(mesh, INV_VOLUME, nullptr, nullptr, dQ, umean, R, 0, 1, 1, 0, 0, st)) return -1;
     return mean_part(mesh, IFACE_INV, nullptr, nullptr, dQ, umean, R, 0, 1, 1, suppress, 0, st);
@@ -401,6 +412,7 @@ int afr_inviscid_from_primitives(const AfrMesh* mesh, const void* dQ, const void
 int afr_inviscid_residual(const AfrMesh* mesh, const void* U, void* R, int32_t suppress, void* stream) {
     if (!mesh || !U || !R) return fail("afr_inviscid_residual: null argument");
     const AfrMeshDesc& d = mesh->d;
+    if (!operators_ready(d, true, false)) return fail("afr_inviscid_residual: mesh has no operator tables");
     if (afr_prepare_state(mesh, U, d.work_q, d.work_umean, stream)) return -1;
     return afr_inviscid_from_primitives(mesh, d.work_q, d.work_umean, R, suppress, stream);
 }
@@ -413,7 +425,7 @@ int ns_of(const AfrMeshDesc& d) { return (d.order + 1) * (d.order + 1) * (d.orde
 
 bool viscous_ready(const AfrMeshDesc& d) {
     return d.adj && d.work_grad && d.work_rvol && d.work_h && d.work_vpack && d.dsp_w[0] && d.dsp_w[1] && d.dsp_i[0] &&
-           d.dsp_i[1] && d.esp_w[0] && d.esp_w[1] && d.esp_i[0] && d.esp_i[1] && d.D[0] && d.D[1] && d.E[0] && d.E[1];
+           d.dsp_i[1] && d.esp_w[0] && d.esp_w[1] && d.esp_i[0] && d.esp_i[1] && operators_ready(d, false, true);
 }
 
 }  // namespace
@@ -453,6 +465,7 @@ int afr_residual(const AfrMesh* mesh, const void* U, const void* mu_t, void* R, 
     if (!mesh || !U || !R) return fail("afr_residual: null argument");
     const AfrMeshDesc& d = mesh->d;
     if (!viscous_ready(d)) return fail("afr_residual: mesh has no viscous work buffers");
+    if (!operators_ready(d, true, true)) return fail("afr_residual: mesh has no operator tables");
     hipStream_t st = (hipStream_t)stream;
     // viscous pack and volume term, inviscid volume term (into R), then both interface terms at once.  Where R
     // lies over U, the state is gone from the second part on: the first prepares dQ and mean |U| for them
@@ -762,6 +775,7 @@ int afr_sst_step(const AfrMesh* mesh, const void* U, void* k, void* omega, const
     if (d.n_records <= 0 || !d.rec_owner || !d.rec_oslot || !d.rec_flags || !d.rec_tn || !d.cell_inc ||
         !d.work_pack || !d.work_nbp || !d.work_tvol || !d.work_tsrc || !d.work_crec || !d.adj)
         return fail("afr_sst_step: mesh has no SST record tables / work buffers");
+    if (!operators_ready(d, false, true)) return fail("afr_sst_step: mesh has no operator tables");
     hipStream_t st = (hipStream_t)stream;
     return d.dtype == AFR_F32
                ? run_sst<float>(d, mesh->so, U, k, omega, d_wall, dt, nu_t, mu_t, rates, mu_molecular, st)

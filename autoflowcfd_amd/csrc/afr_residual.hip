@@ -611,21 +611,25 @@ int afr_residual_norm_cases(const AfrMesh* mesh, const void* R, int32_t n_vars_t
     const int64_t cv = (int64_t)ns_of(d) * 5;
     const auto& po = mesh->case_prism_off;
     const auto& to = mesh->case_tet_off;
-    std::vector<afr_step::NormCase> cases(d.n_cases);
-    for (int i = 0; i < d.n_cases; ++i) {
-        afr_step::NormCase& c = cases[i];
-        c.a0 = po[i] * cv;
-        c.n0 = (po[i + 1] - po[i]) * cv;
-        c.a1 = (d.n_prism + to[i]) * cv;
-        c.n1 = (to[i + 1] - to[i]) * cv;
-        c.n_total = (double)((c.n0 + c.n1) / 5) * n_vars_total;
+    for (int first = 0; first < d.n_cases; first += afr_step::kNormGroup) {
+        afr_step::NormCase cases[afr_step::kNormGroup];   // no heap: nothing here may throw through the C entry
+        const int n = d.n_cases - first < afr_step::kNormGroup ? d.n_cases - first : afr_step::kNormGroup;
+        for (int i = 0; i < n; ++i) {
+            const int k = first + i;
+            afr_step::NormCase& c = cases[i];
+            c.a0 = po[k] * cv;
+            c.n0 = (po[k + 1] - po[k]) * cv;
+            c.a1 = (d.n_prism + to[k]) * cv;
+            c.n1 = (to[k + 1] - to[k]) * cv;
+            c.n_total = (double)((c.n0 + c.n1) / 5) * n_vars_total;
+        }
+        const int rc = d.dtype == AFR_F32
+                           ? afr_step::launch_norm_cases<float>((const float*)R, cases, n, d.work_part,
+                                                                afr_step::kNormParts, out + first, st)
+                           : afr_step::launch_norm_cases<double>((const double*)R, cases, n, d.work_part,
+                                                                 afr_step::kNormParts, out + first, st);
+        if (rc) return fail("residual norm launch failed");
     }
-    const int rc = d.dtype == AFR_F32
-                       ? afr_step::launch_norm_cases<float>((const float*)R, cases.data(), d.n_cases, d.work_part,
-                                                            afr_step::kNormParts, out, st)
-                       : afr_step::launch_norm_cases<double>((const double*)R, cases.data(), d.n_cases, d.work_part,
-                                                             afr_step::kNormParts, out, st);
-    if (rc) return fail("residual norm launch failed");
     return 0;
 }
 

@@ -1,13 +1,15 @@
 """Autotuner of the launch shapes of the residual kernels on one mesh.
 
 Every residual kernel walks its cells with a persistent grid; how many workgroups that grid
-has trades latency hiding against tail effects and L2 sharing (``VARIANTS``: tile-shape codes that a
-kernel takes; both codes of either kernel are one shape).  The best choice depends on the kernel, the order, the precision and the
-mesh size.  ``autotune`` times each kernel's phase with HIP events on the launch stream for every
-(tile variant, grid size) candidate (results do not depend on either: only the time does) and
-leaves the fastest set on the mesh (``afr_mesh_set_variant``, ``afr_mesh_set_grid``).  Choices
-are cached per (device, order, dtype, kernel, size bucket) in memory and, when ``cache_path`` is
-given, in a JSON file.
+has trades latency hiding against tail effects and L2 sharing.  The best choice depends on the
+kernel, the order, the precision, the cell types and the mesh size.  ``autotune`` times with HIP
+events on the launch stream, for every grid size, the smallest call that runs a kernel as the
+residual does (results do not depend on it: only the time does) and leaves the fastest on the mesh
+(``afr_mesh_set_grid``).  Choices are cached per (device, order, dtype, kernel, cell types, size
+bucket, kernel revision) in memory and, when ``cache_path`` is given, in a JSON file.
+
+``VARIANTS``: tile-shape codes that a kernel takes (``afr_mesh_set_variant``).  Both codes of either
+kernel are one shape, so each grid size is timed once, reported for both, and code 0 is set.
 """
 
 import json
@@ -33,7 +35,11 @@ def candidates_for(device=None):
         .multi_processor_count
     return (0,) + tuple(int(n_cu) * k for k in CU_MULTIPLES)
 
-VARIANTS = {"prism_inviscid": (0, 1), "sst_cell": (0, 1)}   # tile shapes (afr_mesh_set_variant)
+VARIANTS = {"prism_inviscid": (0, 1), "sst_cell": (0, 1)}   # tile-shape codes (afr_mesh_set_variant)
+
+# part of the cache key: to be raised when the kernels change, so that choices timed on former ones
+# are not taken for the present ones
+KERNEL_REVISION = 2
 
 _memo = {}
 
@@ -41,7 +47,8 @@ _memo = {}
 def _key(dm, name):
     bucket = int(round(math.log2(max(dm.n_cells, 1))))
     dev = torch.cuda.get_device_name(dm.device)
-    return f"{dev}|P{dm.order}|{str(dm.dtype).split('.')[-1]}|{name}|2^{bucket}"
+    cells = "tet" if dm.n_prism == 0 else ("prism" if dm.n_prism == dm.n_cells else "mixed")
+    return f"{dev}|P{dm.order}|{str(dm.dtype).split('.')[-1]}|{name}|{cells}|2^{bucket}|r{KERNEL_REVISION}"
 
 
 def set_grid(dm, name, cap):
@@ -98,13 +105,14 @@ def autotune(dm, U, mu_t=None, mu=1.8e-5, sst_fields=None, reps=3, candidates=No
         with open(cache_path) as f:
             cache = json.load(f)
     R = torch.empty_like(U)
-    mean = lambda: dm.residual(U, mu_t, R, mu=mu)  # noqa: E731  the mean-flow kernels as one call; one varies
+    dm.viscous_volume(U, mu_t, mu=mu)            # dQ / field means for the inviscid phase
     phases = {}
     if dm.mesh.n_prism:
-        phases["prism_inviscid"] = mean
+        phases["prism_inviscid"] = lambda: dm.inviscid_from_primitives(dm.work_q, dm.work_umean, R)
     if dm.mesh.n_tet:
-        phases["tet_inviscid"] = mean
-    phases["visc_volume"] = phases["visc_iface"] = mean
+        phases["tet_inviscid"] = lambda: dm.inviscid_from_primitives(dm.work_q, dm.work_umean, R)
+    phases["visc_volume"] = lambda: dm.viscous_volume(U, mu_t, mu=mu)
+    phases["visc_iface"] = lambda: dm.residual(U, mu_t, R, mu=mu)   # both jumps in one kernel: the whole call
     if sst_fields is not None and dm.turbulence == "SST":
         k, w, nut, mut = sst_fields
         rates = torch.empty((dm.n_cells, dm.ns, 2), dtype=dm.dtype, device=dm.device)
@@ -121,17 +129,14 @@ def autotune(dm, U, mu_t=None, mu=1.8e-5, sst_fields=None, reps=3, candidates=No
             out[name] = dict(choice, ms=None, cached=True)
             continue
         times = {}
-        for var in VARIANTS.get(name, (0,)):
-            set_variant(dm, name, var)
-            for cap in candidates:
-                set_grid(dm, name, cap)
-                times[(var, cap)] = _time(fn, reps)
-        var, cap = min(times, key=times.get)
-        choice = _apply(dm, name, {"grid": cap, "variant": var})
+        set_variant(dm, name, 0)
+        for cap in candidates:
+            set_grid(dm, name, cap)
+            times[cap] = _time(fn, reps)
+        choice = _apply(dm, name, {"grid": min(times, key=times.get), "variant": 0})
         _memo[key] = choice
         cache[key] = choice
-        out[name] = dict(choice, ms={f"v{v}/g{g}": t for (v, g), t in times.items()})
-    dm.viscous_volume(U, mu_t, mu=mu)
+        out[name] = dict(choice, ms={f"v{v}/g{g}": t for v in VARIANTS.get(name, (0,)) for g, t in times.items()})
     torch.cuda.synchronize(dm.device)
     if cache_path:
         os.makedirs(os.path.dirname(os.path.abspath(cache_path)), exist_ok=True)

@@ -458,6 +458,24 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
 #pragma unroll
             for (int q = 0; q < 3; ++q) A[q] = at<BIG>(a->slot_adjrow, ai + q);
             if constexpr (INV) fb = (at<BIG>(a->slot_fb, sidx) >> fp) & 1;
+            // a product also takes the points that a row does not name, with weights of zero: where the trace
+            // is not finite, it is summed over its row's own points
+            real size = 0;
+#pragma unroll
+            for (int q = 0; q < NP; ++q) size += fabs(pn[q]);
+            if (have && !(size < __builtin_huge_val())) {
+#pragma unroll
+                for (int q = 0; q < NP; ++q) pn[q] = real(0);
+                const int nnz = at<BIG>(a->rows_nnz, (Idx)row);
+#pragma unroll 1
+                for (int k = 0; k < nnz; ++k) {
+                    const Idx e = (Idx)row * KMAX + k;
+                    const real w = at<BIG>(a->rows_w, e);
+                    const int64_t p = ((int64_t)nb * NS + at<BIG>(a->rows_idx, e)) * kPack;
+#pragma unroll
+                    for (int q = 0; q < NP; ++q) pn[q] += w * ((GlobalPtr<real>)a->pack)[p + q];
+                }
+            }
         } else {
             Args* a = fresh();
             const Idx sidx = times<BIG>(cell, 5) + slot;

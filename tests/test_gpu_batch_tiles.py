@@ -1,0 +1,70 @@
+"""GPU: a case's residuals and SST step do not depend on the batch it rides in, bit for bit: small tet and
+mixed cases whose cells fall at other places of the kernels' tiles and waves (12, 16, 7 and 4 cells; waves of
+8 or 2) than alone, at every order and precision, and whose row tables a batch adds up."""
+
+import numpy as np
+import pytest
+
+from cases import freestream, mixed_mesh, smooth_state, tet_box
+
+pytestmark = pytest.mark.gpu
+
+SIZES = (1, 2, 7, 8, 13, 3, 40)
+
+
+def _mesh(n):
+    from autoflowcfd_amd.mesh import BC_FARFIELD, BC_WALL, mesh_from_cells
+    if n == "mixed":
+        m = mixed_mesh()
+    else:
+        src = tet_box(2, seed=1)
+        m = mesh_from_cells(src.nodes, None, src.tet_conn[:n], default_bc=BC_FARFIELD)
+    fr = m.faces
+    low = np.flatnonzero(fr.is_boundary)[:2]
+    fr.bc[low] = BC_WALL
+    m.wall_nodes = np.unique(fr.node_ids[low])
+    m.wall_nodes = m.wall_nodes[m.wall_nodes >= 0]
+    return m
+
+
+@pytest.mark.parametrize("sizes,order,prec", [(s, o, p) for s in (SIZES, ("mixed", 13, "mixed", 2)) for o in (1, 2)
+                                              for p in ("f32", "f64")] + [(SIZES, 3, "f64")])
+def test_case_does_not_depend_on_its_batch(sizes, order, prec):
+    import torch
+    from autoflowcfd_amd.device import DeviceMesh, bc_params_table
+    from autoflowcfd_amd.geometry import map_ref
+    print(f"[gpu] batch tiles {sizes} P{order} {prec}", flush=True)
+    dt = torch.float32 if prec == "f32" else torch.float64
+    turb = "SST" if order < 3 else None
+    Q0 = freestream(0.15, 4.0)
+    bcp = bc_params_table(Q0)
+    rng = np.random.default_rng(4)
+    parts, data = [], []
+    for n in sizes:
+        mesh = _mesh(n)
+        dm = DeviceMesh(mesh, order, dtype=dt, bc_params=bcp, turbulence=turb)
+        xyz = np.zeros((mesh.n_cells, dm.ns, 3))
+        if mesh.n_prism:
+            xyz[:mesh.n_prism] = map_ref(True, dm.T.sps, mesh.nodes[mesh.prism_conn])
+        xyz[mesh.n_prism:] = map_ref(False, dm.T.sps, mesh.nodes[mesh.tet_conn])
+        shape = xyz.shape[:2]
+        x = (smooth_state(xyz, Q0, seed=3), 1.8e-5 * rng.uniform(0.0, 50.0, shape),
+             0.39 * (1 + 0.2 * rng.uniform(-1, 1, shape)), 2660.0 * (1 + 0.2 * rng.uniform(-1, 1, shape)))
+        parts.append(dm)
+        data.append([torch.as_tensor(v, dtype=dt, device="cuda").contiguous() for v in x])
+    batch = DeviceMesh.concat(parts, np.stack([bcp] * len(parts)), parts[0].ref_state)
+
+    def joined(xs):
+        return torch.cat([x[:q.n_prism] for x, q in zip(xs, parts)] + [x[q.n_prism:] for x, q in zip(xs, parts)]).contiguous()
+
+    def evaluate(dm, U, mut, k, w):
+        res = {"full": dm.residual(U, mut), "inviscid": dm.inviscid_residual(U), "viscous": dm.viscous_residual(U, mut)}
+        if turb:
+            k, w, nut, mt = k.clone(), w.clone(), torch.zeros_like(k), torch.zeros_like(k)
+            dm.sst_step(U, k, w, torch.full_like(k, 1e-6), nut, mt)
+            res.update(k=k, omega=w, nu_t=nut)
+        return res
+    alone = [evaluate(q, *x) for q, x in zip(parts, data)]
+    together = evaluate(batch, *(joined([x[i] for x in data]) for i in range(4)))
+    for what, got in together.items():
+        assert torch.equal(got, joined([a[what] for a in alone])), what

@@ -11,13 +11,11 @@ pytestmark = pytest.mark.gpu
 MESHES = {"prism": lambda: wall_box(seed=1), "tet": lambda: tet_box(2, seed=1), "mixed": mixed_mesh}
 
 
-@pytest.mark.parametrize("name", sorted(MESHES))
-@pytest.mark.parametrize("order,prec", [(1, "f32"), (1, "f64"), (2, "f32"), (2, "f64"), (3, "f64")])
+@pytest.mark.parametrize("name,order,prec", [(n, o, p) for n in sorted(MESHES) for o in (1, 2) for p in ("f32", "f64")]
+                         + [("tet", 3, "f64")])
 def test_residual_over_its_state(name, order, prec):
     import torch
     from autoflowcfd_amd.device import DeviceMesh, bc_params_table
-    if order == 3 and name != "tet":
-        pytest.skip("P3 meshes are tets")
     print(f"[gpu] residual in place {name} P{order} {prec}", flush=True)
     dt = torch.float32 if prec == "f32" else torch.float64
     mesh = MESHES[name]()

@@ -5,7 +5,6 @@
 //   euler_flux      src/autoflowcfd/core/fr_operators/flux_kernels.py:29-68
 //   ausm_up         src/autoflowcfd/core/fr_operators/kernels.py:20-155
 //   ghost_state     src/autoflowcfd/boundary/fr_ghost_state.py:26-189
-//   viscous_flux    src/autoflowcfd/core/fr_operators/flux_kernels.py:72-137
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -300,57 +299,6 @@ __host__ __device__ __forceinline__ void ghost_state(int bc, const real qi[5], c
     }
 }
 
-// viscous flux G[i][v]; gv[i][j] = du_i/dx_j
-template <typename real>
-__host__ __device__ __forceinline__ void viscous_flux(const real q[5], const real gv[3][3], const real gT[3], real mu, real Pr,
-                                             real mut, real Prt, real G[3][5]) {
-    real mt = mu + mut;
-    real div = gv[0][0] + gv[1][1] + gv[2][2];
-    real lam = real(-2.0 / 3.0) * mt;
-    real tau[3][3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            tau[i][j] = real(2) * mt * (real(0.5) * (gv[i][j] + gv[j][i])) + (i == j ? lam * div : real(0));
-    const real cp = real(kGamma * kRair / (kGamma - 1.0));
-    real k = mu * cp / Pr + mut * cp / Prt;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        G[i][0] = real(0);
-        G[i][1] = tau[i][0];
-        G[i][2] = tau[i][1];
-        G[i][3] = tau[i][2];
-        real work = q[1] * tau[0][i] + q[2] * tau[1][i] + q[3] * tau[2][i];
-        G[i][4] = work - k * gT[i];
-    }
-}
-
-// A . G for the viscous flux G of viscous_flux, contracted with a direction A (3): the five
-// components A_i G[i][v], computed from tau . A (tau is symmetric) without forming G.
-template <typename real>
-__host__ __device__ __forceinline__ void viscous_flux_dot(const real q[5], const real gv[3][3], const real gT[3],
-                                                         real mu, real Pr, real mut, real Prt, const real A[3],
-                                                         real out[5]) {
-    const real mt = mu + mut;
-    const real lam = real(-2.0 / 3.0) * mt * (gv[0][0] + gv[1][1] + gv[2][2]);
-    real tA[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        real acc = lam * A[j];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) acc += A[i] * (mt * (gv[i][j] + gv[j][i]));
-        tA[j] = acc;
-    }
-    const real cp = real(kGamma * kRair / (kGamma - 1.0));
-    const real k = mu * cp / Pr + mut * cp / Prt;
-    out[0] = real(0);
-    out[1] = tA[0];
-    out[2] = tA[1];
-    out[3] = tA[2];
-    out[4] = q[1] * tA[0] + q[2] * tA[1] + q[3] * tA[2] - k * (A[0] * gT[0] + A[1] * gT[1] + A[2] * gT[2]);
-}
-
 // Per-wave walk over the cells of a persistent grid.  Workgroups are dispatched round-robin
 // over the 8 XCDs (blockIdx % 8); each XCD walks one contiguous range of the cell list so
 // that, with a locality-ordered list (schedule), the neighbour data of consecutive cells is
@@ -367,11 +315,6 @@ struct CellWalk {
         hi = n * (xcd + 1) >> sh;
     }
 };
-
-// cell of list position it: schedule[it] (a permutation of [0, n)) or it itself
-__device__ __forceinline__ int64_t walk_cell(const int* schedule, int64_t it) {
-    return schedule ? (int64_t)__builtin_amdgcn_readfirstlane(schedule[it]) : it;
-}
 
 // persistent grid of at most cap workgroups for n cells at wpb waves per workgroup, a
 // multiple of 8 when at least 8

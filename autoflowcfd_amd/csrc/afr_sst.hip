@@ -66,9 +66,9 @@ template <int P, int CT> struct SO {
 // functions FP32 on the FP32 path).
 //
 // A lane keeps the non-zeros of its derivative rows in registers for the whole kernel (d/da: an a
-// line, d/db: an (a, b) plane, d/dc: a c line of a prism, every point of a tet from LDS), and those
-// of XX are dealt out with the N1^2-wide b face last, so that
-// only the last round is wide).  Fields lie in LDS as 16-byte vectors of perturbations, so a non-zero
+// line, d/db: an (a, b) plane, d/dc: a c line of a prism, every point of a tet from LDS).  The trace rows
+// lie in LDS; a prism's flux points are dealt out to the lanes with the N1^2-wide b face last, so that only
+// the last round is wide.  Fields lie in LDS as 16-byte vectors of perturbations, so a non-zero
 // costs one or two LDS reads and no subtraction.  Traces are written for slots that own a face
 // record only: no other is read.
 //

@@ -772,17 +772,15 @@ template <int P> struct IV32 {
     static constexpr int CPT = 12, NW = SPLIT ? 3 : 4, NT = 64 * NW;
     static constexpr int RW = SPLIT ? NS : (NS + NW - 1) / NW;  // Op rows of a wave
     static constexpr int CH = SPLIT ? NF : 16, NCH = NF / CH;   // fine points at a time
-    // scalars of one wait (scalar loads return out of order: a wait is for all of them): RG rows of KB
-    // columns of Op, KA columns of c2f, about 60 of the wave's 102 scalar registers
+    // columns of Op whose scalars share one wait (scalar loads return out of order: a wait is for all of
+    // them), about 60 of the wave's 102 scalar registers
     static constexpr int KB = SPLIT ? 9 : 8;
-    static constexpr int RG = RW;
-    static constexpr int KA = NS;
-    // sums per direction at P2, where the three cancel (operators up to 4e5)
-    static constexpr int AD = P == 1 ? 1 : 3;
+    // sums per direction at P2, where the three cancel (operators up to 4e5); P1: a wave has one direction
+    static constexpr int AD = SPLIT ? 1 : 3;
     static constexpr int NP = (CPT * CH + NT - 1) / NT;         // fine points of a thread and chunk
     static constexpr int QS = (NS * 5) | 1, FS = (NF * 5) | 1, CS = (CH * 5) | 1;
     static constexpr int N_Q = CPT * (QS > FS ? QS : FS), N_F = 3 * CPT * CS;
-    static_assert(NF % CH == 0 && CH % KB == 0 && NS % KA == 0 && RW % RG == 0, "whole chunks");
+    static_assert(NF % CH == 0 && CH % KB == 0, "whole chunks");
     static_assert(NS * 5 <= FS && (!SPLIT || 3 * CPT * NS * 5 <= N_F), "results over the work areas");
 };
 
@@ -792,7 +790,7 @@ __global__ void __launch_bounds__((IV32<P>::NT)) k_inv_volume_tet_f32(MeanArgs<f
     using L = IV32<P>;
     using uni = typename Uni<real>::type;
     constexpr int NS = L::NS, NF = L::NF, CPT = L::CPT, NW = L::NW, NT = L::NT, RW = L::RW, NP = L::NP, FS = L::FS;
-    constexpr int QS = L::QS, CH = L::CH, CS = L::CS, KA = L::KA, KB = L::KB;
+    constexpr int QS = L::QS, CH = L::CH, CS = L::CS, KB = L::KB;
     __shared__ real s_q[L::N_Q];         // dQ [c][s][5], then Qf [c][j][5], then (rows split) the result
     __shared__ real s_f[L::N_F];         // F~ [m][c][j][5] of a chunk, then (directions split) the parts of the result
     typedef const __attribute__((address_space(4))) MeanArgs<float> Args;
@@ -847,16 +845,11 @@ __global__ void __launch_bounds__((IV32<P>::NT)) k_inv_volume_tet_f32(MeanArgs<f
             const uni c2f = (uni)fresh()->c2f;
 #pragma unroll 1
             for (int j = w; j < NF; j += NW) {
-                real acc = 0;
+                real acc = 0, c[NS];
 #pragma unroll
-                for (int k = 0; k < NS; k += KA) {
-                    real c[KA];
+                for (int e = 0; e < NS; ++e) c[e] = (real)c2f[j * NS + e];
 #pragma unroll
-                    for (int e = 0; e < KA; ++e) c[e] = (real)c2f[j * NS + k + e];
-#pragma unroll
-                    for (int e = 0; e < KA; ++e) acc += c[e] * x[k + e];
-                    if (KA < NS) __builtin_amdgcn_sched_barrier(0);
-                }
+                for (int e = 0; e < NS; ++e) acc += c[e] * x[e];
                 if (on) s_q[lc * FS + j * 5 + lv] = acc;
             }
         }
@@ -903,19 +896,15 @@ __global__ void __launch_bounds__((IV32<P>::NT)) k_inv_volume_tet_f32(MeanArgs<f
 #pragma unroll
                 for (int e = 0; e < KB; ++e) y[e] = f[e * 5];
                 const uni o0 = op + m * NF + k * CH + j0;
+                real c[RW][KB];
 #pragma unroll
-                for (int r0 = 0; r0 < RW; r0 += L::RG) {
-                    real c[L::RG][KB];
+                for (int r = 0; r < RW; ++r)
 #pragma unroll
-                    for (int r = 0; r < L::RG; ++r)
+                    for (int e = 0; e < KB; ++e) c[r][e] = (real)o0[row(r) * 3 * NF + e];
 #pragma unroll
-                        for (int e = 0; e < KB; ++e) c[r][e] = (real)o0[row(r0 + r) * 3 * NF + e];
+                for (int r = 0; r < RW; ++r)
 #pragma unroll
-                    for (int r = 0; r < L::RG; ++r)
-#pragma unroll
-                        for (int e = 0; e < KB; ++e) sum[r0 + r] += c[r][e] * y[e];
-                    if (L::RG < RW) __builtin_amdgcn_sched_barrier(0);
-                }
+                    for (int e = 0; e < KB; ++e) sum[r] += c[r][e] * y[e];
             };
             if constexpr (L::SPLIT) {
 #pragma unroll 1
@@ -925,14 +914,9 @@ __global__ void __launch_bounds__((IV32<P>::NT)) k_inv_volume_tet_f32(MeanArgs<f
 #pragma unroll 1
                     for (int j0 = 0; j0 < CH; j0 += KB) columns(m, j0, sum);
                 };
-                if constexpr (AD == 1) {
-#pragma unroll 1
-                    for (int i = 0; i < 3 * (CH / KB); ++i) columns(i / (CH / KB), i % (CH / KB) * KB, acc[0]);
-                } else {
-                    direction(0, acc[0]);
-                    direction(1, acc[AD > 1 ? 1 : 0]);
-                    direction(2, acc[AD > 1 ? 2 : 0]);
-                }
+                direction(0, acc[0]);
+                direction(1, acc[1]);
+                direction(2, acc[2]);
             }
             __syncthreads();
         }

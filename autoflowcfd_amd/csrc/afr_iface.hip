@@ -25,6 +25,11 @@
 
 #include <type_traits>
 
+// Products are fused with the sums of their own expression only.  Fused wherever the optimiser meets a
+// pair, which it meets depends on the form of the kernel (row width, index width), and a case in a batch,
+// whose rows are padded to the widest of the batch, would differ from itself alone in the last bits.
+#pragma clang fp contract(on)
+
 #include "../../include/afr.h"
 #include "afr_meanflow.hpp"
 #include "afr_outlier.hpp"

@@ -1,11 +1,12 @@
 """GPU: a case's residuals and SST step do not depend on the batch it rides in, bit for bit: small tet and
 mixed cases whose cells fall at other places of the kernels' tiles and waves (12, 16, 7 and 4 cells; waves of
-8 or 2) than alone, at every order and precision, and whose row tables a batch adds up."""
+8 or 2) than alone, at every order and precision, and whose row tables a batch adds up (prisms beside tets: rows padded
+to the tets' width)."""
 
 import numpy as np
 import pytest
 
-from cases import freestream, mixed_mesh, smooth_state, tet_box
+from cases import freestream, mixed_mesh, smooth_state, tet_box, wall_box
 
 pytestmark = pytest.mark.gpu
 
@@ -16,6 +17,8 @@ def _mesh(n):
     from autoflowcfd_amd.mesh import BC_FARFIELD, BC_WALL, mesh_from_cells
     if n == "mixed":
         m = mixed_mesh()
+    elif n == "prism":
+        m = wall_box((3, 2, 2), seed=2)
     else:
         src = tet_box(2, seed=1)
         m = mesh_from_cells(src.nodes, None, src.tet_conn[:n], default_bc=BC_FARFIELD)
@@ -27,7 +30,7 @@ def _mesh(n):
     return m
 
 
-@pytest.mark.parametrize("sizes,order,prec", [(s, o, p) for s in (SIZES, ("mixed", 13, "mixed", 2)) for o in (1, 2)
+@pytest.mark.parametrize("sizes,order,prec", [(s, o, p) for s in (SIZES, ("mixed", 13, "mixed", 2, "prism")) for o in (1, 2)
                                               for p in ("f32", "f64")] + [(SIZES, 3, "f64")])
 def test_case_does_not_depend_on_its_batch(sizes, order, prec):
     import torch

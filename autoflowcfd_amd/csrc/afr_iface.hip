@@ -12,14 +12,14 @@
 // interpolation rows.  The jumps meet in LDS, from where one thread per solution point distributes
 // them; the outlier test runs on the residual in LDS, one lane per (cell, variable).
 //
-// Bound: latency of the gathers (VALU issue takes about half of the time, HBM traffic 8.4 GB at 82^3 P2
+// Bound: latency of the gathers (VALU issue takes about half of the time, HBM traffic 8.2 GB at 82^3 P2
 // FP32).  What this form is there for: one set of traces, slot tables and one residual write serve both
 // jumps, four resident waves per SIMD at no spill, the next tile's tables and own points in flight while
 // this one computes.  Tried and slower: five waves per workgroup with one slot per wave (2 or 3 resident
 // workgroups, uneven SIMDs: 5.0 ms), a lane's gather of all 15 values on its own instead of four lanes
 // sharing 16-byte loads (4.1 ms), a budget of five waves per SIMD (spills).
-// Measured (82^3 hex, 1.1 M prisms, P2 FP32): 2.75 ms; two kernels before, 2.88 ms for the viscous jumps
-// and about half of 2.98 ms for the inviscid ones.  304k P1 prisms FP32 263 us (401 + half of 1014).
+// Measured (82^3 hex, 1.1 M prisms, P2 FP32): 2.43 ms; two kernels before, 2.88 ms for the viscous jumps
+// and about half of 2.98 ms for the inviscid ones.  304k P1 prisms FP32 254 us (401 + half of 1014).
 // P2 and P3 tets FP64: see the matrix products below.
 #include <hip/hip_runtime.h>
 
@@ -232,7 +232,7 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
     // tets at P2 and P3: every own row is dense (the round-off entries of the collapsed basis reach
     // 1e-12 there at P2, 1e-7 at P3; outlier decisions next to a jump see them)
     constexpr bool DENSE = CT == 1 && P >= 2;
-    constexpr int ROWS_CAP = CT == 0 && KMAX == N1 * N1 ? 8 * NFP + 1 : 1;
+    constexpr int ROWS_CAP = CT == 0 && KMAX == N1 * N1 ? 8 * NFP : 1;
     __shared__ __attribute__((aligned(16))) real s_own[L::N_OWN];
     __shared__ real s_a[L::N_A];
     __shared__ real s_j[L::N_J];
@@ -255,7 +255,7 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
     // the deduplicated interpolation rows in LDS when the mesh has few blocks (8 for a graded
     // prism box; a batch of cases or a tet mesh has more and reads them from global memory)
     const int n_rows = args.n_rows;
-    const bool rows_lds = ROWS_CAP > 1 && n_rows < ROWS_CAP;
+    const bool rows_lds = ROWS_CAP > 1 && n_rows <= ROWS_CAP;
     if (rows_lds) {
 #pragma unroll
         for (int u = 0; u < (ROWS_CAP * KMAX + NT - 1) / NT; ++u) {
@@ -264,9 +264,6 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
                 const int i = args.rows_idx[q], nnz = args.rows_nnz[r];
                 s_rw[q] = args.rows_w[q];
                 s_ri[q] = (uint8_t)(i | (q == r * KMAX && nnz > N1 ? 128 : 0));
-            } else if (r == n_rows) {   // after them one of zeros
-                s_rw[q] = real(0);
-                s_ri[q] = 0;
             }
         }
     }
@@ -489,8 +486,9 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
             for (int q = 0; q < 3; ++q) A[q] = at<BIG>(a->slot_adjrow, ai + q);
             if constexpr (INV) fb = (at<BIG>(a->slot_fb, sidx) >> fp) & 1;
             // 1. the other side's trace (the rows hold their non-zeros first); lanes without a source join the
-            //    loads of their quad with weights of zero: the last row in LDS, or the first of the table masked
-            const int r = have ? row : (rows_lds ? n_rows : 0);
+            //    loads of their quad with the first row and weights of zero (chosen after the loads: chosen by a
+            //    branch around them, a mixed P1 evaluation took 270 us, 265 so)
+            const int r = have ? row : 0;
             const Idx p0 = times<BIG>(have ? nb : 0, NS);
             const int qi = tid & 3;
             auto row_entry = [&](int kk, int& i, real& w) {
@@ -499,7 +497,7 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
                     w = s_rw[r * KMAX + kk];
                 } else {
                     i = at<BIG>(a->rows_idx, (Idx)r * KMAX + kk);
-                    w = have ? at<BIG>(a->rows_w, (Idx)r * KMAX + kk) : real(0);
+                    w = at<BIG>(a->rows_w, (Idx)r * KMAX + kk);
                 }
             };
             v4 acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
@@ -521,7 +519,7 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
                         if (rows_lds) i &= 127;
                     }
                     pt[k] = p0 + i;
-                    if (kk != k0 + k) w[k] = real(0);
+                    if (!have || kk != k0 + k) w[k] = real(0);
                 }
                 if constexpr (VISC) {
                     quad_gather<N1, BIG, real>(acc, a->pack, pt, w, qi);
@@ -532,10 +530,9 @@ __global__ void __launch_bounds__((IF<P, CT, real, INV, VISC>::NT))
                         for (int q = 0; q < 5; ++q) pn[q] += w[k] * at<BIG>(a->dQ, pt[k] * 5 + q);
                 }
             };
-            // waves without any source skip the rows (a table without rows is not read).  As a branch it also
-            // keeps the loads before it out of the gather: kernel on 1.1 M P2 prisms FP32 2755 -> 2430 us, 304k
-            // P1 prisms 262 -> 264
-            if (__any(have)) terms(0, std::true_type());
+            // A table without rows is not read.  As a branch this also keeps the loads before it out of the gather:
+            // kernel on 1.1 M P2 prisms FP32 2755 -> 2435 us, 304k P1 prisms 266 -> 254
+            if (n_rows > 0) terms(0, std::true_type());
             // further terms: the quads with a wide row (prism sources), or every lane up to the widest
             // row of the wave (dense rows of tet sources)
             if constexpr (KMAX == N1 * N1) {
@@ -804,17 +801,20 @@ template <int P, int CT, int KMAX, typename real, bool INV, bool VISC>
 int launch_iface_t(const MeanArgs<real>& a, hipStream_t st) {
     using L = IF<P, CT, real, INV, VISC>;
     const int64_t tiles = (a.n_cells + L::CPT - 1) / L::CPT;
-    // 2048 workgroups, twice what is resident, up to some 50 tiles each (whole mean-flow residual, us, 2048
-    // against 4096: 13k tiles P2 313 / 320, 25k P1 437 / 440, 6k P3 tets 700 / 712); 4096 for larger meshes
-    // (220k tiles P2: 4844 / 4823)
+    // 2048 workgroups, twice what is resident, up to some 50 tiles each; 4096 for larger meshes.  Whole
+    // mean-flow residual, us, 2048 against 4096: P2 prisms FP32 13k tiles 289 / 296, 35k 752 / 753, 70k 1504 /
+    // 1502, 100k 2140 / 2123, 150k 3185 / 3156, 220k 4749 / 4691; P1 prisms 25k 466 / 473, 99k 1812 / 1812, 222k
+    // 4112 / 4110; P3 tets 41k 4159 / 4177, 96k 9577 / 9581
     const int grid = walk_grid(tiles, 1, a.grid_cap > 0 ? a.grid_cap : (tiles <= 100000 ? 2048 : 4096));
     // 32-bit byte offsets while the pack of all cells (the largest array by cells) and the table of
     // distinct interpolation rows stay under 4 GiB
     const bool big = a.n_cells_mesh * L::NS * kPack * (int64_t)sizeof(real) >= ((int64_t)1 << 32) ||
                      (int64_t)a.n_rows * KMAX * 8 >= ((int64_t)1 << 32);
     if constexpr (CT == 1 && P >= 2 && VISC && sizeof(real) == 8) {
-        // matrix products wherever the fragments of the rows fit the scratch array (they do unless nearly
-        // every slot has rows of its own).  24.6k P3 tets 369 us, 700 by vector FMAs; 10.3k P2 tets 56 (81).
+        // matrix products wherever the fragments of the rows fit the scratch array: the rows depend on how two
+        // faces meet, not on their shape (6 blocks for any box of tets), so that only meshes of a few cells have
+        // more blocks than cells' scratch.  24.6k P3 tets 327 us, 700 by vector FMAs; 10.3k P2 tets 55 (81).
+        // The sums are the same, term by term.
         const int64_t blocks = (a.n_rows + L::NFP - 1) / L::NFP, n = blocks * FR<P>::KS * 64;
         if (n <= a.work_len && n < ((int64_t)1 << 30)) {
             if (n > 0)

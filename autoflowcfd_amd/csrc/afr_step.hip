@@ -101,7 +101,8 @@ __global__ void __launch_bounds__(kThreads) k_dt_cells(const real* __restrict__ 
 // barrier.  Values cross HBM in consecutive order; a lane holds its filter row in registers for the
 // whole kernel (again when the wave passes from prisms to tets) and reads each point's five values
 // from LDS at once.  Bound: HBM (5 values from 3 arrays and dt in, 5 out, per point).  1024 workgroups
-// are what the device holds at once at P2; 2048 and 4096 cost 2 and 5% (weights loaded by more waves).
+// are what the device holds at once at P2; us at 512 / 1024 / 2048 / 4096 (filter rows loaded by more waves):
+// 66.5k P2 prisms FP32 46 / 35 / 35 / 37, 304k P1 prisms 49 / 38 / 36 / 35, 24.6k P3 tets FP64 90 / 97 / 111 / 137.
 // Measured, 66.5k P2 prisms FP32: 36.8 us, 58.6 with one thread per filtered value and the filter in LDS;
 // 10.3k P2 tets FP64 15.6 us (25.4), P1 tets FP64 8.4 (11.8).
 template <int NS> struct RK {

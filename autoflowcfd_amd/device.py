@@ -209,11 +209,11 @@ class DeviceMesh:
         self.slot_bc = devi(np.where(sl.bc >= 0, sl.bc | (np.maximum(sl.rows_of_bc(), 0) << 4), sl.bc))
         self.slot_tn = dev(sl.tn)
         self.rows = dev(sl.rows)
-        # sparse rows plus one trailing all-zero row (index n_rows) for lanes without a source
+        # sparse rows plus one trailing all-zero row (index n_rows; the SST face kernel takes it for
+        # records without a source)
         nnz, idx, w = sparse_rows(np.concatenate([sl.rows, np.zeros((1, sl.rows.shape[1]))]))
         # slot mask: bit fp = flux point fp takes source 1; bit 30 = the slot's first-source rows
-        # are wider than order + 1 (the viscous interface kernel's helper lanes need no row load
-        # to find them)
+        # are wider than order + 1 (a hint of the C ABI; the kernels take widths from rows_nnz)
         self.slot_mask = devi(slot_mask_with_wide_flag(sl.mask, np.asarray(sl.blk)[..., 0], nnz, int(sl.n_blocks),
                                                        T.nfp, order))
         # fixed row width: (P+1)^2 when every row fits (prism sources), else (P+1)^3, zero-padded,
@@ -904,7 +904,8 @@ class DeviceMesh:
         return R
 
     def viscous_volume(self, U, mu_t=None, mu=1.8e-5, Pr=0.72, Pr_t=0.9):
-        """Prepared state, gradients and viscous volume term of U into the work buffers."""
+        """Prepared state (work_q, work_umean), interface pack and viscous volume term of U into the work
+        buffers."""
         self._check_state(U)
         _lib.check(self.lib.afr_viscous_volume(self.handle, ctypes.c_void_p(U.data_ptr()), self._check_mut(mu_t),
                                                float(mu), float(Pr), float(Pr_t), self._stream()),

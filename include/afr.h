@@ -264,15 +264,15 @@ int afr_inviscid_from_primitives(const AfrMesh *mesh, const void *dQ, const void
 /* Viscous BR1 FR residual dU/dt (C, ns, 5); mu_t (C, ns) or NULL.
  * mu, Pr, Pr_t as in the reference (1.8e-5, 0.72, 0.9 by default).  Uses the
  * work buffers work_q, work_umean, work_rvol, work_grad and work_vpack; on return work_q /
- * work_umean hold the prepared state of U. */
+ * work_umean hold the prepared state of U (the other work buffers are scratch of the library's own layout). */
 int afr_viscous_residual(const AfrMesh *mesh, const void *U, const void *mu_t, void *R, double mu,
                          double Pr, double Pr_t, int32_t suppress, void *stream);
 
 /* The two phases of afr_viscous_residual, for callers that interleave other work:
  * afr_viscous_volume writes the prepared state (work_q, work_umean), the interface
  * pack (work_vpack) and the viscous volume term (work_rvol) from U;
- * afr_viscous_interface adds the BR1 interface correction, applies the outlier zeroing when suppress != 0 and writes (accumulate == 0) or adds
- * (accumulate != 0) the result to R. */
+ * afr_viscous_interface adds the BR1 interface correction, applies the outlier zeroing when
+ * suppress != 0 and writes (accumulate == 0) or adds (accumulate != 0) the result to R. */
 int afr_viscous_volume(const AfrMesh *mesh, const void *U, const void *mu_t, double mu, double Pr, double Pr_t,
                        void *stream);
 int afr_viscous_interface(const AfrMesh *mesh, const void *U, const void *mu_t, void *R, double mu, double Pr,
@@ -280,7 +280,8 @@ int afr_viscous_interface(const AfrMesh *mesh, const void *U, const void *mu_t, 
 
 /* Full Navier-Stokes FR residual dU/dt = inviscid + viscous (each with its own
  * outlier zeroing when suppress != 0), as the reference solver sums them
- * (src/autoflowcfd/core/fr_solver/solver.py:360-420).  mu_t may be NULL.  R may lie over U. */
+ * (src/autoflowcfd/core/fr_solver/solver.py:360-420).  mu_t may be NULL.  R may lie over U.  Uses the
+ * work buffers of afr_viscous_residual; work_q and work_umean hold nothing of use afterwards. */
 int afr_residual(const AfrMesh *mesh, const void *U, const void *mu_t, void *R, double mu, double Pr,
                  double Pr_t, int32_t suppress, void *stream);
 

@@ -1,7 +1,7 @@
 // Residual outlier zeroing of a whole field, as one entry point:
 //   suppress_residual_outliers  src/autoflowcfd/core/fr_operators/troubled_cell.py:382-408
-// The residual kernels apply the same device routine (afr_outlier.hpp) to each cell's block before
-// it leaves LDS; this entry point runs it over a field held in device memory, one wavefront per
+// The interface and SST update kernels apply the same rule to each cell's block, in forms that fit
+// their lanes, before it leaves LDS or registers; this entry point runs it over a field held in device memory, one wavefront per
 // cell, for callers that hold a residual of their own (any order, any number of variables).
 #include <hip/hip_runtime.h>
 

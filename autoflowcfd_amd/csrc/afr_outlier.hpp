@@ -1,4 +1,4 @@
-// Residual outlier zeroing of one cell (device side), shared by every kernel that applies it.
+// Residual outlier zeroing of one cell (device side): the rule, and its form for one wavefront per cell.
 //
 // src/autoflowcfd/core/fr_operators/troubled_cell.py:339-408: for each variable v of a cell,
 //   ref = max(median_s |R[s][v]|, 1e-9 mean_s |U[s][v]|, 1e-300),  R[s][v] = 0 where |R| > 1e4 ref,

@@ -349,9 +349,10 @@ __global__ void __launch_bounds__(256) k_sst_face(SstArgs<real> a) {
     __shared__ int s_ri[ROWS_CAP * KMAX];
     const bool rows_lds = a.n_rows + 1 <= ROWS_CAP;
     if (rows_lds) {
-        for (int i = threadIdx.x; i < (a.n_rows + 1) * KMAX; i += 256) {
-            s_rw[i] = a.rows_w[i];
-            s_ri[i] = a.rows_idx[i];
+        for (int i = threadIdx.x; i < (a.n_rows + 1) * KMAX; i += 256) {   // the rows and one of zeros
+            const bool in = i < a.n_rows * KMAX;
+            s_rw[i] = in ? a.rows_w[i] : real(0);
+            s_ri[i] = in ? a.rows_idx[i] : 0;
         }
     }
     __syncthreads();
@@ -372,8 +373,9 @@ __global__ void __launch_bounds__(256) k_sst_face(SstArgs<real> a) {
             const int src = (a.slot_mask[sidx] >> fp) & 1;
             int row = a.slot_blk[sidx * 2 + src] * NFP + fp;
             const int nbc = a.slot_nb[sidx * 2 + src];
-            if (row < 0 || row >= a.n_rows || nbc < 0) row = a.n_rows;
-            const int64_t nb = nbc >= 0 ? nbc : 0;
+            const bool have = row >= 0 && row < a.n_rows && nbc >= 0;
+            const int64_t nb = have ? nbc : 0;
+            if (!have) row = rows_lds ? a.n_rows : 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) pn[q] = 0.0;
             int spk[KMAX];
@@ -388,7 +390,8 @@ __global__ void __launch_bounds__(256) k_sst_face(SstArgs<real> a) {
 #pragma unroll
                 for (int kk = 0; kk < KMAX; ++kk) {
                     spk[kk] = a.rows_idx[(int64_t)row * KMAX + kk];
-                    wk[kk] = a.rows_w[(int64_t)row * KMAX + kk];
+                    const real w = a.rows_w[(int64_t)row * KMAX + kk];
+                    wk[kk] = have ? w : real(0);
                 }
             }
 #pragma unroll

@@ -209,8 +209,7 @@ class DeviceMesh:
         self.slot_bc = devi(np.where(sl.bc >= 0, sl.bc | (np.maximum(sl.rows_of_bc(), 0) << 4), sl.bc))
         self.slot_tn = dev(sl.tn)
         self.rows = dev(sl.rows)
-        # sparse rows plus one trailing all-zero row (index n_rows; the SST face kernel takes it for
-        # records without a source)
+        # sparse rows plus one trailing all-zero row (index n_rows)
         nnz, idx, w = sparse_rows(np.concatenate([sl.rows, np.zeros((1, sl.rows.shape[1]))]))
         # slot mask: bit fp = flux point fp takes source 1; bit 30 = the slot's first-source rows
         # are wider than order + 1 (a hint of the C ABI; the kernels take widths from rows_nnz)

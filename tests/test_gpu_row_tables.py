@@ -7,21 +7,20 @@
 
 import pytest
 
-from cases import freestream, mixed_mesh, rotated_prism_box, wall_box
-from cases import smooth_state
+from cases import freestream, mixed_mesh, rotated_prism_box, smooth_state, wall_box
 
 pytestmark = pytest.mark.gpu
 
 MESHES = {"wallbox": lambda: wall_box(seed=4), "rotated": lambda: rotated_prism_box(seed=2), "mixed": mixed_mesh}
 
 
-def _device(mesh, order, dtype):
+def _device(mesh, order, dtype, turbulence=None):
     import numpy as np
     import torch
     from autoflowcfd_amd.device import DeviceMesh, bc_params_table
     from autoflowcfd_amd.geometry import map_ref
     Q0 = freestream(0.15, 4.0)
-    dm = DeviceMesh(mesh, order, dtype=dtype, bc_params=bc_params_table(Q0))
+    dm = DeviceMesh(mesh, order, dtype=dtype, bc_params=bc_params_table(Q0), turbulence=turbulence)
     xyz = np.zeros((mesh.n_cells, dm.ns, 3))
     if mesh.n_prism:
         xyz[:mesh.n_prism] = map_ref(True, dm.T.sps, mesh.nodes[mesh.prism_conn])
@@ -86,13 +85,25 @@ def test_row_tables_past_two_to_the_31_entries(name, order, prec):
 def test_no_row_is_used_past_the_last(name, order, prec):
     import numpy as np
     import torch
-    from autoflowcfd_amd.mesh import BC_FARFIELD, mesh_from_cells
+    from autoflowcfd_amd.mesh import BC_FARFIELD, BC_WALL, mesh_from_cells
     print(f"[gpu] end of the row table {name} P{order} {prec}", flush=True)
     src = wall_box(seed=2)
     mesh = (mesh_from_cells(src.nodes, src.prism_conn[:1], default_bc=BC_FARFIELD) if name == "one"
             else MESHES[name]())
-    dm, U, mut = _device(mesh, order, torch.float32 if prec == "f32" else torch.float64)
-    ref = _residuals(dm, U, mut)
+    fr = mesh.faces
+    low = np.flatnonzero(fr.is_boundary)[:2]
+    fr.bc[low] = BC_WALL
+    mesh.wall_nodes = np.unique(fr.node_ids[low])
+    mesh.wall_nodes = mesh.wall_nodes[mesh.wall_nodes >= 0]
+    dm, U, mut = _device(mesh, order, torch.float32 if prec == "f32" else torch.float64, "SST")
+    k0, w0 = torch.full_like(mut, 0.39), torch.full_like(mut, 2660.0)
+    step = torch.full_like(mut, 1e-6)
+
+    def results():
+        k, w = k0.clone(), w0.clone()
+        dm.sst_step(U, k, w, step, torch.zeros_like(k), torch.zeros_like(k))
+        return _residuals(dm, U, mut) + [k, w]
+    ref = results()
     n = 0 if name == "one" else dm.n_rows                    # a lone cell needs no row
     assert n > 0 or bool((dm.slot_bc >= 0).all())
 
@@ -102,5 +113,5 @@ def test_no_row_is_used_past_the_last(name, order, prec):
         return y
     _with_tables(dm, n, ended(dm.rows_nnz, dm.rows_knz), ended(dm.rows_idx, (1 << 30) - 1),
                  ended(dm.rows_w, float(np.nan)))
-    for a, b in zip(_residuals(dm, U, mut), ref):
+    for a, b in zip(results(), ref):
         assert torch.equal(a, b)
